@@ -13,7 +13,7 @@
 //   F_ij        = (c * A_j) / s, 0 if s == 0            (:62-64)
 #include <algorithm>
 
-#include "ray.h"
+#include "wide.h"
 
 namespace flux {
 
@@ -46,137 +46,233 @@ __device__ __forceinline__ T ff_value(T c, const T *Pi, const T *Pj, T Aj) {
   return (c * Aj) / s;
 }
 
-// The bit word w of row p of the candidate / visibility mask.
-template <typename T, bool CAST_RAYS>
-__device__ __forceinline__ void ff_mask_word(const flux_scene &S, const T *__restrict__ P,
-                                             const T *__restrict__ N,
-                                             const int64_t *__restrict__ I,
-                                             const int64_t *__restrict__ J, int64_t n, T eps,
-                                             int mode, uint64_t *__restrict__ mask, int64_t W,
-                                             int64_t wave, int lane) {
-  const int64_t p = wave / W, w = wave % W;
-  const int64_t q = w * 64 + lane;
-  const int64_t i64 = I[p];
-  const bool row_ok = i64 >= 0 && i64 < S.nf;
-  const int i = row_ok ? (int)i64 : 0;
-  T Pi[3] = {P[i * 3], P[i * 3 + 1], P[i * 3 + 2]};
-  T Ni[3] = {N[i * 3], N[i * 3 + 1], N[i * 3 + 2]};
-  bool bit = false;
-  if (q < n && row_ok && J[q] >= 0 && J[q] < S.nf) {
-    const int j = (int)J[q];
-    T Pj[3] = {P[(int64_t)j * 3], P[(int64_t)j * 3 + 1], P[(int64_t)j * 3 + 2]};
-    T Nj[3] = {N[(int64_t)j * 3], N[(int64_t)j * 3 + 1], N[(int64_t)j * 3 + 2]};
-    T c = ff_prefilter(Pi, Ni, Pj, Nj);
-    if (i != j && c > eps) {
-      if (CAST_RAYS) {
-        bit = face_to_face_vis(S, i, j, mode, Pi, Pj);
-      } else {
-        bit = true;
-      }
-    }
-  }
-  const uint64_t b = __ballot(bit);
-  if (lane == 0) mask[p * W + w] = b;
-}
-
-// One wave per (row p, 64-column word w), the waves of the grid striding
-// over all m W words.  With CAST_RAYS == false the bit is the prefilter
-// alone (the set of pairs that get a ray).
-template <typename T, bool CAST_RAYS = true>
-__global__ void __launch_bounds__(256) k_ff_mask(flux_scene S, const T *__restrict__ P,
-                                                 const T *__restrict__ N,
-                                                 const int64_t *__restrict__ I, int64_t m,
-                                                 const int64_t *__restrict__ J, int64_t n,
-                                                 T eps, int mode, uint64_t *__restrict__ mask,
-                                                 int64_t W) {
+// Candidate bits (the pairs that get a ray): one wave per (row p, 64-column
+// word w), the waves of the grid striding over all m W words.
+template <typename T>
+__global__ void __launch_bounds__(256) k_ff_candidates(int64_t nf, const T *__restrict__ P,
+                                                       const T *__restrict__ N,
+                                                       const int64_t *__restrict__ I, int64_t m,
+                                                       const int64_t *__restrict__ J, int64_t n,
+                                                       T eps, uint64_t *__restrict__ mask,
+                                                       int64_t W) {
   const int lane = threadIdx.x & 63;
   const int64_t nwaves = (int64_t)gridDim.x * (blockDim.x >> 6);
   for (int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6; wave < m * W;
        wave += nwaves) {
-    ff_mask_word<T, CAST_RAYS>(S, P, N, I, J, n, eps, mode, mask, W, wave, lane);
+    const int64_t p = wave / W, q = (wave % W) * 64 + lane;
+    const int64_t i64 = I[p];
+    const bool row_ok = i64 >= 0 && i64 < nf;
+    const int64_t i = row_ok ? i64 : 0;
+    const T Pi[3] = {P[i * 3], P[i * 3 + 1], P[i * 3 + 2]};
+    const T Ni[3] = {N[i * 3], N[i * 3 + 1], N[i * 3 + 2]};
+    bool bit = false;
+    if (q < n && row_ok && J[q] >= 0 && J[q] < nf) {
+      const int64_t j = J[q];
+      const T Pj[3] = {P[j * 3], P[j * 3 + 1], P[j * 3 + 2]};
+      const T Nj[3] = {N[j * 3], N[j * 3 + 1], N[j * 3 + 2]};
+      bit = i != j && ff_prefilter(Pi, Ni, Pj, Nj) > eps;
+    }
+    const uint64_t b = __ballot(bit);
+    if (lane == 0) mask[wave] = b;
   }
 }
 
-// Same result as k_ff_mask<T, true>, with stream compaction: one wave per
-// row p.  The row is scanned 64 columns at a time; prefilter candidates are
-// appended to a per-wave LDS queue and rays are cast only when 64 are
-// queued, so every lane of the wave traces (the prefilter keeps ~1/4 of the
-// pairs on terrain, which leaves 3/4 of a one-pair-per-lane wave idle).
-// Each lane walks the tree on its own: tracing the 64 queued rays as one
-// wave-coherent packet (one shared node sequence) measured 1.9x slower on
-// the 41,472-facet terrain, because the rays of a queue fan out widely and
-// the union of their node sets is far larger than any single ray's.
-// Results collect in a per-wave LDS bitmask for a segment of 64 words (4096
-// columns), flushed to the mask after each segment.  All LDS traffic is
-// wave-private, so no workgroup barrier is needed.
-template <typename T>
-__global__ void __launch_bounds__(256) k_ff_mask_rows(flux_scene S, const T *__restrict__ P,
-                                                      const T *__restrict__ N,
-                                                      const int64_t *__restrict__ I, int64_t m,
-                                                      const int64_t *__restrict__ J, int64_t n,
-                                                      T eps, int mode,
-                                                      uint64_t *__restrict__ mask, int64_t W) {
-  __shared__ int32_t queue[4][128];
-  __shared__ unsigned long long bits[4][64];
-  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int64_t p = (int64_t)blockIdx.x * 4 + wv;
-  if (p >= m) return;  // uniform per wave
-  const int64_t i64 = I[p];
-  const bool row_ok = i64 >= 0 && i64 < S.nf;
-  const int i = row_ok ? (int)i64 : 0;
-  T Pi[3] = {P[i * 3], P[i * 3 + 1], P[i * 3 + 2]};
-  T Ni[3] = {N[i * 3], N[i * 3 + 1], N[i * 3 + 2]};
-  const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  int count = 0;
+// Rays of the pairs (p, q) of m x n positions for trace_wave (wide.h).  A
+// wave takes tiles of one row p and up to 64 words of 64 columns each,
+// evaluates the prefilter 64 columns at a time and keeps the pairs that
+// need a ray in a small queue in LDS, from which lanes out of work are
+// served (the prefilter keeps ~1/4 of the pairs on terrain).  A visible
+// pair sets its bit in the zeroed mask.  Lanes of a wave may work on
+// different rows, so no lane waits for the end of a row: with one wave per
+// row and batches of 64 rays, a row of a small mesh was a serial chain of
+// batches (1131 us for 1,922 facets) and every batch waited for its longest
+// ray.
+constexpr int kPairQueue = 128;  // < 64 left over + one word of 64
 
-  auto cast = [&](int active) {
-    if (lane < active) {
-      const int32_t q = queue[wv][lane];
-      const int j = (int)J[q];
-      T Pj[3] = {0, 0, 0};
-      if (mode == FLUX_MODE_EMBREE)
-        for (int c = 0; c < 3; ++c) Pj[c] = P[(int64_t)j * 3 + c];
-      if (face_to_face_vis(S, i, j, mode, Pi, Pj))
-        atomicOr(&bits[wv][(q >> 6) & 63], 1ull << (q & 63));
-    }
-    __builtin_amdgcn_wave_barrier();
-  };
+// The tiles of a wave.  Large problems draw them from a counter, one atomic
+// per 64 words of 64 columns.  Smaller ones have smaller tiles, too many for
+// that (an atomic on one address costs the chip about 18 ns: 59,582 one-word
+// tiles of 1,922 facets took 1.0 ms drawn and 0.21 ms dealt out): there each
+// wave has one tile of every round, in a place that moves from round to
+// round (at a fixed place a wave would keep to one column range).
+constexpr int64_t kPairTiles = 40960;  // tiles aimed at, 8 a wave
+constexpr int64_t kTileShift = 977;    // below 5,120 waves, which rounds need
 
-  for (int64_t w0 = 0; w0 < W; w0 += 64) {
-    bits[wv][lane] = 0ull;
-    __builtin_amdgcn_wave_barrier();
-    const int64_t w1 = min(W, w0 + 64);
-    for (int64_t w = w0; w < w1; ++w) {
-      const int64_t q = w * 64 + lane;
-      bool cand = false;
-      if (q < n && row_ok) {
-        const int64_t j64 = J[q];
-        if (j64 >= 0 && j64 < S.nf && j64 != i) {
-          const int j = (int)j64;
-          T Pj[3] = {P[(int64_t)j * 3], P[(int64_t)j * 3 + 1], P[(int64_t)j * 3 + 2]};
-          T Nj[3] = {N[(int64_t)j * 3], N[(int64_t)j * 3 + 1], N[(int64_t)j * 3 + 2]};
-          cand = ff_prefilter(Pi, Ni, Pj, Nj) > eps;
-        }
-      }
-      const unsigned long long bal = __ballot(cand);
-      if (cand) queue[wv][count + __popcll(bal & below)] = (int32_t)q;
-      count += __popcll(bal);
-      __builtin_amdgcn_wave_barrier();
-      if (count >= 64) {
-        cast(64);
-        const int rest = count - 64;
-        if (lane < rest) queue[wv][lane] = queue[wv][64 + lane];
-        __builtin_amdgcn_wave_barrier();
-        count = rest;
-      }
-    }
-    if (count > 0) {
-      cast(count);
-      count = 0;
-    }
-    if (w0 + lane < W) mask[p * W + w0 + lane] = bits[wv][lane];
-    __builtin_amdgcn_wave_barrier();
+struct TileWalk {
+  int64_t ntiles, base, slot, nwaves;
+  unsigned long long *counter;
+
+  __device__ __forceinline__ void init(int64_t n, unsigned long long *c) {
+    ntiles = n;
+    counter = c;
+    nwaves = (int64_t)gridDim.x * 4;
+    base = 0;
+    slot = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
   }
+
+  // The next tile, or one past the last.
+  __device__ __forceinline__ int64_t next() {
+    if (counter) {
+      unsigned long long t = 0;
+      if ((threadIdx.x & 63) == 0) t = atomicAdd(counter, 1ull);
+      return ((int64_t)__builtin_amdgcn_readfirstlane((int)(t >> 32)) << 32) |
+             (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)t);
+    }
+    const int64_t tile = base + slot;
+    base += nwaves;
+    slot = slot + kTileShift < nwaves ? slot + kTileShift : slot + kTileShift - nwaves;
+    return tile < ntiles ? tile : ntiles;
+  }
+};
+
+static inline int64_t tile_width(int64_t words) {
+  return std::max<int64_t>(1, std::min<int64_t>(64, words / kPairTiles));
+}
+
+// Rays of the pairs (p, q) of m x n positions for trace_wave (wide.h).  A
+// wave takes tiles of one row p, evaluates the prefilter 64 columns at a
+// time and keeps the pairs that need a ray in a small queue in LDS, from
+// which lanes out of work are served (the prefilter keeps ~1/4 of the pairs
+// on terrain).  A visible pair sets its bit in the zeroed mask.  Lanes of a
+// wave may work on different rows, so none waits for the end of a row: with
+// one wave per row and batches of 64 rays, a row of a small mesh was a
+// serial chain of batches and every batch waited for its longest ray.
+// Binary walks in such batches took 404 ms for the 41,472-facet terrain
+// (seed 5) and 1131 us for a 1,922-facet crater; this takes 90.7 ms and
+// 214 us.  It is bound by VALU issue (99 % busy, 52 % of lanes active).
+template <typename T>
+struct PairSource {
+  const T *P, *N;
+  const int64_t *I, *J;
+  int64_t n, W, tile_words, tiles_per_row;
+  T eps;
+  int mode;
+  uint64_t *mask;
+  TileWalk tiles;
+  int2 *queue;
+  // wave state
+  int64_t p, w, wend;
+  int count, lane;
+  bool exhausted;
+  T Pi[3], Ni[3];
+  int i_row;
+  // the lane's ray
+  int lp, lq;
+
+  __device__ __forceinline__ bool drained() const { return exhausted && count == 0; }
+
+  __device__ __forceinline__ bool next_tile(const flux_scene &S) {
+    const int64_t tile = tiles.next();
+    if (tile >= tiles.ntiles) return false;
+    p = tile / tiles_per_row;
+    w = (tile - p * tiles_per_row) * tile_words;
+    wend = min(W, w + tile_words);
+    const int64_t i64 = I[p];
+    i_row = i64 >= 0 && i64 < S.nf ? (int)i64 : -1;
+    const int64_t i = i_row < 0 ? 0 : i_row;
+    for (int c = 0; c < 3; ++c) {
+      Pi[c] = P[i * 3 + c];
+      Ni[c] = N[i * 3 + c];
+    }
+    if (i_row < 0) w = wend;
+    return true;
+  }
+
+  // Queue the candidates of the next word; false when no tiles are left.
+  __device__ __forceinline__ bool push_word(const flux_scene &S) {
+    while (w >= wend) {
+      if (!next_tile(S)) {
+        exhausted = true;
+        return false;
+      }
+    }
+    const int64_t q = w * 64 + lane;
+    ++w;
+    bool cand = false;
+    if (q < n) {
+      const int64_t j = J[q];
+      if (j >= 0 && j < S.nf && j != i_row) {
+        const T Pj[3] = {P[j * 3], P[j * 3 + 1], P[j * 3 + 2]};
+        const T Nj[3] = {N[j * 3], N[j * 3 + 1], N[j * 3 + 2]};
+        cand = ff_prefilter(Pi, Ni, Pj, Nj) > eps;
+      }
+    }
+    const uint64_t bal = __ballot(cand);
+    if (cand) queue[count + lane_rank(bal)] = make_int2((int)p, (int)q);
+    count += __popcll(bal);
+    return true;
+  }
+
+  __device__ __forceinline__ void emit(int a, int b) {
+    atomicOr((unsigned long long *)&mask[(int64_t)a * W + (b >> 6)], 1ull << (b & 63));
+  }
+
+  __device__ __forceinline__ bool refill(const flux_scene &S, LaneRay &L) {
+    if (L.cur == kLaneVisible) emit(lp, lq);
+    if (L.cur <= kLaneDone) L.cur = kLaneIdle;
+    const uint64_t idle = __ballot(L.cur == kLaneIdle);
+    const int want = __popcll(idle);
+    while (count < want && push_word(S)) {
+    }
+    wave_lds_order();
+    const int take = min(count, want), rank = lane_rank(idle);
+    if (L.cur == kLaneIdle && rank < take) {
+      const int2 e = queue[count - 1 - rank];
+      lp = e.x;
+      lq = e.y;
+      const int64_t i = I[lp], j = J[lq];
+      const T a[3] = {P[i * 3], P[i * 3 + 1], P[i * 3 + 2]};
+      const T b[3] = {P[j * 3], P[j * 3 + 1], P[j * 3 + 2]};
+      pair_begin(S, L, (int)i, (int)j, mode, a, b);
+    }
+    wave_lds_order();
+    count -= take;
+    return __ballot(L.cur > kLaneIdle) != 0 || !drained();
+  }
+
+  __device__ __forceinline__ void leaf(const flux_scene &S, LaneRay &L, const int *stk) {
+    lane_leaf(S, L, stk);
+  }
+};
+
+template <typename T>
+__global__ void __launch_bounds__(256, 5) k_ff_mask_rays(
+    flux_scene S, const T *__restrict__ P, const T *__restrict__ N,
+    const int64_t *__restrict__ I, int64_t m, const int64_t *__restrict__ J, int64_t n, T eps,
+    int mode, uint64_t *__restrict__ mask, int64_t W, int64_t tile_words,
+    int64_t tiles_per_row, unsigned long long *__restrict__ counter) {
+  __shared__ int stack[4][kWideStack][64];
+  __shared__ int2 queue[4][kPairQueue];
+  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  PairSource<T> src;
+  src.P = P;
+  src.N = N;
+  src.I = I;
+  src.J = J;
+  src.n = n;
+  src.W = W;
+  src.tile_words = tile_words;
+  src.tiles_per_row = tiles_per_row;
+  src.eps = eps;
+  src.mode = mode;
+  src.mask = mask;
+  src.tiles.init(m * tiles_per_row, counter);
+  src.queue = queue[wv];
+  src.p = src.w = src.wend = 0;
+  src.count = 0;
+  src.lane = lane;
+  src.exhausted = false;
+  src.lp = src.lq = 0;
+  trace_wave(S, src, &stack[wv][0][lane]);
+}
+
+// mask and the tile counter set to zero (no memset: callers may capture)
+__global__ void k_mask_clear(uint64_t *__restrict__ mask, int64_t words,
+                             unsigned long long *__restrict__ counter) {
+  const int64_t step = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < words; k += step)
+    mask[k] = 0ull;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *counter = 0ull;
 }
 
 // row_nnz[p] = popcount of mask row p; one wave per row.
@@ -304,15 +400,23 @@ extern "C" int flux_ff_mask(const flux_scene *scene, const void *P, const void *
   hipStream_t st = as_stream(stream);
   const int64_t W = (n + 63) / 64;
   if (W > 0) {
-    const unsigned blocks = ceil_div_u(m, 4);
+    FLUX_CHECK(m < ((int64_t)1 << 31), "flux_ff_mask: m too large for int32 rows");
+    // row_nnz[0] is the tile counter until k_row_count writes it
+    const int64_t tw = tile_width(m * W);
+    const int64_t tpr = (W + tw - 1) / tw;
+    unsigned long long *counter = (unsigned long long *)row_nnz;
+    hipLaunchKernelGGL(k_mask_clear, dim3(grid_1d(m * W, 1024)), dim3(256), 0, st, mask, m * W,
+                       counter);
+    if (tw < 64) counter = nullptr;
+    const unsigned blocks = trace_groups(m * tpr);
     if (dtype == FLUX_F64)
-      hipLaunchKernelGGL(k_ff_mask_rows<double>, dim3(blocks), dim3(256), 0, st, *scene,
+      hipLaunchKernelGGL(k_ff_mask_rays<double>, dim3(blocks), dim3(256), 0, st, *scene,
                          (const double *)P, (const double *)N, I, m, J, n, (double)eps, mode,
-                         mask, W);
+                         mask, W, tw, tpr, counter);
     else
-      hipLaunchKernelGGL(k_ff_mask_rows<float>, dim3(blocks), dim3(256), 0, st, *scene,
+      hipLaunchKernelGGL(k_ff_mask_rays<float>, dim3(blocks), dim3(256), 0, st, *scene,
                          (const float *)P, (const float *)N, I, m, J, n, (float)eps, mode,
-                         mask, W);
+                         mask, W, tw, tpr, counter);
     FLUX_LAUNCH_CHECK();
   }
   hipLaunchKernelGGL(k_row_count, dim3(ceil_div_u(m, 4)), dim3(256), 0, st, mask, m, W,
@@ -335,13 +439,11 @@ extern "C" int flux_ff_candidates(const flux_scene *scene, const void *P, const 
   if (W > 0) {
     const unsigned blocks = (unsigned)std::min<int64_t>((m * W + 3) / 4, 1 << 20);
     if (dtype == FLUX_F64)
-      hipLaunchKernelGGL((k_ff_mask<double, false>), dim3(blocks), dim3(256), 0, st, *scene,
-                         (const double *)P, (const double *)N, I, m, J, n, (double)eps, 0,
-                         mask, W);
+      hipLaunchKernelGGL(k_ff_candidates<double>, dim3(blocks), dim3(256), 0, st, scene->nf,
+                         (const double *)P, (const double *)N, I, m, J, n, (double)eps, mask, W);
     else
-      hipLaunchKernelGGL((k_ff_mask<float, false>), dim3(blocks), dim3(256), 0, st, *scene,
-                         (const float *)P, (const float *)N, I, m, J, n, (float)eps, 0, mask,
-                         W);
+      hipLaunchKernelGGL(k_ff_candidates<float>, dim3(blocks), dim3(256), 0, st, scene->nf,
+                         (const float *)P, (const float *)N, I, m, J, n, (float)eps, mask, W);
     FLUX_LAUNCH_CHECK();
   }
   hipLaunchKernelGGL(k_row_count, dim3(ceil_div_u(m, 4)), dim3(256), 0, st, mask, m, W,

@@ -57,32 +57,46 @@ __device__ __forceinline__ double sel3(const double *v, int k) {
   return k == 0 ? v[0] : (k == 1 ? v[1] : v[2]);
 }
 
-// Returns t >= 0 of the hit, or -1 for a miss.  v: 9 doubles (A, B, C).
-__device__ __forceinline__ double tri_hit(const Ray64 &r, const double *__restrict__ v) {
+// Edge functions U, V, W of the triangle v (9 doubles A, B, C) in the ray's
+// sheared frame and the vertices' coordinates along the ray's main axis,
+// relative to the origin.
+struct TriEdges {
+  double U, V, W, A_z, B_z, C_z;
+};
+
+__device__ __forceinline__ TriEdges tri_edges(const Ray64 &r, const double *__restrict__ v) {
+  TriEdges e;
   const double A_x = sel3(v, r.kx) - sel3(r.o, r.kx);
   const double A_y = sel3(v, r.ky) - sel3(r.o, r.ky);
-  const double A_z = sel3(v, r.kz) - sel3(r.o, r.kz);
+  e.A_z = sel3(v, r.kz) - sel3(r.o, r.kz);
   const double B_x = sel3(v + 3, r.kx) - sel3(r.o, r.kx);
   const double B_y = sel3(v + 3, r.ky) - sel3(r.o, r.ky);
-  const double B_z = sel3(v + 3, r.kz) - sel3(r.o, r.kz);
+  e.B_z = sel3(v + 3, r.kz) - sel3(r.o, r.kz);
   const double C_x = sel3(v + 6, r.kx) - sel3(r.o, r.kx);
   const double C_y = sel3(v + 6, r.ky) - sel3(r.o, r.ky);
-  const double C_z = sel3(v + 6, r.kz) - sel3(r.o, r.kz);
-  const double Ax = A_x - r.Sx * A_z;
-  const double Ay = A_y - r.Sy * A_z;
-  const double Bx = B_x - r.Sx * B_z;
-  const double By = B_y - r.Sy * B_z;
-  const double Cx = C_x - r.Sx * C_z;
-  const double Cy = C_y - r.Sy * C_z;
-  const double U = Cx * By - Cy * Bx;
-  const double V = Ax * Cy - Ay * Cx;
-  const double W = Bx * Ay - By * Ax;
+  e.C_z = sel3(v + 6, r.kz) - sel3(r.o, r.kz);
+  const double Ax = A_x - r.Sx * e.A_z;
+  const double Ay = A_y - r.Sy * e.A_z;
+  const double Bx = B_x - r.Sx * e.B_z;
+  const double By = B_y - r.Sy * e.B_z;
+  const double Cx = C_x - r.Sx * e.C_z;
+  const double Cy = C_y - r.Sy * e.C_z;
+  e.U = Cx * By - Cy * Bx;
+  e.V = Ax * Cy - Ay * Cx;
+  e.W = Bx * Ay - By * Ax;
+  return e;
+}
+
+// Returns t >= 0 of the hit, or -1 for a miss.  v: 9 doubles (A, B, C).
+__device__ __forceinline__ double tri_hit(const Ray64 &r, const double *__restrict__ v) {
+  const TriEdges e = tri_edges(r, v);
+  const double U = e.U, V = e.V, W = e.W;
   if ((U < 0.0 || V < 0.0 || W < 0.0) && (U > 0.0 || V > 0.0 || W > 0.0)) return -1.0;
   const double det = U + V + W;
   if (det == 0.0) return -1.0;
-  const double Az = r.Sz * A_z;
-  const double Bz = r.Sz * B_z;
-  const double Cz = r.Sz * C_z;
+  const double Az = r.Sz * e.A_z;
+  const double Bz = r.Sz * e.B_z;
+  const double Cz = r.Sz * e.C_z;
   const double T = U * Az + V * Bz + W * Cz;
   const double t = T / det;
   if (!(t >= 0.0)) return -1.0;
@@ -228,39 +242,6 @@ __device__ inline void embree_sun_ray(const T *Pi, const T *Ni, const double *D,
     o[c] = (double)(float)oc;
     d[c] = (double)(float)D[c];
   }
-}
-
-// Facet-to-facet visibility of facet i -> facet j.
-//   CGAL mode (aabb_wrapper.cpp:64-93): origin = FP64 centroid of i,
-//   direction = centroid_j - centroid_i, i skipped, visible iff j is the
-//   closest hit; i == j -> false.
-//   EMBREE mode (shape.py:349-398): the ray of embree_pair_ray from the
-//   model centroids Pi, Pj (read in this mode only), nothing skipped,
-//   visible iff j is the closest hit.
-template <typename T>
-__device__ inline bool face_to_face_vis(const flux_scene &S, int i, int j, int mode,
-                                        const T *Pi, const T *Pj) {
-  double o[3], d[3];
-  int skip = -1;
-  if (mode == FLUX_MODE_CGAL) {
-    if (i == j) return false;
-    const double *ci = S.cen + (int64_t)i * 3;
-    const double *cj = S.cen + (int64_t)j * 3;
-    for (int c = 0; c < 3; ++c) {
-      o[c] = ci[c];
-      d[c] = cj[c] - ci[c];
-    }
-    skip = i;
-  } else {
-    if (!embree_pair_ray(Pi, Pj, o, d)) return true;
-  }
-  Ray64 r;
-  ray_setup(r, o, d);
-  double tj = tri_hit(r, S.tri + (int64_t)j * 9);
-  if (tj < 0.0) return false;
-  RayBox rb;
-  raybox_setup(rb, o, d);
-  return !any_blocker(S, r, rb, tj, j, skip, j);
 }
 
 template <typename T>

@@ -1,67 +1,124 @@
 // Visibility, sun occlusion and single-ray queries on a scene.
-#include "ray.h"
+#include "wide.h"
 
 namespace flux {
 
-// One thread per (p, q) pair; rays of a workgroup share the source facet
-// I[p], so their traversals stay coherent.
-template <typename T>
-__global__ void k_vis_mn(flux_scene S, const int64_t *__restrict__ I, int64_t m,
-                         const int64_t *__restrict__ J, int64_t n, int mode,
-                         const T *__restrict__ Pm, uint8_t *__restrict__ out) {
-  int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  int64_t p = blockIdx.y + (int64_t)blockIdx.z * 65535;
-  if (q >= n || p >= m) return;
-  if (I[p] < 0 || I[p] >= S.nf || J[q] < 0 || J[q] >= S.nf) {
-    out[p * n + q] = 0;
-    return;
-  }
-  int i = (int)I[p], j = (int)J[q];
-  T pi[3] = {0, 0, 0}, pj[3] = {0, 0, 0};
-  if (mode == FLUX_MODE_EMBREE) {
-    for (int c = 0; c < 3; ++c) {
-      pi[c] = Pm[(int64_t)i * 3 + c];
-      pj[c] = Pm[(int64_t)j * 3 + c];
-    }
-  }
-  out[p * n + q] = face_to_face_vis(S, i, j, mode, pi, pj) ? 1 : 0;
+template <typename Query>
+__global__ void __launch_bounds__(256, 5) k_query(flux_scene S, Query q, int64_t total,
+                                                  int64_t block) {
+  __shared__ int stack[4][kWideStack][64];
+  IndexSource<Query> src;
+  src.init(q, total, block);
+  trace_wave(S, src, &stack[threadIdx.x >> 6][0][threadIdx.x & 63]);
 }
 
-// occlusion: CGAL mode ray from the FP64 centroid, facet skipped
-// (aabb_wrapper.cpp:95-108); EMBREE mode from P + 1e-3 N, nothing skipped
-// (shape.py:400-421).
+template <typename Query>
+static int launch_query(const flux_scene *scene, const Query &q, int64_t total, hipStream_t st) {
+  const int64_t block = trace_block(total);
+  hipLaunchKernelGGL(k_query<Query>, dim3(trace_groups((total + block - 1) / block)), dim3(256),
+                     0, st, *scene, q, total, block);
+  FLUX_LAUNCH_CHECK();
+  return 0;
+}
+
+// Facet-to-facet visibility of the pairs (p, q), row by row: consecutive
+// rays share their source facet.
 template <typename T>
-__global__ void k_occluded(flux_scene S, const int64_t *__restrict__ I, int64_t m,
-                           const double *__restrict__ D, int64_t M, int per_face,
-                           int mode, const T *__restrict__ Nrm,
-                           const T *__restrict__ Pm, uint8_t *__restrict__ out) {
-  int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  int64_t cols = per_face ? 1 : M;
-  if (idx >= m * cols) return;
-  int64_t p = idx / cols, q = idx % cols;
-  if (I[p] < 0 || I[p] >= S.nf) {
-    out[idx] = 0;
-    return;
+struct VisQuery {
+  const int64_t *I, *J;
+  int64_t n;
+  int mode;
+  const T *P;
+  uint8_t *out;
+
+  __device__ __forceinline__ void begin(const flux_scene &S, LaneRay &L, int64_t r) const {
+    const int64_t p = r / n, i64 = I[p], j64 = J[r - p * n];
+    L.cur = kLaneBlocked;
+    if (i64 < 0 || i64 >= S.nf || j64 < 0 || j64 >= S.nf) return;
+    const int i = (int)i64, j = (int)j64;
+    T pi[3] = {0, 0, 0}, pj[3] = {0, 0, 0};
+    if (mode == FLUX_MODE_EMBREE)
+      for (int c = 0; c < 3; ++c) {
+        pi[c] = P[i64 * 3 + c];
+        pj[c] = P[j64 * 3 + c];
+      }
+    pair_begin(S, L, i, j, mode, pi, pj);
   }
-  int i = (int)I[p];
-  const double *dq = D + (per_face ? p : q) * 3;
-  double o[3], d[3] = {dq[0], dq[1], dq[2]};
+  __device__ __forceinline__ void end(const flux_scene &, int64_t r, bool blocked) const {
+    out[r] = blocked ? 0 : 1;
+  }
+};
+
+// The ray from facet f towards a direction d: CGAL mode from the FP64
+// centroid, facet skipped (aabb_wrapper.cpp:95-108); EMBREE mode from
+// P + 1e-3 N, nothing skipped (shape.py:400-421).
+template <typename T>
+__device__ __forceinline__ void sun_begin(const flux_scene &S, LaneRay &L, int64_t f,
+                                          const double *dir, int mode, const T *P, const T *N) {
+  double o[3], d[3] = {dir[0], dir[1], dir[2]};
   int skip = -1;
   if (mode == FLUX_MODE_CGAL) {
-    const double *ci = S.cen + (int64_t)i * 3;
-    o[0] = ci[0];
-    o[1] = ci[1];
-    o[2] = ci[2];
-    skip = i;
+    for (int c = 0; c < 3; ++c) o[c] = S.cen[f * 3 + c];
+    skip = (int)f;
   } else {
-    embree_sun_ray(Pm + (int64_t)i * 3, Nrm + (int64_t)i * 3, dq, o, d);
+    embree_sun_ray(P + f * 3, N + f * 3, dir, o, d);
   }
-  Ray64 r;
-  ray_setup(r, o, d);
-  RayBox rb;
-  raybox_setup(rb, o, d);
-  out[idx] = any_blocker(S, r, rb, INFINITY, 0x7fffffff, skip, -1) ? 1 : 0;
+  ray_setup(L.r, o, d);
+  lane_begin(S, L, o, d, INFINITY, 0x7fffffff, skip, -1);
 }
+
+// Occlusion of facet I[p] towards D[q] (or D[p]): all facets of one
+// direction after the other, so a wave's rays run in parallel.
+template <typename T>
+struct OccQuery {
+  const int64_t *I;
+  int64_t m;
+  const double *D;
+  int64_t M;
+  int per_face, mode;
+  const T *Nrm, *P;
+  uint8_t *out;
+
+  __device__ __forceinline__ void begin(const flux_scene &S, LaneRay &L, int64_t r) const {
+    const int64_t q = r / m, p = r - q * m, f = I[p];
+    L.cur = kLaneVisible;
+    if (f < 0 || f >= S.nf) return;
+    sun_begin(S, L, f, D + (per_face ? p : q) * 3, mode, P, Nrm);
+  }
+  __device__ __forceinline__ void end(const flux_scene &, int64_t r, bool blocked) const {
+    const int64_t q = r / m, p = r - q * m;
+    out[per_face ? p : p * M + q] = blocked ? 1 : 0;
+  }
+};
+
+// E[f, k] = F0 * max(0, N_f . d_k) if facet f sees sun k, else 0: the 1-D
+// sun branch of get_direct_irradiance (shape.py:224-226) for M suns at once.
+// The dot product is taken in FP64 (N . Dsun of a mesh-dtype N with an FP64
+// direction promotes to FP64 in NumPy) and stored in the mesh dtype.  The
+// rays go out sun by sun in Morton order of the facets: neighbours in a wave
+// walk the same nodes.
+template <typename T>
+struct IrradianceQuery {
+  const T *Nrm, *P;
+  const double *D;
+  int64_t M;
+  double F0;
+  int mode;
+  T *E;
+
+  __device__ __forceinline__ void begin(const flux_scene &S, LaneRay &L, int64_t r) const {
+    const int64_t k = r / S.nf;
+    sun_begin(S, L, S.order[r - k * S.nf], D + k * 3, mode, P, Nrm);
+  }
+  __device__ __forceinline__ void end(const flux_scene &S, int64_t r, bool blocked) const {
+    const int64_t k = r / S.nf, f = S.order[r - k * S.nf];
+    const double *d = D + k * 3;
+    double nf3[3];
+    load3(Nrm, f, nf3);
+    const double cosi = (nf3[0] * d[0] + nf3[1] * d[1]) + nf3[2] * d[2];
+    E[f * M + k] = blocked ? (T)0 : (T)(F0 * (cosi > 0.0 ? cosi : 0.0));
+  }
+};
 
 __global__ void k_intersect1(flux_scene S, const double *__restrict__ x,
                              const double *__restrict__ d, int64_t nr,
@@ -80,37 +137,6 @@ __global__ void k_intersect1(flux_scene S, const double *__restrict__ x,
   for (int c = 0; c < 3; ++c) xt[k * 3 + c] = h >= 0 ? o[c] + t * dd[c] : 0.0;
 }
 
-// E[f, k] = F0 * max(0, N_f . d_k) if facet f sees sun k, else 0: the 1-D
-// sun branch of get_direct_irradiance (shape.py:224-226) for M suns at once.
-// The dot product is taken in FP64 (N . Dsun of a mesh-dtype N with an FP64
-// direction promotes to FP64 in NumPy) and stored in the mesh dtype.
-template <typename T>
-__global__ void k_direct_irradiance(flux_scene S, const T *__restrict__ Nrm,
-                                    const T *__restrict__ Pm, const double *__restrict__ D,
-                                    int64_t M, double F0, int mode, T *__restrict__ E) {
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= S.nf * M) return;
-  const int64_t f = idx / M, k = idx % M;
-  const double d[3] = {D[k * 3], D[k * 3 + 1], D[k * 3 + 2]};
-  double nf3[3];
-  load3(Nrm, f, nf3);
-  double o[3];
-  int skip = -1;
-  if (mode == FLUX_MODE_CGAL) {
-    for (int c = 0; c < 3; ++c) o[c] = S.cen[f * 3 + c];
-    skip = (int)f;
-  }
-  double dr[3] = {d[0], d[1], d[2]};  // the ray's direction (FP32 in EMBREE mode)
-  if (mode != FLUX_MODE_CGAL) embree_sun_ray(Pm + f * 3, Nrm + f * 3, d, o, dr);
-  Ray64 r;
-  ray_setup(r, o, dr);
-  RayBox rb;
-  raybox_setup(rb, o, dr);
-  const bool occ = any_blocker(S, r, rb, INFINITY, 0x7fffffff, skip, -1);
-  const double cosi = (nf3[0] * d[0] + nf3[1] * d[1]) + nf3[2] * d[2];
-  E[idx] = occ ? (T)0 : (T)(F0 * (cosi > 0.0 ? cosi : 0.0));
-}
-
 }  // namespace flux
 
 using namespace flux;
@@ -127,18 +153,16 @@ extern "C" int flux_direct_irradiance(const flux_scene *scene, const void *P, co
   if (total == 0) return 0;
   FLUX_CHECK(Nrm && D && E && (mode == FLUX_MODE_CGAL || P),
              "flux_direct_irradiance: NULL array");
-  const int TB = 256;
   hipStream_t st = as_stream(stream);
   if (dtype == FLUX_F64)
-    hipLaunchKernelGGL(k_direct_irradiance<double>, dim3(ceil_div_u(total, TB)), dim3(TB), 0, st,
-                       *scene, (const double *)Nrm, (const double *)P, D, M, F0, mode,
-                       (double *)E);
-  else
-    hipLaunchKernelGGL(k_direct_irradiance<float>, dim3(ceil_div_u(total, TB)), dim3(TB), 0, st,
-                       *scene, (const float *)Nrm, (const float *)P, D, M, F0, mode,
-                       (float *)E);
-  FLUX_LAUNCH_CHECK();
-  return 0;
+    return launch_query(scene,
+                        IrradianceQuery<double>{(const double *)Nrm, (const double *)P, D, M, F0,
+                                                mode, (double *)E},
+                        total, st);
+  return launch_query(scene,
+                      IrradianceQuery<float>{(const float *)Nrm, (const float *)P, D, M, F0, mode,
+                                             (float *)E},
+                      total, st);
 }
 
 extern "C" int flux_vis_mn(const flux_scene *scene, const int64_t *I, int64_t m,
@@ -154,17 +178,10 @@ extern "C" int flux_vis_mn(const flux_scene *scene, const int64_t *I, int64_t m,
   FLUX_CHECK(I && J && out, "flux_vis_mn: NULL array");
   FLUX_CHECK(m <= (int64_t)65535 * 65535, "flux_vis_mn: m too large");
   hipStream_t st = as_stream(stream);
-  const int TB = 256;
-  dim3 grid(ceil_div_u(n, TB), (unsigned)(m < 65535 ? m : 65535),
-            (unsigned)((m + 65534) / 65535));
   if (dtype == FLUX_F64)
-    hipLaunchKernelGGL(k_vis_mn<double>, grid, dim3(TB), 0, st, *scene, I, m, J, n, mode,
-                       (const double *)P, out);
-  else
-    hipLaunchKernelGGL(k_vis_mn<float>, grid, dim3(TB), 0, st, *scene, I, m, J, n, mode,
-                       (const float *)P, out);
-  FLUX_LAUNCH_CHECK();
-  return 0;
+    return launch_query(scene, VisQuery<double>{I, J, n, mode, (const double *)P, out}, m * n,
+                        st);
+  return launch_query(scene, VisQuery<float>{I, J, n, mode, (const float *)P, out}, m * n, st);
 }
 
 extern "C" int flux_occluded(const flux_scene *scene, const int64_t *I, int64_t m,
@@ -182,18 +199,16 @@ extern "C" int flux_occluded(const flux_scene *scene, const int64_t *I, int64_t 
   FLUX_CHECK(mode == FLUX_MODE_CGAL || (Nrm != nullptr && P != nullptr),
              "flux_occluded: EMBREE mode needs P and N");
   hipStream_t st = as_stream(stream);
-  const int TB = 256;
-  int64_t total = m * (per_face ? 1 : M);
+  const int64_t total = m * (per_face ? 1 : M);
   if (dtype == FLUX_F64)
-    hipLaunchKernelGGL(k_occluded<double>, dim3(ceil_div_u(total, TB)), dim3(TB), 0, st,
-                       *scene, I, m, D, M, per_face, mode, (const double *)Nrm,
-                       (const double *)P, out);
-  else
-    hipLaunchKernelGGL(k_occluded<float>, dim3(ceil_div_u(total, TB)), dim3(TB), 0, st,
-                       *scene, I, m, D, M, per_face, mode, (const float *)Nrm,
-                       (const float *)P, out);
-  FLUX_LAUNCH_CHECK();
-  return 0;
+    return launch_query(scene,
+                        OccQuery<double>{I, m, D, M, per_face, mode, (const double *)Nrm,
+                                         (const double *)P, out},
+                        total, st);
+  return launch_query(scene,
+                      OccQuery<float>{I, m, D, M, per_face, mode, (const float *)Nrm,
+                                      (const float *)P, out},
+                      total, st);
 }
 
 extern "C" int flux_intersect1(const flux_scene *scene, const double *x, const double *d,

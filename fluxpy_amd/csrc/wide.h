@@ -1,0 +1,296 @@
+// Four-wide BVH and the wave-scheduled any-hit traversal behind the
+// form-factor mask, the visibility matrix and the sun queries.
+//
+// A walk of the binary preorder layouts (ray.h) takes about 80 dependent
+// node loads per facet-to-facet ray of a terrain, and in a wave of such
+// walks nearly every step has a few lanes at a leaf, so the FP64 triangle
+// test runs with 3 or 4 of 64 lanes active.  Here
+//  * a node holds the quantised boxes of up to four children in 64 bytes
+//    (one cache line segment, four 16-byte loads), which cuts the dependent
+//    loads per ray to about 21 nodes + 5 triangles;
+//  * each lane is at a node, at a leaf or without work, and every iteration
+//    of the wave runs one of the two steps, for the larger group;
+//  * lanes whose ray has ended take new rays once a quarter of the wave is
+//    out of work, instead of waiting for the longest ray of 64.
+//
+// Decisions do not depend on any of this: the set of triangles tested always
+// contains every triangle the FP64 test hits on the queried segment (the
+// quantised boxes contain the padded FP32 boxes), and a query's answer is a
+// property of that set.
+#pragma once
+#include "ray.h"
+
+namespace flux {
+
+// Child codes: >= 0 a wide node, < 0 the leaf of triangle ~code.  Lane
+// states below every leaf code (facet counts are below 2^30):
+constexpr int kLaneIdle = INT32_MIN;         // no ray
+constexpr int kLaneVisible = INT32_MIN + 1;  // walk ended without a blocker
+constexpr int kLaneBlocked = INT32_MIN + 2;  // a blocker was found
+constexpr int kLaneDone = INT32_MIN + 2;     // states <= kLaneDone have no step to run
+
+// Deferred children per lane (LDS, 256 B per entry and wave).  Terrains of
+// 41k facets reach 14, a walk that would need more marks itself and is
+// repeated on the stackless layout.
+constexpr int kWideStack = 24;
+// Out-of-work lanes that trigger a refill: a refill's ray set-up costs about
+// one node step, whatever the number of lanes it serves.
+constexpr int kRefill = 16;
+
+enum : int { kFlagLost = 4 };
+
+struct LaneRay {
+  Ray64 r;
+  float inv[3];
+  float tmax;
+  double tlim;   // hits at (t, k) before (tlim, klim) block
+  int klim;
+  int skip1, skip2;
+  int cur, sp, flags;
+};
+
+__device__ __forceinline__ void lane_begin(const flux_scene &S, LaneRay &L, const double o[3],
+                                           const double d[3], double tlim, int klim, int skip1,
+                                           int skip2) {
+  RayBox rb;
+  raybox_setup(rb, o, d);
+  for (int c = 0; c < 3; ++c) L.inv[c] = fminf(fmaxf(rb.inv[c], -S.inv_max), S.inv_max);
+  L.tmax = isinf(tlim) ? 3.0e38f : (float)(tlim * (1.0 + 1e-5)) + 1e-30f;
+  L.tlim = tlim;
+  L.klim = klim;
+  L.skip1 = skip1;
+  L.skip2 = skip2;
+  L.sp = 0;
+  L.cur = S.root;
+}
+
+// The ray that decides whether facet i sees facet j; a pair decided without
+// a walk leaves the lane visible or blocked.
+//   CGAL mode (aabb_wrapper.cpp:64-93): origin = FP64 centroid of i,
+//   direction = centroid_j - centroid_i, i skipped, visible iff j is the
+//   closest hit; i == j -> false.
+//   EMBREE mode (shape.py:349-398): the ray of embree_pair_ray from the
+//   model centroids Pi, Pj (read in this mode only), nothing skipped,
+//   visible iff j is the closest hit.
+template <typename T>
+__device__ __forceinline__ void pair_begin(const flux_scene &S, LaneRay &L, int i, int j,
+                                           int mode, const T *Pi, const T *Pj) {
+  double o[3], d[3];
+  int skip = -1;
+  L.cur = kLaneBlocked;
+  if (mode == FLUX_MODE_CGAL) {
+    if (i == j) return;
+    const double *ci = S.cen + (int64_t)i * 3, *cj = S.cen + (int64_t)j * 3;
+    for (int c = 0; c < 3; ++c) {
+      o[c] = ci[c];
+      d[c] = cj[c] - ci[c];
+    }
+    skip = i;
+  } else if (!embree_pair_ray(Pi, Pj, o, d)) {
+    L.cur = kLaneVisible;
+    return;
+  }
+  ray_setup(L.r, o, d);
+  const double tj = tri_hit(L.r, S.tri + (int64_t)j * 9);
+  if (tj >= 0.0) lane_begin(S, L, o, d, tj, j, skip, j);
+}
+
+__device__ __forceinline__ void lane_pop(LaneRay &L, const int *stk) {
+  if (L.sp > 0) {
+    --L.sp;
+    L.cur = stk[L.sp * 64];
+  } else {
+    L.cur = kLaneVisible;
+  }
+}
+
+// One child word per axis and side: byte c is the quantised plane of child c.
+__device__ __forceinline__ float plane(uint32_t w, int c, float s, float b) {
+  return fmaf((float)((w >> (8 * c)) & 0xffu), s, b);
+}
+
+// The lane's node: test the four children, go on with the first one hit in
+// the node's order for the ray's octant and defer the others (stk: the
+// lane's column of the wave's stack).
+__device__ __forceinline__ void lane_node(const flux_scene &S, LaneRay &L, int *stk) {
+  const uint4 *nd = S.wide + (int64_t)L.cur * 4;
+  const uint4 n0 = nd[0], n1 = nd[1], n2 = nd[2], n3 = nd[3];
+  const float sx = __uint_as_float((n0.w & 0xffu) << 23) * L.inv[0];
+  const float sy = __uint_as_float(((n0.w >> 8) & 0xffu) << 23) * L.inv[1];
+  const float sz = __uint_as_float(((n0.w >> 16) & 0xffu) << 23) * L.inv[2];
+  const float bx = (__uint_as_float(n0.x) - (float)L.r.o[0]) * L.inv[0];
+  const float by = (__uint_as_float(n0.y) - (float)L.r.o[1]) * L.inv[1];
+  const float bz = (__uint_as_float(n0.z) - (float)L.r.o[2]) * L.inv[2];
+  const bool gx = L.inv[0] < 0.0f, gy = L.inv[1] < 0.0f, gz = L.inv[2] < 0.0f;
+  const uint32_t ax = gx ? n2.w : n2.x, fx = gx ? n2.x : n2.w;
+  const uint32_t ay = gy ? n3.x : n2.y, fy = gy ? n2.y : n3.x;
+  const uint32_t az = gz ? n3.y : n2.z, fz = gz ? n2.z : n3.y;
+  uint32_t hit = 0;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const float tn = fmaxf(fmaxf(plane(ax, c, sx, bx), plane(ay, c, sy, by)),
+                           fmaxf(plane(az, c, sz, bz), 0.0f));
+    const float tf = fminf(fminf(plane(fx, c, sx, bx), plane(fy, c, sy, by)),
+                           fminf(plane(fz, c, sz, bz), L.tmax));
+    hit |= tn <= tf ? 1u << c : 0u;
+  }
+  hit &= n0.w >> 24;  // slots in use
+  const uint32_t ow = gz ? n3.w : n3.z;
+  const uint32_t ord = ow >> ((gx ? 8 : 0) + (gy ? 16 : 0));
+  // visit order back to front: what is left in `next` at the end is the
+  // first child hit
+  int next = kLaneIdle;
+#pragma unroll
+  for (int k = 3; k >= 0; --k) {
+    const uint32_t s = (ord >> (2 * k)) & 3u;
+    if ((hit >> s) & 1u) {
+      if (next != kLaneIdle) {
+        if (L.sp < kWideStack) {
+          stk[L.sp * 64] = next;
+          ++L.sp;
+        } else {
+          L.flags |= kFlagLost;
+        }
+      }
+      next = (int)(s < 2 ? (s == 0 ? n1.x : n1.y) : (s == 2 ? n1.z : n1.w));
+    }
+  }
+  if (next != kLaneIdle)
+    L.cur = next;
+  else
+    lane_pop(L, stk);
+}
+
+// The lane's leaf, for queries that stop at the first blocker.
+__device__ __forceinline__ void lane_leaf(const flux_scene &S, LaneRay &L, const int *stk) {
+  const int t = ~L.cur;
+  bool block = false;
+  if (t != L.skip1 && t != L.skip2) {
+    const double th = tri_hit(L.r, S.tri + (int64_t)t * 9);
+    block = th >= 0.0 && (th < L.tlim || (th == L.tlim && t < L.klim));
+  }
+  if (block)
+    L.cur = kLaneBlocked;
+  else
+    lane_pop(L, stk);
+}
+
+// A walk that ran out of stack has skipped children: repeat it on the
+// stackless layout unless it found a blocker anyway.
+__device__ __forceinline__ void lane_recover(const flux_scene &S, LaneRay &L) {
+  if (L.cur == kLaneVisible && (L.flags & kFlagLost)) {
+    RayBox rb;
+    for (int c = 0; c < 3; ++c) {
+      rb.o[c] = (float)L.r.o[c];
+      rb.inv[c] = L.inv[c];
+    }
+    if (any_blocker(S, L.r, rb, L.tlim, L.klim, L.skip1, L.skip2)) L.cur = kLaneBlocked;
+  }
+  L.flags &= ~kFlagLost;
+}
+
+// The wave's loop.  src.refill(S, L) ends the rays of done lanes, hands new
+// ones out and returns false once no lane of the wave has one and none are
+// left; src.drained() says that none are left to hand out.
+template <typename Src>
+__device__ __forceinline__ void trace_wave(const flux_scene &S, Src &src, int *stk) {
+  LaneRay L;
+  L.cur = kLaneIdle;
+  L.sp = 0;
+  L.flags = 0;
+  while (true) {
+    const int nn = __popcll(__ballot(L.cur >= 0));
+    const int nl = __popcll(__ballot(L.cur < 0 && L.cur > kLaneDone));
+    if (nn + nl == 0 || (nn + nl <= 64 - kRefill && !src.drained())) {
+      lane_recover(S, L);
+      if (!src.refill(S, L)) break;
+      continue;
+    }
+    if (nn >= nl) {
+      if (L.cur >= 0) lane_node(S, L, stk);
+    } else {
+      if (L.cur < 0 && L.cur > kLaneDone) src.leaf(S, L, stk);
+    }
+  }
+}
+
+// LDS written by some lanes of the wave is read by others (the wave's LDS
+// operations complete in order; this keeps the compiler's order too).
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Index of this lane among the set lanes of m.
+__device__ __forceinline__ int lane_rank(uint64_t m) {
+  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                        __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+// Rays numbered 0 .. total - 1 for trace_wave: a wave takes blocks of
+// `block` consecutive rays, `nwaves` blocks apart.  Query::begin sets up ray
+// r and Query::end stores its answer (every ray has begin, then end).
+template <typename Query>
+struct IndexSource {
+  Query q;
+  int64_t total, block, stride, base, next, stop;
+  int64_t ray;  // the lane's
+
+  __device__ __forceinline__ void init(const Query &query, int64_t n, int64_t blk) {
+    q = query;
+    total = n;
+    block = blk;
+    const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    stride = (((int64_t)gridDim.x * blockDim.x) >> 6) * blk;
+    base = wave * blk;
+    next = min(base, total);
+    stop = min(base + blk, total);
+    ray = 0;
+  }
+
+  __device__ __forceinline__ bool drained() const { return next >= stop; }
+
+  __device__ __forceinline__ bool refill(const flux_scene &S, LaneRay &L) {
+    if (L.cur == kLaneVisible || L.cur == kLaneBlocked) q.end(S, ray, L.cur == kLaneBlocked);
+    if (L.cur <= kLaneDone) L.cur = kLaneIdle;
+    const uint64_t idle = __ballot(L.cur == kLaneIdle);
+    const int want = __popcll(idle);
+    const int rank = L.cur == kLaneIdle ? lane_rank(idle) : -1;
+    int given = 0;
+    while (given < want && next < stop) {
+      const int take = (int)min((int64_t)(want - given), stop - next);
+      if (rank >= given && rank < given + take) {
+        ray = next + (rank - given);
+        q.begin(S, L, ray);
+      }
+      given += take;
+      next += take;
+      if (next >= stop) {
+        base += stride;
+        next = min(base, total);
+        stop = min(base + block, total);
+      }
+    }
+    return given > 0 || __ballot(L.cur > kLaneIdle) != 0;
+  }
+
+  __device__ __forceinline__ void leaf(const flux_scene &S, LaneRay &L, const int *stk) {
+    lane_leaf(S, L, stk);
+  }
+};
+
+// Rays per block: a full wave's, or fewer so that a small query spreads over
+// the chip (its time is its longest walk, which lanes at other steps delay).
+static inline int64_t trace_block(int64_t total) {
+  const int64_t b = total / (1280 * 4);
+  return b < 8 ? 8 : (b < 64 ? b : 64);
+}
+
+// Workgroups of four waves that fill the chip (20 waves a CU: 102 VGPRs and
+// 8 KB of LDS each), or as many as there is work for.
+static inline unsigned trace_groups(int64_t wave_items) {
+  const int64_t g = (wave_items + 3) / 4;
+  return (unsigned)(g < 1 ? 1 : (g < 1280 ? g : 1280));
+}
+
+}  // namespace flux

@@ -1,0 +1,81 @@
+"""The four-wide BVH walk against the CPU oracle, bit for bit, where it can
+go wrong: trees of a few facets (a root that is a leaf, nodes with empty
+slots), meshes without extent along an axis, coordinates of very different
+size, rays along an axis, and walks that need more deferred children than
+the stack holds."""
+import numpy as np
+import pytest
+
+from fluxpy_amd import meshes
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch_dev():
+    import torch
+    torch.cuda.set_device(0)
+    return torch
+
+
+def _soup(nf, seed, scale=1.0, offset=0.0, flat=False):
+    """Random triangles, many of them large enough to overlap each other."""
+    rng = np.random.default_rng(seed)
+    c = rng.uniform(-1, 1, (nf, 1, 3))
+    s = np.exp(rng.uniform(np.log(0.01), np.log(1.5), (nf, 1, 1)))
+    V = (c + s * rng.uniform(-1, 1, (nf, 3, 3))) * scale + offset
+    if flat:
+        V[..., 2] = offset
+    return V.reshape(-1, 3), np.arange(3 * nf).reshape(nf, 3)
+
+
+def deep_mesh():
+    """16,000 large triangles whose centroids halve their distance to a
+    corner again and again and then coincide, so the Morton tree is a chain
+    of clusters over a deep balanced part; every box is as wide as the mesh
+    and the planes are parallel, so a walk defers nearly all it meets."""
+    rng = np.random.default_rng(3)
+    t = np.concatenate([np.full(16, 0.9 * 0.5 ** k) for k in range(11)]
+                       + [np.full(1 << 14, 2e-4)])
+    n = t.size
+    c = t[:, None] * np.array([1.0, 1.0, 0.3])
+    a = rng.uniform(-2, 2, (n, 2, 2))
+    e = np.stack([a[..., 0], a[..., 1], a[..., 0]], -1)     # in the planes z = x + const
+    V = np.stack([c + e[:, 0], c + e[:, 1], c - e[:, 0] - e[:, 1]], 1)
+    return V.reshape(-1, 3), np.arange(3 * n).reshape(n, 3)
+
+
+@pytest.mark.parametrize("cls", ["cgal", "embree"])
+@pytest.mark.parametrize("nf,kw", [
+    (1, {}), (2, {}), (3, {}), (4, {}), (5, {}), (17, {}), (200, {}),
+    (60, {"flat": True}), (60, {"scale": 1e6, "offset": 3e7}), (60, {"scale": 1e-4})])
+def test_soup_matches_oracle(torch_dev, oracle_mod, nf, kw, cls):
+    from fluxpy_amd.shape import CgalTrimeshShapeModel, EmbreeTrimeshShapeModel
+    V, F = _soup(nf, 100 + nf, **kw)
+    sm = (CgalTrimeshShapeModel if cls == "cgal" else EmbreeTrimeshShapeModel)(V, F)
+    S = oracle_mod.OracleScene(V, F)
+    I = np.arange(nf)
+    if cls == "cgal":
+        assert np.array_equal(sm.get_visibility_matrix(), S.vis_mn(I, I))
+    else:
+        assert np.array_equal(sm.get_visibility_matrix(), S.vis_mn(I, I, mode=oracle_mod.MODE_EMBREE, P=sm.P))
+    D = np.concatenate([np.eye(3), -np.eye(3), [[1.0, 0, 1e-9], [0, 1e-300, 1.0]],
+                        meshes.sun_directions(5, seed=nf)])
+    for d in D:
+        if cls == "cgal":
+            want = S.occluded(I, d)[:, 0]
+        else:
+            want = S.occluded(I, d, mode=oracle_mod.MODE_EMBREE, P=sm.P, N=sm.N)[:, 0]
+        assert np.array_equal(sm.is_occluded(I, d), want)
+
+
+def test_stack_overflow_matches_oracle(torch_dev, oracle_mod):
+    from fluxpy_amd.shape import CgalTrimeshShapeModel
+    V, F = deep_mesh()
+    sm = CgalTrimeshShapeModel(V, F)
+    S = oracle_mod.OracleScene(V, F)
+    I = np.concatenate([np.arange(0, 176, 5), np.arange(176, len(F), 401)])
+    for d in ([1.0, 0.13, 1.0], [-1.0, 0.4, -1.0], [0.02, 1.0, 0.02], [0.3, -0.2, 1.0]):
+        d = np.array(d) / np.linalg.norm(d)
+        assert np.array_equal(sm.is_occluded(I, d), S.occluded(I, d)[:, 0])
+    assert np.array_equal(sm.get_visibility(I, I), S.vis_mn(I, I))
