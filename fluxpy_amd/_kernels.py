@@ -128,16 +128,26 @@ def ff_csr(shape_model, I=None, J=None, eps=None, dtype=None):
     st = _lib.stream()
     code = _lib.dtype_code(mdt)
     rows_per_chunk = max(1, min(m, _MASK_BYTES // max(1, W * 8)))
+    # One list for rows and columns: the CGAL rays of (i, j) and (j, i) run
+    # along one line, and the mask is built from half of them.
+    square = (rows_per_chunk == m == n and shape_model._mode == _lib.MODE_CGAL
+              and np.array_equal(I, J))
+    whole = square and n == nf and bool((I == np.arange(nf)).all())
     parts = []
     for r0 in range(0, m, rows_per_chunk):
         Ic = I[r0:r0 + rows_per_chunk]
         mc = Ic.size
-        Id = _lib.to_dev(Ic)
+        Id = Jd if square else _lib.to_dev(Ic)
         mask = t.empty((mc, max(W, 1)), dtype=t.int64, device=dev)
         row_nnz = t.empty(mc, dtype=t.int64, device=dev)
-        _lib.call("flux_ff_mask", shape_model._scene.handle, P.data_ptr(), N.data_ptr(), code,
-                  Id.data_ptr(), mc, Jd.data_ptr(), n, float(eps), shape_model._mode,
-                  mask.data_ptr(), row_nnz.data_ptr(), st)
+        if square:
+            _lib.call("flux_ff_mask_square", shape_model._scene.handle, P.data_ptr(),
+                      N.data_ptr(), code, None if whole else Id.data_ptr(), n, float(eps),
+                      mask.data_ptr(), row_nnz.data_ptr(), st)
+        else:
+            _lib.call("flux_ff_mask", shape_model._scene.handle, P.data_ptr(), N.data_ptr(),
+                      code, Id.data_ptr(), mc, Jd.data_ptr(), n, float(eps), shape_model._mode,
+                      mask.data_ptr(), row_nnz.data_ptr(), st)
         indptr = t.empty(mc + 1, dtype=t.int64, device=dev)
         total = _lib.ctypes.c_int64()
         _lib.call("flux_scan_i64", row_nnz.data_ptr(), mc, indptr.data_ptr(),

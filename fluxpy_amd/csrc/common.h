@@ -75,4 +75,5 @@ struct flux_scene {
   int32_t *order;  // facets in Morton order
   int32_t root;    // child code of the root (wide.h)
   float inv_max;   // bound on a ray's reciprocal direction in the slab tests
+  double edge_tol; // twelve times the rounding of an edge function (wide.h)
 };

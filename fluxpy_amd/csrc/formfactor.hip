@@ -266,6 +266,160 @@ __global__ void __launch_bounds__(256, 5) k_ff_mask_rays(
   trace_wave(S, src, &stack[wv][0][lane]);
 }
 
+// The same for all pairs of one list of n facets in CGAL mode, where the
+// rays i -> j and j -> i run along one line: one walk decides both unless
+// rounding may (wide.h), so the pairs s < t are walked once.  The list is
+// taken in Morton order of the facets (I == NULL: facet ids) or in its own
+// order (cluster order elsewhere).
+template <typename T>
+struct BothSource {
+  const T *P, *N;
+  const int64_t *I;
+  int64_t n, W, tile_words, tiles_per_row;
+  T eps;
+  uint64_t *mask;
+  TileWalk tiles;
+  int2 *queue;
+  int64_t s, w, wend;
+  int count, lane;
+  bool exhausted;
+  T Pi[3], Ni[3];
+  int i_row, p_row;
+  int lp, lq;
+
+  __device__ __forceinline__ bool drained() const { return exhausted && count == 0; }
+
+  // position and facet of place k of the walking order
+  __device__ __forceinline__ int place(const flux_scene &S, int64_t k) const {
+    return I ? (int)k : S.order[k];
+  }
+  __device__ __forceinline__ int facet(const flux_scene &S, int pos) const {
+    if (!I) return pos;
+    const int64_t i = I[pos];
+    return i >= 0 && i < S.nf ? (int)i : -1;
+  }
+
+  __device__ __forceinline__ bool next_tile(const flux_scene &S) {
+    const int64_t tile = tiles.next();
+    if (tile >= tiles.ntiles) return false;
+    s = tile / tiles_per_row;
+    w = (tile - s * tiles_per_row) * tile_words;
+    wend = min(W, w + tile_words);
+    w = max(w, (s + 1) >> 6);
+    p_row = place(S, s);
+    i_row = facet(S, p_row);
+    const int64_t i = i_row < 0 ? 0 : i_row;
+    for (int c = 0; c < 3; ++c) {
+      Pi[c] = P[i * 3 + c];
+      Ni[c] = N[i * 3 + c];
+    }
+    if (i_row < 0) w = wend;
+    return true;
+  }
+
+  __device__ __forceinline__ bool push_word(const flux_scene &S) {
+    while (w >= wend) {
+      if (!next_tile(S)) {
+        exhausted = true;
+        return false;
+      }
+    }
+    const int64_t t = w * 64 + lane;
+    ++w;
+    bool fwd = false, rev = false;
+    int q = 0;
+    if (t > s && t < n) {
+      q = place(S, t);
+      const int64_t j = facet(S, q);
+      if (j >= 0 && j != i_row) {
+        const T Pj[3] = {P[j * 3], P[j * 3 + 1], P[j * 3 + 2]};
+        const T Nj[3] = {N[j * 3], N[j * 3 + 1], N[j * 3 + 2]};
+        fwd = ff_prefilter(Pi, Ni, Pj, Nj) > eps;
+        rev = ff_prefilter(Pj, Nj, Pi, Ni) > eps;
+      }
+    }
+    const uint64_t bal = __ballot(fwd || rev);
+    // bit 30: both directions need a ray; else the pair is stored the way
+    // round that does
+    if (fwd || rev)
+      queue[count + lane_rank(bal)] =
+          fwd ? make_int2(p_row | (rev ? 1 << 30 : 0), q) : make_int2(q, p_row);
+    count += __popcll(bal);
+    return true;
+  }
+
+  __device__ __forceinline__ void emit(int a, int b) {
+    atomicOr((unsigned long long *)&mask[(int64_t)a * W + (b >> 6)], 1ull << (b & 63));
+  }
+
+  __device__ __forceinline__ bool refill(const flux_scene &S, LaneRay &L) {
+    bool start = false, both = false;
+    if (L.cur == kLaneVisible || L.cur == kLaneBlocked) {
+      if (L.cur == kLaneVisible) {
+        emit(lp, lq);
+        if ((L.flags & (kFlagPair | kFlagReverse)) == kFlagPair) emit(lq, lp);
+      }
+      if (L.flags & kFlagReverse) {
+        const int a = lp;
+        lp = lq;
+        lq = a;
+        start = true;
+      }
+    }
+    if (L.cur <= kLaneDone) L.cur = kLaneIdle;
+    const bool free_lane = L.cur == kLaneIdle && !start;
+    const uint64_t idle = __ballot(free_lane);
+    const int want = __popcll(idle);
+    while (count < want && push_word(S)) {
+    }
+    wave_lds_order();
+    const int take = min(count, want), rank = lane_rank(idle);
+    if (free_lane && rank < take) {
+      const int2 e = queue[count - 1 - rank];
+      lp = e.x & ~(1 << 30);
+      lq = e.y;
+      both = (e.x >> 30) & 1;
+      start = true;
+    }
+    if (start) both_begin(S, L, facet(S, lp), facet(S, lq), both);
+    wave_lds_order();
+    count -= take;
+    return __ballot(L.cur > kLaneIdle) != 0 || !drained();
+  }
+
+  __device__ __forceinline__ void leaf(const flux_scene &S, LaneRay &L, const int *stk) {
+    both_leaf(S, L, stk);
+  }
+};
+
+template <typename T>
+__global__ void __launch_bounds__(256, 5) k_ff_mask_both(
+    flux_scene S, const T *__restrict__ P, const T *__restrict__ N,
+    const int64_t *__restrict__ I, int64_t n, T eps, uint64_t *__restrict__ mask, int64_t W,
+    int64_t tile_words, int64_t tiles_per_row, unsigned long long *__restrict__ counter) {
+  __shared__ int stack[4][kWideStack][64];
+  __shared__ int2 queue[4][kPairQueue];
+  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  BothSource<T> src;
+  src.P = P;
+  src.N = N;
+  src.I = I;
+  src.n = n;
+  src.W = W;
+  src.tile_words = tile_words;
+  src.tiles_per_row = tiles_per_row;
+  src.eps = eps;
+  src.mask = mask;
+  src.tiles.init(n * tiles_per_row, counter);
+  src.queue = queue[wv];
+  src.s = src.w = src.wend = 0;
+  src.count = 0;
+  src.lane = lane;
+  src.exhausted = false;
+  src.lp = src.lq = 0;
+  trace_wave(S, src, &stack[wv][0][lane]);
+}
+
 // mask and the tile counter set to zero (no memset: callers may capture)
 __global__ void k_mask_clear(uint64_t *__restrict__ mask, int64_t words,
                              unsigned long long *__restrict__ counter) {
@@ -421,6 +575,39 @@ extern "C" int flux_ff_mask(const flux_scene *scene, const void *P, const void *
   }
   hipLaunchKernelGGL(k_row_count, dim3(ceil_div_u(m, 4)), dim3(256), 0, st, mask, m, W,
                      row_nnz);
+  FLUX_LAUNCH_CHECK();
+  return 0;
+}
+
+extern "C" int flux_ff_mask_square(const flux_scene *scene, const void *P, const void *N,
+                                   int dtype, const int64_t *I, int64_t n, double eps,
+                                   uint64_t *mask, int64_t *row_nnz, void *stream) {
+  FLUX_CHECK(scene != nullptr, "flux_ff_mask_square: NULL scene");
+  FLUX_CHECK(n >= 0, "flux_ff_mask_square: negative size");
+  FLUX_CHECK(dtype == FLUX_F32 || dtype == FLUX_F64, "flux_ff_mask_square: dtype must be F32/F64");
+  FLUX_CHECK(n < ((int64_t)1 << 30), "flux_ff_mask_square: n too large");
+  FLUX_CHECK(I || n == scene->nf, "flux_ff_mask_square: without I, n must be the facet count");
+  if (n == 0) return 0;
+  FLUX_CHECK(P && N && mask && row_nnz, "flux_ff_mask_square: NULL array");
+  hipStream_t st = as_stream(stream);
+  const int64_t W = (n + 63) / 64;
+  const int64_t tw = tile_width(n * W / 2);
+  const int64_t tpr = (W + tw - 1) / tw;
+  unsigned long long *counter = (unsigned long long *)row_nnz;
+  hipLaunchKernelGGL(k_mask_clear, dim3(grid_1d(n * W, 1024)), dim3(256), 0, st, mask, n * W,
+                     counter);
+  if (tw < 64) counter = nullptr;
+  const unsigned blocks = trace_groups(n * tpr);
+  if (dtype == FLUX_F64)
+    hipLaunchKernelGGL(k_ff_mask_both<double>, dim3(blocks), dim3(256), 0, st, *scene,
+                       (const double *)P, (const double *)N, I, n, (double)eps, mask, W, tw, tpr,
+                       counter);
+  else
+    hipLaunchKernelGGL(k_ff_mask_both<float>, dim3(blocks), dim3(256), 0, st, *scene,
+                       (const float *)P, (const float *)N, I, n, (float)eps, mask, W, tw, tpr,
+                       counter);
+  FLUX_LAUNCH_CHECK();
+  hipLaunchKernelGGL(k_row_count, dim3(ceil_div_u(n, 4)), dim3(256), 0, st, mask, n, W, row_nnz);
   FLUX_LAUNCH_CHECK();
   return 0;
 }

@@ -549,6 +549,7 @@ extern "C" int flux_scene_create(const void *V, int64_t nv, const int64_t *F,
     for (int c = 0; c < 3; ++c) wmax = fmax(wmax, hb[3 + c] - hb[c]);
     double sc[3];
     for (int c = 0; c < 3; ++c) sc[c] = wmax > 0 ? 1023.0 / wmax : 0.0;
+    s->edge_tol = extent * extent * 0x1p-42;
     // large enough that a clamped axis never shortens a ray's interval
     // inside a padded box, small enough that plane distances stay finite
     s->inv_max = (float)fmin(1e30, 1e37 / fmax(maxabs, extent));

@@ -37,7 +37,7 @@ constexpr int kWideStack = 24;
 // one node step, whatever the number of lanes it serves.
 constexpr int kRefill = 16;
 
-enum : int { kFlagLost = 4 };
+enum : int { kFlagPair = 1, kFlagReverse = 2, kFlagLost = 4 };
 
 struct LaneRay {
   Ray64 r;
@@ -175,6 +175,93 @@ __device__ __forceinline__ void lane_leaf(const flux_scene &S, LaneRay &L, const
     lane_pop(L, stk);
 }
 
+// What a triangle says about a line that is walked in one direction (origin
+// centroid i, end centroid j) and could be walked from j to i instead.
+// Both directions compute the same edge functions but for rounding: the
+// origin and the sheared coordinates differ by at most 16 u L (u = 2^-53, L
+// the scene's extent; |S| <= 1), so each of U, V, W differs by less than
+// 152 u L^2, and edge_tol = 2^-42 L^2 is more than twelve times that.  With
+// t' = 1 - t, t differs by at most edge_tol (|Az| + |Bz| + |Cz| + 4) / |det|.
+//  kMiss    the line passes outside, both ways
+//  kThrough it passes inside at t, known to 2^-12 both ways
+//  kUnsure  rounding may decide
+enum : int { kMiss = 0, kThrough = 1, kUnsure = 2 };
+
+__device__ __forceinline__ int tri_sides(const Ray64 &r, const TriEdges &e, double tol,
+                                         double *t) {
+  const double hi = fmax(fmax(e.U, e.V), e.W), lo = fmin(fmin(e.U, e.V), e.W);
+  if (hi > tol && lo < -tol) return kMiss;
+  if (!(lo > tol || hi < -tol)) return kUnsure;
+  const double det = e.U + e.V + e.W;
+  const double Az = r.Sz * e.A_z, Bz = r.Sz * e.B_z, Cz = r.Sz * e.C_z;
+  *t = (e.U * Az + e.V * Bz + e.W * Cz) / det;
+  return tol * (fabs(Az) + fabs(Bz) + fabs(Cz) + 4.0) <= 0x1p-12 * fabs(det) ? kThrough : kUnsure;
+}
+
+constexpr double kEndBand = 0x1p-10;  // t this close to 0 or 1 decides nothing
+
+// The ray i -> j for both directions at once (kFlagPair), if both facets
+// are hit clearly at the ends; else for i -> j alone, with j -> i to follow
+// (kFlagReverse).
+__device__ __forceinline__ void both_begin(const flux_scene &S, LaneRay &L, int i, int j,
+                                           bool both) {
+  double o[3], d[3];
+  const double *ci = S.cen + (int64_t)i * 3, *cj = S.cen + (int64_t)j * 3;
+  for (int c = 0; c < 3; ++c) {
+    o[c] = ci[c];
+    d[c] = cj[c] - ci[c];
+  }
+  ray_setup(L.r, o, d);
+  const double tj = tri_hit(L.r, S.tri + (int64_t)j * 9);
+  L.flags = 0;
+  if (both) {
+    double ti = 2.0, te = 2.0;
+    const bool ok =
+        tri_sides(L.r, tri_edges(L.r, S.tri + (int64_t)i * 9), S.edge_tol, &ti) == kThrough &&
+        tri_sides(L.r, tri_edges(L.r, S.tri + (int64_t)j * 9), S.edge_tol, &te) == kThrough &&
+        fabs(ti) < 0.5 * kEndBand && fabs(te - 1.0) < 0.5 * kEndBand;
+    L.flags = ok ? kFlagPair : kFlagReverse;
+  }
+  L.skip1 = i;
+  L.skip2 = j;
+  L.cur = kLaneBlocked;
+  if (tj >= 0.0) lane_begin(S, L, o, d, tj, j, i, j);
+}
+
+// The lane's leaf in such a walk.  A blocker that is clear of the ends and
+// of its own edges blocks both directions; any other triangle that is not a
+// clear miss leaves the reverse direction to a walk of its own.
+__device__ __forceinline__ void both_leaf(const flux_scene &S, LaneRay &L, const int *stk) {
+  const int t = ~L.cur;
+  bool block = false;
+  if (t != L.skip1 && t != L.skip2) {
+    const TriEdges e = tri_edges(L.r, S.tri + (int64_t)t * 9);
+    const double U = e.U, V = e.V, W = e.W;
+    const bool mixed = (U < 0.0 || V < 0.0 || W < 0.0) && (U > 0.0 || V > 0.0 || W > 0.0);
+    const double det = U + V + W;
+    const double Az = L.r.Sz * e.A_z, Bz = L.r.Sz * e.B_z, Cz = L.r.Sz * e.C_z;
+    const double th = (U * Az + V * Bz + W * Cz) / det;
+    block = !mixed && det != 0.0 && th >= 0.0 && (th < L.tlim || (th == L.tlim && t < L.klim));
+    if (L.flags & kFlagPair) {
+      const double hi = fmax(fmax(U, V), W), lo = fmin(fmin(U, V), W);
+      const bool miss = hi > S.edge_tol && lo < -S.edge_tol;
+      const bool thru = (lo > S.edge_tol || hi < -S.edge_tol) &&
+                        S.edge_tol * (fabs(Az) + fabs(Bz) + fabs(Cz) + 4.0) <=
+                            0x1p-12 * fabs(det);
+      const bool inside = thru && th > kEndBand && th < 1.0 - kEndBand;
+      const bool beyond = thru && (th < -kEndBand || th > 1.0 + kEndBand);
+      if (inside)
+        L.flags &= ~kFlagReverse;
+      else if (!miss && !beyond)
+        L.flags |= kFlagReverse;
+    }
+  }
+  if (block)
+    L.cur = kLaneBlocked;
+  else
+    lane_pop(L, stk);
+}
+
 // A walk that ran out of stack has skipped children: repeat it on the
 // stackless layout unless it found a blocker anyway.
 __device__ __forceinline__ void lane_recover(const flux_scene &S, LaneRay &L) {
@@ -185,6 +272,7 @@ __device__ __forceinline__ void lane_recover(const flux_scene &S, LaneRay &L) {
       rb.inv[c] = L.inv[c];
     }
     if (any_blocker(S, L.r, rb, L.tlim, L.klim, L.skip1, L.skip2)) L.cur = kLaneBlocked;
+    if (L.flags & kFlagPair) L.flags |= kFlagReverse;
   }
   L.flags &= ~kFlagLost;
 }

@@ -145,6 +145,14 @@ int flux_ff_mask(const flux_scene *scene, const void *P, const void *N,
                  int64_t n, double eps, int mode, uint64_t *mask,
                  int64_t *row_nnz, void *stream);
 
+/* flux_ff_mask in CGAL mode for rows and columns that are one list of n
+ * facets, I (NULL: facets 0 .. nf - 1, n = nf): the same mask, in about half
+ * the rays, since the rays i -> j and j -> i run along one line.
+ * n < 2^30. */
+int flux_ff_mask_square(const flux_scene *scene, const void *P, const void *N,
+                        int dtype, const int64_t *I, int64_t n, double eps,
+                        uint64_t *mask, int64_t *row_nnz, void *stream);
+
 /* The prefilter alone: bit q of row p of `mask` is set iff the pair passes
  * the eps test (form_factors.py:46-52), i.e. iff flux_ff_mask casts a ray
  * for it; row_cnt[p] = popcount.  Used to count rays for Mrays/s. */

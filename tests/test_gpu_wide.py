@@ -79,3 +79,43 @@ def test_stack_overflow_matches_oracle(torch_dev, oracle_mod):
         d = np.array(d) / np.linalg.norm(d)
         assert np.array_equal(sm.is_occluded(I, d), S.occluded(I, d)[:, 0])
     assert np.array_equal(sm.get_visibility(I, I), S.vis_mn(I, I))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("mesh", ["soup", "crater", "terrain", "far", "sheet"])
+def test_square_mask_equals_general_mask(torch_dev, oracle_mod, mesh, dtype):
+    """All pairs of one list from one walk per pair against one walk per
+    direction (the same list as rows and columns, the columns permuted so
+    that the general path takes them) and against the oracle.  `sheet` has
+    facets in common planes and rays through edges and vertices, where
+    rounding decides and the two directions may differ."""
+    from fluxpy_amd.form_factors import get_form_factor_matrix
+    from fluxpy_amd.shape import CgalTrimeshShapeModel
+    if mesh == "soup":
+        V, F = _soup(150, 7)
+    elif mesh == "crater":
+        V, F = meshes.spherical_crater(npts=18, seed=5, depth=0.3)
+    elif mesh == "terrain":
+        V, F = meshes.fractal_terrain(grid=24, levels=5, n_craters=6, seed=8)
+    elif mesh == "far":
+        V, F = meshes.fractal_terrain(grid=16, levels=4, n_craters=4, seed=9)
+        V = V * 3.0 + np.array([4e3, -9e3, 2e3])
+    else:
+        # a regular corrugated sheet: equal facets, symmetric rays
+        x = np.arange(17.0)
+        Z = np.abs((x % 8) - 4.0)[:, None] + 0 * x[None, :]
+        V, F = meshes.grid_mesh(x, x, Z)
+    V = V.astype(dtype)
+    sm = CgalTrimeshShapeModel(V, F)
+    nf = sm.num_faces
+    I = np.arange(nf)
+    full = get_form_factor_matrix(sm)
+    S = oracle_mod.OracleScene(V, F)
+    want = S.form_factor_matrix(sm.P, sm.N, sm.A)
+    assert full.nnz == want.nnz and (full != want).nnz == 0
+    rev = get_form_factor_matrix(sm, I, I[::-1].copy())       # general path
+    assert (full.toarray()[:, ::-1] == rev.toarray()).all()
+    rng = np.random.default_rng(1)
+    sub = rng.integers(0, nf, max(1, nf // 3))                # a list with repeats
+    assert (get_form_factor_matrix(sm, sub, sub).toarray()
+            == full.toarray()[np.ix_(sub, sub)]).all()
