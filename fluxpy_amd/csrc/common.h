@@ -67,13 +67,14 @@ struct flux_scene {
   float4 *nodes;  // kOctants layouts of 2 * nnodes: {lo.xyz, escape bits}, {hi.xyz, tri bits}
   float pad;      // absolute box padding used at build
   // four-wide nodes (wide.h; scene.hip builds them), 4 x uint4 each:
-  //   {box lo x, y, z; exponents x | y << 8 | z << 16 | slots in use << 24}
-  //   {child codes}
-  //   {lo x, lo y, lo z, hi x}  quantised child planes, byte c = child c
-  //   {hi y, hi z, visit orders of octants 0-3, of octants 4-7 (byte o & 3)}
+  //   {box lo x, y, z; exponents x | y << 8 | z << 16, signed bytes}
+  //   {child codes}: slots 0, 1 below the left child, 2, 3 below the right
+  //   {lo x, lo y, lo z, hi x}  quantised child planes, byte c = slot c
+  //   {hi y, hi z, visit order (3 bits per octant), 0}
   uint4 *wide;
-  int32_t *order;  // facets in Morton order
-  int32_t root;    // child code of the root (wide.h)
-  float inv_max;   // bound on a ray's reciprocal direction in the slab tests
-  double edge_tol; // twelve times the rounding of an edge function (wide.h)
+  int32_t *order;   // facets in Morton order
+  int32_t root;     // child code of the root (wide.h)
+  float inv_max;    // bound on a ray's reciprocal direction in the slab tests
+  double box[6];    // bounds of the vertices: lo x, y, z, hi x, y, z
+  double edge_tol;  // twelve times the rounding of an edge function (wide.h)
 };

@@ -241,7 +241,7 @@ __global__ void __launch_bounds__(256, 5) k_ff_mask_rays(
     const int64_t *__restrict__ I, int64_t m, const int64_t *__restrict__ J, int64_t n, T eps,
     int mode, uint64_t *__restrict__ mask, int64_t W, int64_t tile_words,
     int64_t tiles_per_row, unsigned long long *__restrict__ counter) {
-  __shared__ int stack[4][kWideStack][64];
+  __shared__ int stack[4][kStackRows][64];
   __shared__ int2 queue[4][kPairQueue];
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   PairSource<T> src;
@@ -397,7 +397,7 @@ __global__ void __launch_bounds__(256, 5) k_ff_mask_both(
     flux_scene S, const T *__restrict__ P, const T *__restrict__ N,
     const int64_t *__restrict__ I, int64_t n, T eps, uint64_t *__restrict__ mask, int64_t W,
     int64_t tile_words, int64_t tiles_per_row, unsigned long long *__restrict__ counter) {
-  __shared__ int stack[4][kWideStack][64];
+  __shared__ int stack[4][kStackRows][64];
   __shared__ int2 queue[4][kPairQueue];
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   BothSource<T> src;

@@ -19,15 +19,16 @@
 namespace flux {
 
 struct Ray64 {
-  double o[3];
+  double o[3];  // origin in the order kx, ky, kz
   double Sx, Sy, Sz;
   int kx, ky, kz;
 };
 
+__device__ __forceinline__ double sel3(const double *v, int k) {
+  return k == 0 ? v[0] : (k == 1 ? v[1] : v[2]);
+}
+
 __device__ __forceinline__ void ray_setup(Ray64 &r, const double o[3], const double d[3]) {
-  r.o[0] = o[0];
-  r.o[1] = o[1];
-  r.o[2] = o[2];
   double ax = fabs(d[0]), ay = fabs(d[1]), az = fabs(d[2]);
   int kz = 0;
   double mx = ax;
@@ -48,13 +49,12 @@ __device__ __forceinline__ void ray_setup(Ray64 &r, const double o[3], const dou
   r.kx = kx;
   r.ky = ky;
   r.kz = kz;
+  r.o[0] = sel3(o, kx);
+  r.o[1] = sel3(o, ky);
+  r.o[2] = sel3(o, kz);
   r.Sx = d[kx] / d[kz];
   r.Sy = d[ky] / d[kz];
   r.Sz = 1.0 / d[kz];
-}
-
-__device__ __forceinline__ double sel3(const double *v, int k) {
-  return k == 0 ? v[0] : (k == 1 ? v[1] : v[2]);
 }
 
 // Edge functions U, V, W of the triangle v (9 doubles A, B, C) in the ray's
@@ -66,15 +66,15 @@ struct TriEdges {
 
 __device__ __forceinline__ TriEdges tri_edges(const Ray64 &r, const double *__restrict__ v) {
   TriEdges e;
-  const double A_x = sel3(v, r.kx) - sel3(r.o, r.kx);
-  const double A_y = sel3(v, r.ky) - sel3(r.o, r.ky);
-  e.A_z = sel3(v, r.kz) - sel3(r.o, r.kz);
-  const double B_x = sel3(v + 3, r.kx) - sel3(r.o, r.kx);
-  const double B_y = sel3(v + 3, r.ky) - sel3(r.o, r.ky);
-  e.B_z = sel3(v + 3, r.kz) - sel3(r.o, r.kz);
-  const double C_x = sel3(v + 6, r.kx) - sel3(r.o, r.kx);
-  const double C_y = sel3(v + 6, r.ky) - sel3(r.o, r.ky);
-  e.C_z = sel3(v + 6, r.kz) - sel3(r.o, r.kz);
+  const double A_x = sel3(v, r.kx) - r.o[0];
+  const double A_y = sel3(v, r.ky) - r.o[1];
+  e.A_z = sel3(v, r.kz) - r.o[2];
+  const double B_x = sel3(v + 3, r.kx) - r.o[0];
+  const double B_y = sel3(v + 3, r.ky) - r.o[1];
+  e.B_z = sel3(v + 3, r.kz) - r.o[2];
+  const double C_x = sel3(v + 6, r.kx) - r.o[0];
+  const double C_y = sel3(v + 6, r.ky) - r.o[1];
+  e.C_z = sel3(v + 6, r.kz) - r.o[2];
   const double Ax = A_x - r.Sx * e.A_z;
   const double Ay = A_y - r.Sy * e.A_z;
   const double Bx = B_x - r.Sx * e.B_z;

@@ -6,7 +6,7 @@ namespace flux {
 template <typename Query>
 __global__ void __launch_bounds__(256, 5) k_query(flux_scene S, Query q, int64_t total,
                                                   int64_t block) {
-  __shared__ int stack[4][kWideStack][64];
+  __shared__ int stack[4][kStackRows][64];
   IndexSource<Query> src;
   src.init(q, total, block);
   trace_wave(S, src, &stack[threadIdx.x >> 6][0][threadIdx.x & 63]);
@@ -64,7 +64,10 @@ __device__ __forceinline__ void sun_begin(const flux_scene &S, LaneRay &L, int64
     embree_sun_ray(P + f * 3, N + f * 3, dir, o, d);
   }
   ray_setup(L.r, o, d);
-  lane_begin(S, L, o, d, INFINITY, 0x7fffffff, skip, -1);
+  // the walk ends where the ray leaves the scene along its main axis
+  const double lo = sel3(S.box, L.r.kz), hi = sel3(S.box + 3, L.r.kz);
+  const double tmax = fmax(((L.r.Sz < 0.0 ? lo : hi) - L.r.o[2]) * L.r.Sz, 0.0);
+  lane_begin(S, L, o, d, tmax, INFINITY, 0x7fffffff, skip, -1);
 }
 
 // Occlusion of facet I[p] towards D[q] (or D[p]): all facets of one

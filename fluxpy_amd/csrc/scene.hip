@@ -334,27 +334,28 @@ __global__ void k_wide_emit(const uint64_t *__restrict__ keys, const float *__re
                             uint4 *__restrict__ wide) {
   const int u = blockIdx.x * blockDim.x + threadIdx.x;
   if (u >= n - 1 || !wflag[u]) return;
-  int ch[4], nc = 0;
-  for (int side = 0; side < 2; ++side) {
-    const int c = side ? rch[u] : lch[u];
-    if (c >= n - 1) {
-      ch[nc++] = c;
-    } else {
-      ch[nc++] = lch[c];
-      ch[nc++] = rch[c];
-    }
+  const int l = lch[u], r = rch[u];
+  int ch[4] = {l, -1, r, -1};
+  if (l < n - 1) {
+    ch[0] = lch[l];
+    ch[1] = rch[l];
+  }
+  if (r < n - 1) {
+    ch[2] = lch[r];
+    ch[3] = rch[r];
   }
   const float *nb = boxes + (int64_t)u * 6;
   uint32_t q[6] = {0, 0, 0, 0, 0, 0};  // lo x, y, z, hi x, y, z
-  uint32_t ex = ((1u << nc) - 1u) << 24;
+  uint32_t ex = 0;
   for (int c = 0; c < 3; ++c) {
     // 2^e > extent / 255: every plane is within 0 .. 255 steps of the low
     // corner; the differences and the scaling are exact in FP64, so the
     // rounded planes enclose the child's box
     const double ext = (double)nb[3 + c] - (double)nb[c];
     const int e = max(ilogb(ext / 255.0) + 1, -126);
-    ex |= (uint32_t)(e + 127) << (8 * c);
-    for (int k = 0; k < nc; ++k) {
+    ex |= (uint32_t)(e & 0xff) << (8 * c);
+    for (int k = 0; k < 4; ++k) {
+      if (ch[k] < 0) continue;
       const float *b = boxes + (int64_t)ch[k] * 6;
       const double lo = floor(ldexp((double)b[c] - (double)nb[c], -e));
       const double hi = ceil(ldexp((double)b[3 + c] - (double)nb[c], -e));
@@ -362,38 +363,24 @@ __global__ void k_wide_emit(const uint64_t *__restrict__ keys, const float *__re
       q[3 + c] |= (uint32_t)fmin(fmax(hi, 0.0), 255.0) << (8 * k);
     }
   }
-  // per octant, the children by the coordinate of their box centre along
-  // the octant's diagonal, the nearest in the low bits
-  uint32_t ord[2] = {0, 0};
+  // per octant: 1 the right pair first, 2 slot 1 before 0, 4 slot 3 before 2
+  uint32_t ord = 0;
   for (int oct = 0; oct < kOctants; ++oct) {
-    float key[4];
-    for (int k = 0; k < nc; ++k) {
-      const float *b = boxes + (int64_t)ch[k] * 6;
-      key[k] = 0.0f;
-      for (int c = 0; c < 3; ++c) {
-        const float sg = ((oct >> c) & 1) ? -1.0f : 1.0f;
-        key[k] += sg * (b[c] + b[3 + c]);
-      }
-    }
-    uint32_t byte = 0;
-    for (int k = 0; k < 4; ++k) {
-      int pos = k;
-      if (k < nc) {
-        pos = 0;
-        for (int j = 0; j < nc; ++j) pos += key[j] < key[k] || (key[j] == key[k] && j < k);
-      }
-      byte |= (uint32_t)k << (2 * pos);
-    }
-    ord[oct >> 2] |= byte << (8 * (oct & 3));
+    uint32_t o3 = child_first(boxes, l, r, oct) ? 0u : 1u;
+    if (ch[1] >= 0 && !child_first(boxes, ch[0], ch[1], oct)) o3 |= 2u;
+    if (ch[3] >= 0 && !child_first(boxes, ch[2], ch[3], oct)) o3 |= 4u;
+    ord |= o3 << (3 * oct);
   }
-  int code[4] = {-1, -1, -1, -1};
-  for (int k = 0; k < nc; ++k)
-    code[k] = ch[k] >= n - 1 ? ~(int)(keys[ch[k] - (n - 1)] & 0xffffffffull) : widx[ch[k]];
+  int code[4];
+  for (int k = 0; k < 4; ++k)
+    code[k] = ch[k] < 0 ? INT32_MIN
+                        : (ch[k] >= n - 1 ? ~(int)(keys[ch[k] - (n - 1)] & 0xffffffffull)
+                                          : widx[ch[k]]);
   uint4 *w = wide + (int64_t)widx[u] * 4;
   w[0] = make_uint4(__float_as_uint(nb[0]), __float_as_uint(nb[1]), __float_as_uint(nb[2]), ex);
   w[1] = make_uint4((uint32_t)code[0], (uint32_t)code[1], (uint32_t)code[2], (uint32_t)code[3]);
   w[2] = make_uint4(q[0], q[1], q[2], q[3]);
-  w[3] = make_uint4(q[4], q[5], ord[0], ord[1]);
+  w[3] = make_uint4(q[4], q[5], ord, 0u);
 }
 
 __global__ void k_morton_order(const uint64_t *__restrict__ keys, int n,
@@ -552,6 +539,7 @@ extern "C" int flux_scene_create(const void *V, int64_t nv, const int64_t *F,
     s->edge_tol = extent * extent * 0x1p-42;
     // large enough that a clamped axis never shortens a ray's interval
     // inside a padded box, small enough that plane distances stay finite
+    for (int c = 0; c < 6; ++c) s->box[c] = hb[6 + c];
     s->inv_max = (float)fmin(1e30, 1e37 / fmax(maxabs, extent));
     uint64_t *keys = (uint64_t *)tb_keys.p;
     hipLaunchKernelGGL(k_morton, dim3(ceil_div_u(P, TB)), dim3(TB), 0, st, s->cen, nf, P,

@@ -29,10 +29,11 @@ constexpr int kLaneVisible = INT32_MIN + 1;  // walk ended without a blocker
 constexpr int kLaneBlocked = INT32_MIN + 2;  // a blocker was found
 constexpr int kLaneDone = INT32_MIN + 2;     // states <= kLaneDone have no step to run
 
-// Deferred children per lane (LDS, 256 B per entry and wave).  Terrains of
-// 41k facets reach 14, a walk that would need more marks itself and is
-// repeated on the stackless layout.
+// Deferred children per lane (LDS, 256 B per entry and wave) and the room
+// for a node's writes past them.  Terrains of 41k facets reach 14, a walk
+// that would need more marks itself and is repeated on the stackless layout.
 constexpr int kWideStack = 24;
+constexpr int kStackRows = kWideStack + 3;
 // Out-of-work lanes that trigger a refill: a refill's ray set-up costs about
 // one node step, whatever the number of lanes it serves.
 constexpr int kRefill = 16;
@@ -41,21 +42,37 @@ enum : int { kFlagPair = 1, kFlagReverse = 2, kFlagLost = 4 };
 
 struct LaneRay {
   Ray64 r;
-  float inv[3];
-  float tmax;
+  // slab tests run in t / tmax, so that the walked part of the ray is 0 .. 1:
+  // plane p is at p inv - oi
+  float inv[3], oi[3];
+  int oct;       // 3 x the direction octant
   double tlim;   // hits at (t, k) before (tlim, klim) block
   int klim;
   int skip1, skip2;
-  int cur, sp, flags;
+  int cur, flags;
+  int sp;        // deferred children, in LDS words
 };
 
+// Walk the ray up to tlim (finite).  Rounding of a plane's position, in
+// units of 2^-24 of the scene's scale: the FP32 origin 1, the reciprocal
+// direction over tmax 4, inv x origin 1, the two fused steps 2.  The node
+// boxes contain boxes padded by 16 units, so a triangle hit at t in 0 .. tlim
+// has a slab interval of positive length inside 0 .. 1.
 __device__ __forceinline__ void lane_begin(const flux_scene &S, LaneRay &L, const double o[3],
-                                           const double d[3], double tlim, int klim, int skip1,
-                                           int skip2) {
-  RayBox rb;
-  raybox_setup(rb, o, d);
-  for (int c = 0; c < 3; ++c) L.inv[c] = fminf(fmaxf(rb.inv[c], -S.inv_max), S.inv_max);
-  L.tmax = isinf(tlim) ? 3.0e38f : (float)(tlim * (1.0 + 1e-5)) + 1e-30f;
+                                           const double d[3], double tmax, double tlim, int klim,
+                                           int skip1, int skip2) {
+  const float rt = 1.0f / ((float)(tmax * (1.0 + 1e-5)) + 1e-30f);
+  int oct = 0;
+  for (int c = 0; c < 3; ++c) {
+    const float dc = (float)d[c];
+    const bool neg = dc < 0.0f;
+    float iv = fabsf(1.0f / dc * rt);
+    iv = fminf(iv, S.inv_max);
+    L.inv[c] = neg ? -iv : iv;
+    L.oi[c] = (float)o[c] * L.inv[c];
+    oct += neg ? 3 << c : 0;
+  }
+  L.oct = oct;
   L.tlim = tlim;
   L.klim = klim;
   L.skip1 = skip1;
@@ -92,73 +109,70 @@ __device__ __forceinline__ void pair_begin(const flux_scene &S, LaneRay &L, int 
   }
   ray_setup(L.r, o, d);
   const double tj = tri_hit(L.r, S.tri + (int64_t)j * 9);
-  if (tj >= 0.0) lane_begin(S, L, o, d, tj, j, skip, j);
+  if (tj >= 0.0) lane_begin(S, L, o, d, tj, tj, j, skip, j);
 }
 
 __device__ __forceinline__ void lane_pop(LaneRay &L, const int *stk) {
   if (L.sp > 0) {
-    --L.sp;
-    L.cur = stk[L.sp * 64];
+    L.sp -= 64;
+    L.cur = stk[L.sp];
   } else {
     L.cur = kLaneVisible;
   }
 }
 
-// One child word per axis and side: byte c is the quantised plane of child c.
+// t / tmax of a quantised plane (byte c of w), clamped to the walked part.
 __device__ __forceinline__ float plane(uint32_t w, int c, float s, float b) {
-  return fmaf((float)((w >> (8 * c)) & 0xffu), s, b);
+  return __builtin_amdgcn_fmed3f(fmaf((float)((w >> (8 * c)) & 0xffu), s, b), 0.0f, 1.0f);
 }
 
-// The lane's node: test the four children, go on with the first one hit in
-// the node's order for the ray's octant and defer the others (stk: the
-// lane's column of the wave's stack).
+// The lane's node: test the four children, go on with the first one in the
+// node's order for the ray's octant and defer the others that are hit (stk:
+// the lane's column of the wave's stack).  About 110 VALU instructions:
+// every deferral is an unconditional LDS write below a pointer that moves
+// only past hits, so the order needs no loop over slots and no branches.
 __device__ __forceinline__ void lane_node(const flux_scene &S, LaneRay &L, int *stk) {
   const uint4 *nd = S.wide + (int64_t)L.cur * 4;
   const uint4 n0 = nd[0], n1 = nd[1], n2 = nd[2], n3 = nd[3];
-  const float sx = __uint_as_float((n0.w & 0xffu) << 23) * L.inv[0];
-  const float sy = __uint_as_float(((n0.w >> 8) & 0xffu) << 23) * L.inv[1];
-  const float sz = __uint_as_float(((n0.w >> 16) & 0xffu) << 23) * L.inv[2];
-  const float bx = (__uint_as_float(n0.x) - (float)L.r.o[0]) * L.inv[0];
-  const float by = (__uint_as_float(n0.y) - (float)L.r.o[1]) * L.inv[1];
-  const float bz = (__uint_as_float(n0.z) - (float)L.r.o[2]) * L.inv[2];
+  const int ex = (int)n0.w;
+  const float sx = __builtin_amdgcn_ldexpf(L.inv[0], (int)(int8_t)ex);
+  const float sy = __builtin_amdgcn_ldexpf(L.inv[1], (int)(int8_t)(ex >> 8));
+  const float sz = __builtin_amdgcn_ldexpf(L.inv[2], (int)(int8_t)(ex >> 16));
+  const float bx = fmaf(__uint_as_float(n0.x), L.inv[0], -L.oi[0]);
+  const float by = fmaf(__uint_as_float(n0.y), L.inv[1], -L.oi[1]);
+  const float bz = fmaf(__uint_as_float(n0.z), L.inv[2], -L.oi[2]);
   const bool gx = L.inv[0] < 0.0f, gy = L.inv[1] < 0.0f, gz = L.inv[2] < 0.0f;
   const uint32_t ax = gx ? n2.w : n2.x, fx = gx ? n2.x : n2.w;
   const uint32_t ay = gy ? n3.x : n2.y, fy = gy ? n2.y : n3.x;
   const uint32_t az = gz ? n3.y : n2.z, fz = gz ? n2.z : n3.y;
-  uint32_t hit = 0;
+  int c[4] = {(int)n1.x, (int)n1.y, (int)n1.z, (int)n1.w};
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const float tn = fmaxf(fmaxf(plane(ax, c, sx, bx), plane(ay, c, sy, by)),
-                           fmaxf(plane(az, c, sz, bz), 0.0f));
-    const float tf = fminf(fminf(plane(fx, c, sx, bx), plane(fy, c, sy, by)),
-                           fminf(plane(fz, c, sz, bz), L.tmax));
-    hit |= tn <= tf ? 1u << c : 0u;
+  for (int k = 0; k < 4; ++k) {
+    const float tn =
+        fmaxf(fmaxf(plane(ax, k, sx, bx), plane(ay, k, sy, by)), plane(az, k, sz, bz));
+    const float tf =
+        fminf(fminf(plane(fx, k, sx, bx), plane(fy, k, sy, by)), plane(fz, k, sz, bz));
+    c[k] = tn < tf ? c[k] : kLaneIdle;
   }
-  hit &= n0.w >> 24;  // slots in use
-  const uint32_t ow = gz ? n3.w : n3.z;
-  const uint32_t ord = ow >> ((gx ? 8 : 0) + (gy ? 16 : 0));
-  // visit order back to front: what is left in `next` at the end is the
-  // first child hit
-  int next = kLaneIdle;
-#pragma unroll
-  for (int k = 3; k >= 0; --k) {
-    const uint32_t s = (ord >> (2 * k)) & 3u;
-    if ((hit >> s) & 1u) {
-      if (next != kLaneIdle) {
-        if (L.sp < kWideStack) {
-          stk[L.sp * 64] = next;
-          ++L.sp;
-        } else {
-          L.flags |= kFlagLost;
-        }
-      }
-      next = (int)(s < 2 ? (s == 0 ? n1.x : n1.y) : (s == 2 ? n1.z : n1.w));
-    }
+  const uint32_t ord = n3.z >> L.oct;
+  const bool w0 = ord & 2u, w1 = ord & 4u, wp = ord & 1u;
+  const int a0 = w0 ? c[1] : c[0], a1 = w0 ? c[0] : c[1];
+  const int b0 = w1 ? c[3] : c[2], b1 = w1 ? c[2] : c[3];
+  const int d0 = wp ? b0 : a0, d1 = wp ? b1 : a1, d2 = wp ? a0 : b0, d3 = wp ? a1 : b1;
+  int sp = L.sp;
+  stk[sp] = d3;
+  sp += d3 != kLaneIdle ? 64 : 0;
+  stk[sp] = d2;
+  sp += d2 != kLaneIdle ? 64 : 0;
+  stk[sp] = d1;
+  sp += d1 != kLaneIdle ? 64 : 0;
+  if (sp > kWideStack * 64) {
+    sp = kWideStack * 64;
+    L.flags |= kFlagLost;
   }
-  if (next != kLaneIdle)
-    L.cur = next;
-  else
-    lane_pop(L, stk);
+  L.sp = sp;
+  L.cur = d0;
+  if (d0 == kLaneIdle) lane_pop(L, stk);
 }
 
 // The lane's leaf, for queries that stop at the first blocker.
@@ -225,7 +239,7 @@ __device__ __forceinline__ void both_begin(const flux_scene &S, LaneRay &L, int 
   L.skip1 = i;
   L.skip2 = j;
   L.cur = kLaneBlocked;
-  if (tj >= 0.0) lane_begin(S, L, o, d, tj, j, i, j);
+  if (tj >= 0.0) lane_begin(S, L, o, d, tj, tj, j, i, j);
 }
 
 // The lane's leaf in such a walk.  A blocker that is clear of the ends and
@@ -266,11 +280,16 @@ __device__ __forceinline__ void both_leaf(const flux_scene &S, LaneRay &L, const
 // stackless layout unless it found a blocker anyway.
 __device__ __forceinline__ void lane_recover(const flux_scene &S, LaneRay &L) {
   if (L.cur == kLaneVisible && (L.flags & kFlagLost)) {
-    RayBox rb;
+    // the ray's box test again, from the shears
+    double o[3] = {0.0, 0.0, 0.0}, d[3] = {0.0, 0.0, 0.0};
+    const double dz = 1.0 / L.r.Sz;
     for (int c = 0; c < 3; ++c) {
-      rb.o[c] = (float)L.r.o[c];
-      rb.inv[c] = L.inv[c];
+      if (c == L.r.kx) o[c] = L.r.o[0], d[c] = L.r.Sx * dz;
+      if (c == L.r.ky) o[c] = L.r.o[1], d[c] = L.r.Sy * dz;
+      if (c == L.r.kz) o[c] = L.r.o[2], d[c] = dz;
     }
+    RayBox rb;
+    raybox_setup(rb, o, d);
     if (any_blocker(S, L.r, rb, L.tlim, L.klim, L.skip1, L.skip2)) L.cur = kLaneBlocked;
     if (L.flags & kFlagPair) L.flags |= kFlagReverse;
   }
