@@ -218,153 +218,348 @@ __global__ void __launch_bounds__(256) k_batched_gemm(const int64_t *__restrict_
     }
 }
 
+// LDS written by some lanes of a wave is read by others of the same wave.
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Tournament pairing of step `step` of a cyclic Jacobi sweep over npad
-// (even) indices: index 0 stays, the others rotate; pair k is (p, q), p < q.
+// (even) indices: the last index stays, the others rotate; pair k is (p, q),
+// p < q, and pair 0 has the last index (a padding index if n is odd).
 __device__ __forceinline__ void jacobi_pair(int k, int step, int npad, int &p, int &q) {
-  const int x = (k == 0) ? 0 : ((k - 1 + step) % (npad - 1)) + 1;
-  const int y = ((npad - 2 - k + step) % (npad - 1)) + 1;
+  // both sums are below 2 (npad - 1): k <= npad / 2 - 1, step <= npad - 2
+  int x = k - 1 + step, y = npad - 2 - k + step;
+  x -= x >= npad - 1 ? npad - 1 : 0;
+  y -= y >= npad - 1 ? npad - 1 : 0;
+  x = k == 0 ? npad - 1 : x;
   p = min(x, y);
   q = max(x, y);
 }
 
-// Rotation (c, s) that zeroes a_pq of the 2x2 symmetric block.
+// Rotation (c, s) that zeroes a_pq of the 2x2 symmetric block, |s| <= c:
+// with d = a_qq - a_pp and h = sqrt(d^2 + 4 a_pq^2), c^2 = (1 + |d| / h) / 2
+// and s = sign(d) a_pq / (h c).  Two reciprocal square roots and no division
+// (a division, a square root and another of each in sequence were most of a
+// step); entries whose squares leave the range of FP64 take the tangent.
 __device__ __forceinline__ void jacobi_rotation(double app, double aqq, double apq, double &c,
                                                 double &s) {
   c = 1.0;
   s = 0.0;
   if (apq != 0.0) {
-    const double tau = (aqq - app) / (2.0 * apq);
-    const double t = (tau >= 0.0 ? 1.0 : -1.0) / (fabs(tau) + sqrt(1.0 + tau * tau));
-    c = 1.0 / sqrt(1.0 + t * t);
-    s = t * c;
+    const double d = aqq - app;
+    const double x = d * d + 4.0 * (apq * apq);
+    if (x > 1e-280 && x < 1e280) {
+      const double y = rsqrt(x);
+      const double x2 = 0.5 + 0.5 * (fabs(d) * y);
+      const double rc = rsqrt(x2);
+      c = x2 * rc;
+      s = (d >= 0.0 ? apq : -apq) * y * rc;
+    } else {
+      const double tau = d / (2.0 * apq);
+      const double t = (tau >= 0.0 ? 1.0 : -1.0) / (fabs(tau) + sqrt(1.0 + tau * tau));
+      c = 1.0 / sqrt(1.0 + t * t);
+      s = t * c;
+    }
   }
 }
 
-// Sum of v over the workgroup (blockDim.x == 256); every thread gets it.
-__device__ __forceinline__ double block_sum_256(double v, double *red) {
-  const int tid = threadIdx.x;
-  red[tid] = v;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (tid < w) red[tid] += red[tid + w];
-    __syncthreads();
-  }
-  const double out = red[0];
-  __syncthreads();
-  return out;
+// Batched symmetric eigensolver: cyclic Jacobi in the round-robin
+// (tournament) order.  A sweep over a matrix is a serial chain of n - 1
+// steps, each with n / 2 rotations that need the matrix as the step before
+// left it, so its time is the time of a step in one workgroup, and only what
+// the chain needs is in it:
+//  * k_eig_sweep rotates the matrix alone: the lower triangle, in LDS up to
+//    n = kEigLds, one 2 x 2 block of (pair, pair) at a time, read and written
+//    once (rows and columns of the full matrix in turn read and wrote four
+//    times as much, and the eigenvectors from global memory on top).  It
+//    leaves the sweep's rotations in global memory.
+//  * k_eig_apply applies them to the eigenvectors, whose columns are
+//    independent: one wave per two columns, all over the chip.
+// A matrix that has converged leaves a flag, and the remaining launches of
+// the max_sweeps return at once.  12 matrices of n = 88 from a 1,922-facet
+// crater: 89 us a sweep and 12 us to apply it, 6 to 20 sweeps, 1.6 ms a call
+// on average (11.2 ms before); n = 168: 450 us a sweep, 9 to 14 sweeps
+// (69 ms a call before).
+
+// Largest matrix whose triangle k_eig_sweep holds in LDS (127,448 B).
+constexpr int kEigLds = 178;
+constexpr int kEigThreads = 1024;
+
+__device__ __forceinline__ int tri_at(int i, int j) {
+  const unsigned hi = max(i, j), lo = min(i, j);
+  return (int)((__umul24(hi, hi + 1) >> 1) + lo);
 }
 
-// Largest matrix the LDS-resident eigensolver holds (A with a row stride
-// of n + 1 doubles: 132 KiB at n = 128).
-constexpr int kEigLds = 128;
-
-// Same algorithm as k_batched_syevj for n <= kEigLds, with A in LDS and
-// the rotations accumulated in W = V^T (rows p and q of W are contiguous,
-// so the update is coalesced) at Ww + offA[b] in global memory.  A is read,
-// not overwritten.  Cost per sweep: n^3 LDS operations and 2 n^2 doubles of
-// W traffic per step instead of 4 n^2 doubles of global A and V traffic.
-__global__ void __launch_bounds__(256) k_batched_syevj_lds(
-    const int64_t *__restrict__ ns, const double *__restrict__ A,
-    const int64_t *__restrict__ offA, double *__restrict__ Ww, double *__restrict__ Vout,
-    double *__restrict__ evals, const int64_t *__restrict__ offE, int max_sweeps) {
-  __shared__ double a[kEigLds * (kEigLds + 1)];
-  __shared__ double cs[kEigLds / 2], sn[kEigLds / 2];
-  __shared__ int pp[kEigLds / 2], qq[kEigLds / 2];
-  __shared__ double red[256];
-  const int64_t b = blockIdx.x;
-  const int n = (int)ns[b];
-  const int s = n + 1;
-  const double *ag = A + offA[b];
-  double *w = Ww + offA[b];
-  double *vo = Vout + offA[b];
-  double *ev = evals + offE[b];
-  const int tid = threadIdx.x, nt = blockDim.x;
-  for (int k = tid; k < n * n; k += nt) {
-    const int i = k / n, j = k % n;
-    a[i * s + j] = ag[k];
-    w[k] = (i == j) ? 1.0 : 0.0;
-  }
+// Sum of v over the workgroup of kEigThreads; every thread gets it.
+__device__ __forceinline__ double block_sum_eig(double v, double *red) {
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
-  if (n <= 1) {
-    if (tid == 0 && n == 1) {
-      ev[0] = a[0];
-      vo[0] = 1.0;
+  double t = 0.0;
+  for (int w = 0; w < kEigThreads / 64; ++w) t += red[w];
+  __syncthreads();
+  return t;
+}
+
+struct Rotation {
+  double x, y;  // cosine, sine
+};
+
+// The rotations of a sweep: step by step, the pairs without a padding index
+// (n odd: pair 0 has it); n (n - 1) doubles, and the flag in the last of n^2.
+__device__ __forceinline__ int64_t rot_at(int step, int k, int n) {
+  return (int64_t)step * (n / 2) + (k - (n & 1));
+}
+
+// Rotation of pair k of a step: into cs, into the sweep's list, and applied
+// to the pair's own 2 x 2 block.
+template <typename At>
+__device__ __forceinline__ void eig_rotation(int n, int npad, int step, int k, At at,
+                                             double2 *cs, Rotation *rots) {
+  int p, q;
+  jacobi_pair(k, step, npad, p, q);
+  double c = 1.0, sv = 0.0;
+  if (q < n) {
+    double &pp = at(p, p), &qq = at(q, q), &pq = at(q, p);
+    const double app = pp, aqq = qq, apq = pq;
+    jacobi_rotation(app, aqq, apq, c, sv);
+    if (sv != 0.0) {
+      const double a1 = c * app - sv * apq, b1 = c * apq - sv * aqq;
+      const double a2 = sv * app + c * apq, b2 = sv * apq + c * aqq;
+      pp = c * a1 - sv * b1;
+      qq = sv * a2 + c * b2;
+      pq = 0.0;
     }
-    return;
+    rots[rot_at(step, k, n)] = Rotation{c, sv};
   }
-  const int npad = n + (n & 1);
-  const int half = npad / 2;
-  for (int sweep = 0; sweep < max_sweeps; ++sweep) {
-    double off = 0.0, dia = 0.0;
-    for (int k = tid; k < n * n; k += nt) {
-      const int i = k / n, j = k % n;
-      const double x = a[i * s + j];
-      if (i != j)
-        off += x * x;
-      else
-        dia += x * x;
-    }
-    const double off_all = block_sum_256(off, red);
-    const double dia_all = block_sum_256(dia, red);
-    if (off_all <= 1e-30 * dia_all || off_all == 0.0) break;
-    for (int step = 0; step < npad - 1; ++step) {
-      for (int k = tid; k < half; k += nt) {
-        int p, q;
-        jacobi_pair(k, step, npad, p, q);
-        double c = 1.0, sv = 0.0;
-        if (q < n) jacobi_rotation(a[p * s + p], a[q * s + q], a[p * s + q], c, sv);
-        pp[k] = p;
-        qq[k] = q;
-        cs[k] = c;
-        sn[k] = sv;
+  cs[k] = make_double2(c, sv);
+}
+
+// Rotations k1 (rows) and k2 (columns) on their 2 x 2 block.  PAD: the
+// matrix has room for the padding index (a zero row that stays zero).
+template <bool PAD, typename At>
+__device__ __forceinline__ void eig_block(int n, int npad, int step, int k1, int k2, At at,
+                                          const double2 *cs) {
+  const double2 r1 = cs[k1], r2 = cs[k2];
+  int p, q, r, t;
+  jacobi_pair(k1, step, npad, p, q);
+  jacobi_pair(k2, step, npad, r, t);
+  const bool q_ok = PAD || q < n, t_ok = PAD || t < n;  // at most one is false
+  double &ppr = at(p, r);
+  double &ppt = t_ok ? at(p, t) : ppr;
+  double &pqr = q_ok ? at(q, r) : ppr;
+  double &pqt = q_ok ? (t_ok ? at(q, t) : pqr) : ppt;
+  const double apr = ppr, apt = t_ok ? ppt : 0.0;
+  const double aqr = q_ok ? pqr : 0.0, aqt = q_ok && t_ok ? pqt : 0.0;
+  const double xpr = r2.x * apr - r2.y * apt, xpt = r2.y * apr + r2.x * apt;
+  const double xqr = r2.x * aqr - r2.y * aqt, xqt = r2.y * aqr + r2.x * aqt;
+  ppr = r1.x * xpr - r1.y * xqr;
+  if (t_ok) ppt = r1.x * xpt - r1.y * xqt;
+  if (q_ok) pqr = r1.y * xpr + r1.x * xqr;
+  if (q_ok && t_ok) pqt = r1.y * xpt + r1.x * xqt;
+}
+
+// Blocks that hold the off-diagonal element of a pair of the next step: next
+// pair k joins one index each of pairs k - 1 and k + 1, the outer ones of
+// pairs 0 and 1 and of the last two.
+__device__ __forceinline__ bool eig_ahead(int k1, int k2, int half) {
+  return k2 - k1 == 2 || (k1 == 0 && k2 == 1) || (k1 == half - 2 && k2 == half - 1);
+}
+
+// One sweep over the triangle behind at(i, j).  The first wave rotates the
+// blocks that the next step's rotations need and computes those (divisions
+// and square roots in sequence, the longer half of a step) while the other
+// waves rotate the rest, so a step is one barrier.  The rest is bound by
+// instruction issue (one CU, about 70 VALU instructions a block), so the
+// blocks are dealt one to a thread, full waves, and their index arithmetic
+// is kept short: 1.7 -> 1.0 us a step at n = 88.  cs: two steps' rotations.
+template <bool PAD, typename At>
+__device__ __forceinline__ void eig_steps(int n, At at, double2 (*cs)[512], Rotation *rots) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int npad = n + (n & 1), half = npad / 2, nsteps = npad - 1;
+  // this thread's first item and the stride of kEigThreads - 64 items
+  const int d0 = 1 + (tid - 64) / half, k0 = (tid - 64) % half;
+  const int dd = (kEigThreads - 64) / half, dk = (kEigThreads - 64) % half;
+  if (wave == 0)
+    for (int k = lane; k < half; k += 64) eig_rotation(n, npad, 0, k, at, cs[0], rots);
+  __syncthreads();
+  for (int step = 0; step < nsteps; ++step) {
+    const double2 *now = cs[step & 1];
+    if (wave == 0) {
+      for (int k = lane; k < half; k += 64) {
+        const int k1 = k == 0 ? 0 : (k == half - 1 ? half - 2 : k - 1);
+        const int k2 = k == 0 ? 1 : (k == half - 1 ? half - 1 : k + 1);
+        if (k2 < half && (k == 0 || half > 2)) eig_block<PAD>(n, npad, step, k1, k2, at, now);
       }
-      __syncthreads();
-      // columns of A and rows of W
-      for (int x = tid; x < half * n; x += nt) {
-        const int k = x / n, i = x % n;
-        const int p = pp[k], q = qq[k];
-        if (q >= n || sn[k] == 0.0) continue;
-        const double c = cs[k], sv = sn[k];
-        const double aip = a[i * s + p], aiq = a[i * s + q];
-        a[i * s + p] = c * aip - sv * aiq;
-        a[i * s + q] = sv * aip + c * aiq;
-        const double wpi = w[(int64_t)p * n + i], wqi = w[(int64_t)q * n + i];
-        w[(int64_t)p * n + i] = c * wpi - sv * wqi;
-        w[(int64_t)q * n + i] = sv * wpi + c * wqi;
-      }
-      __syncthreads();
-      // rows of A
-      for (int x = tid; x < half * n; x += nt) {
-        const int k = x / n, j = x % n;
-        const int p = pp[k], q = qq[k];
-        if (q >= n || sn[k] == 0.0) continue;
-        const double c = cs[k], sv = sn[k];
-        const double apj = a[p * s + j], aqj = a[q * s + j];
-        a[p * s + j] = c * apj - sv * aqj;
-        a[q * s + j] = sv * apj + c * aqj;
-      }
-      __syncthreads();
-      for (int k = tid; k < half; k += nt) {
-        const int p = pp[k], q = qq[k];
-        if (q < n && sn[k] != 0.0) {
-          a[p * s + q] = 0.0;
-          a[q * s + p] = 0.0;
+      wave_order();
+      if (step + 1 < nsteps)
+        for (int k = lane; k < half; k += 64)
+          eig_rotation(n, npad, step + 1, k, at, cs[(step + 1) & 1], rots);
+    } else {
+      // item (d, k): the pair of pairs k and k + d (mod half), each unordered
+      // pair once
+      int d = d0, k = k0;
+      while (d <= half / 2) {
+        const int m = k + d < half ? k + d : k + d - half;
+        const int k1 = min(k, m), k2 = max(k, m);
+        if ((2 * d < half || k < m) && !eig_ahead(k1, k2, half))
+          eig_block<PAD>(n, npad, step, k1, k2, at, now);
+        k += dk;
+        d += dd;
+        if (k >= half) {
+          k -= half;
+          ++d;
         }
       }
-      __syncthreads();
+    }
+    __syncthreads();
+  }
+}
+
+__global__ void __launch_bounds__(kEigThreads) k_eig_sweep(
+    const int64_t *__restrict__ ns, double *A, const int64_t *__restrict__ offA, double *rot,
+    int sweep) {
+  __shared__ double tri[kEigLds * (kEigLds + 1) / 2];
+  __shared__ double2 cs[2][512];
+  __shared__ double red[kEigThreads / 64];
+  const int64_t b = blockIdx.x;
+  const int n = (int)ns[b], tid = threadIdx.x;
+  if (n <= 1) return;
+  double *ag = A + offA[b];
+  double *rb = rot + offA[b];
+  double *flag = rb + (int64_t)n * n - 1;
+  if (sweep > 0 && *flag == 0.0) return;
+  const bool lds = n <= kEigLds;
+  double off = 0.0, dia = 0.0;
+  for (int64_t k = tid; k < (int64_t)n * n; k += kEigThreads) {
+    const int i = (int)(k / n), j = (int)(k - (int64_t)i * n);
+    if (j > i) continue;
+    const double x = ag[k];
+    if (lds) tri[tri_at(i, j)] = x;
+    if (i != j)
+      off += 2.0 * (x * x);
+    else
+      dia += x * x;
+  }
+  const double off_all = block_sum_eig(off, red);
+  const double dia_all = block_sum_eig(dia, red);
+  const bool done = off_all <= 1e-30 * dia_all || off_all == 0.0;
+  if (tid == 0) *flag = done ? 0.0 : 1.0;
+  if (done) return;
+  if (lds) {
+    if (n & 1)
+      for (int j = tid; j <= n; j += kEigThreads) tri[tri_at(n, j)] = 0.0;
+    __syncthreads();
+    eig_steps<true>(
+        n, [&](int i, int j) -> double & { return tri[tri_at(i, j)]; }, cs, (Rotation *)rb);
+    for (int64_t k = tid; k < (int64_t)n * n; k += kEigThreads) {
+      const int i = (int)(k / n), j = (int)(k - (int64_t)i * n);
+      if (j <= i) ag[k] = tri[tri_at(i, j)];
+    }
+  } else {
+    eig_steps<false>(
+        n,
+        [&](int i, int j) -> double & {
+          return ag[i >= j ? (int64_t)i * n + j : (int64_t)j * n + i];
+        },
+        cs, (Rotation *)rb);
+  }
+}
+
+// W <- J^T W for the sweep's rotations (W = V^T, n x n row-major; W = I
+// first if init).  A wave keeps two columns in LDS; lane l takes pairs l,
+// l + 64, ..., and the next step's rotations are on their way meanwhile.
+template <int NI>
+__global__ void __launch_bounds__(256) k_eig_apply(const int64_t *__restrict__ ns,
+                                                   const int64_t *__restrict__ offA,
+                                                   const double *__restrict__ rot,
+                                                   double *__restrict__ W, int init, int rotate) {
+  extern __shared__ double2 wcols[];  // 4 waves x lds_rows
+  const int64_t b = blockIdx.x;
+  const int n = (int)ns[b];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int i0 = ((int)blockIdx.y * 4 + wave) * 2;
+  if (i0 >= n) return;
+  const double *rb = rot + offA[b];
+  double *wb = W + offA[b];
+  const bool run = rotate && n > 1 && rb[(int64_t)n * n - 1] != 0.0;
+  if (!init && !run) return;
+  double2 *w = wcols + (int64_t)wave * 64 * 2 * NI;
+  const bool two = i0 + 1 < n;
+  for (int p = lane; p < n; p += 64) {
+    double2 v;
+    if (init)
+      v = make_double2(p == i0 ? 1.0 : 0.0, p == i0 + 1 ? 1.0 : 0.0);
+    else
+      v = make_double2(wb[(int64_t)p * n + i0], two ? wb[(int64_t)p * n + i0 + 1] : 0.0);
+    w[p] = v;
+  }
+  wave_order();
+  if (run) {
+    const Rotation *rots = (const Rotation *)rb;
+    const int npad = n + (n & 1), half = npad / 2, k0 = n & 1;
+    Rotation next[NI];
+#pragma unroll
+    for (int u = 0; u < NI; ++u) {
+      const int k = k0 + lane + 64 * u;
+      next[u] = k < half ? rots[rot_at(0, k, n)] : Rotation{1.0, 0.0};
+    }
+    for (int step = 0; step < npad - 1; ++step) {
+      Rotation r[NI];
+#pragma unroll
+      for (int u = 0; u < NI; ++u) {
+        const int k = k0 + lane + 64 * u;
+        r[u] = next[u];
+        if (k < half && step + 1 < npad - 1) next[u] = rots[rot_at(step + 1, k, n)];
+      }
+#pragma unroll
+      for (int u = 0; u < NI; ++u) {
+        const int k = k0 + lane + 64 * u;
+        if (k >= half || r[u].y == 0.0) continue;
+        int p, q;
+        jacobi_pair(k, step, npad, p, q);
+        const double2 x = w[p], y = w[q];
+        w[p] = make_double2(r[u].x * x.x - r[u].y * y.x, r[u].x * x.y - r[u].y * y.y);
+        w[q] = make_double2(r[u].y * x.x + r[u].x * y.x, r[u].y * x.y + r[u].x * y.y);
+      }
+      wave_order();
     }
   }
-  // sort descending (rank by counting; ties by index); eigenvector i is row
-  // i of W
-  for (int i = tid; i < n; i += nt) {
-    const double di = a[i * s + i];
-    int rank = 0;
-    for (int j = 0; j < n; ++j) {
-      const double dj = a[j * s + j];
-      rank += (dj > di) || (dj == di && j < i);
-    }
-    ev[rank] = di;
-    for (int r = 0; r < n; ++r) vo[(int64_t)r * n + rank] = w[(int64_t)i * n + r];
+  for (int p = lane; p < n; p += 64) {
+    const double2 v = w[p];
+    wb[(int64_t)p * n + i0] = v.x;
+    if (two) wb[(int64_t)p * n + i0 + 1] = v.y;
+  }
+}
+
+// Eigenvalues descending (rank by counting, ties by index) and the
+// eigenvectors, row i of W, as columns of Vout.
+__global__ void __launch_bounds__(256) k_eig_sort(const int64_t *__restrict__ ns,
+                                                  const double *__restrict__ A,
+                                                  const int64_t *__restrict__ offA,
+                                                  const double *__restrict__ W,
+                                                  double *__restrict__ Vout,
+                                                  double *__restrict__ evals,
+                                                  const int64_t *__restrict__ offE) {
+  __shared__ double d[1024];
+  __shared__ int rank[1024];
+  const int64_t b = blockIdx.x;
+  const int n = (int)ns[b], tid = threadIdx.x;
+  const double *a = A + offA[b];
+  for (int i = tid; i < n; i += 256) d[i] = a[(int64_t)i * n + i];
+  __syncthreads();
+  for (int i = tid; i < n; i += 256) {
+    int r = 0;
+    for (int j = 0; j < n; ++j) r += (d[j] > d[i]) || (d[j] == d[i] && j < i);
+    rank[i] = r;
+    if (blockIdx.y == 0) evals[offE[b] + r] = d[i];
+  }
+  __syncthreads();
+  for (int64_t k = (int64_t)blockIdx.y * 256 + tid; k < (int64_t)n * n;
+       k += (int64_t)gridDim.y * 256) {
+    const int i = (int)(k / n), r = (int)(k - (int64_t)i * n);
+    Vout[offA[b] + (int64_t)r * n + rank[i]] = W[offA[b] + k];
   }
 }
 
@@ -378,138 +573,6 @@ __global__ void k_ns_factor(const int64_t *__restrict__ ns, double *__restrict__
        k += (int64_t)gridDim.x * blockDim.x) {
     const double g = G[offG[b] + k];
     G[offG[b] + k] = ((k / n == k % n) ? 1.5 : 0.0) - 0.5 * g;
-  }
-}
-
-// Batched symmetric eigensolver: cyclic Jacobi with the round-robin
-// (tournament) ordering, one workgroup per matrix, matrices in global memory
-// (n x n row-major, overwritten).  Outputs eigenvalues sorted descending and
-// the matching eigenvectors as COLUMNS of Vout (n x n row-major).
-__global__ void __launch_bounds__(256) k_batched_syevj(
-    const int64_t *__restrict__ ns, double *__restrict__ A, const int64_t *__restrict__ offA,
-    double *__restrict__ Vw, double *__restrict__ Vout, double *__restrict__ evals,
-    const int64_t *__restrict__ offE, int max_sweeps) {
-  const int64_t b = blockIdx.x;
-  const int n = (int)ns[b];
-  double *a = A + offA[b];
-  double *v = Vw + offA[b];
-  double *vo = Vout + offA[b];
-  double *ev = evals + offE[b];
-  const int tid = threadIdx.x, nt = blockDim.x;
-  const int npad = n + (n & 1);
-  __shared__ double cs[512], sn[512];
-  __shared__ int pp[512], qq[512];
-  __shared__ double red[256];
-  for (int64_t k = tid; k < (int64_t)n * n; k += nt) v[k] = (k / n == k % n) ? 1.0 : 0.0;
-  __syncthreads();
-  if (n <= 1) {
-    if (tid == 0 && n == 1) {
-      ev[0] = a[0];
-      vo[0] = 1.0;
-    }
-    return;
-  }
-  const int half = npad / 2;
-  for (int sweep = 0; sweep < max_sweeps; ++sweep) {
-    // convergence: off-diagonal mass vs diagonal mass
-    double off = 0.0, dia = 0.0;
-    for (int64_t k = tid; k < (int64_t)n * n; k += nt) {
-      const int64_t i = k / n, j = k % n;
-      const double x = a[k];
-      if (i != j)
-        off += x * x;
-      else
-        dia += x * x;
-    }
-    red[tid] = off;
-    __syncthreads();
-    for (int w = nt / 2; w > 0; w >>= 1) {
-      if (tid < w) red[tid] += red[tid + w];
-      __syncthreads();
-    }
-    const double off_all = red[0];
-    __syncthreads();
-    red[tid] = dia;
-    __syncthreads();
-    for (int w = nt / 2; w > 0; w >>= 1) {
-      if (tid < w) red[tid] += red[tid + w];
-      __syncthreads();
-    }
-    const double dia_all = red[0];
-    __syncthreads();
-    if (off_all <= 1e-30 * dia_all || off_all == 0.0) break;
-    for (int step = 0; step < npad - 1; ++step) {
-      // tournament pairing: position 0 fixed, others rotate
-      for (int k = tid; k < half; k += nt) {
-        int x = (k == 0) ? 0 : ((k - 1 + step) % (npad - 1)) + 1;
-        int y = ((npad - 2 - k + step) % (npad - 1)) + 1;
-        int p = min(x, y), q = max(x, y);
-        double c = 1.0, s = 0.0;
-        if (q < n) {
-          const double apq = a[(int64_t)p * n + q];
-          if (apq != 0.0) {
-            const double app = a[(int64_t)p * n + p], aqq = a[(int64_t)q * n + q];
-            const double tau = (aqq - app) / (2.0 * apq);
-            const double t = (tau >= 0.0 ? 1.0 : -1.0) / (fabs(tau) + sqrt(1.0 + tau * tau));
-            c = 1.0 / sqrt(1.0 + t * t);
-            s = t * c;
-          }
-        }
-        pp[k] = p;
-        qq[k] = q;
-        cs[k] = c;
-        sn[k] = s;
-      }
-      __syncthreads();
-      // columns: A <- A J, V <- V J.  Consecutive threads take consecutive
-      // pairs of one row, so a wave's loads stay within that row (a
-      // thread per row of one column would touch a cache line per lane).
-      for (int64_t w = tid; w < (int64_t)half * n; w += nt) {
-        const int k = (int)(w % half);
-        const int64_t i = w / half;
-        const int p = pp[k], q = qq[k];
-        if (q >= n || sn[k] == 0.0) continue;
-        const double c = cs[k], s = sn[k];
-        const double aip = a[i * n + p], aiq = a[i * n + q];
-        a[i * n + p] = c * aip - s * aiq;
-        a[i * n + q] = s * aip + c * aiq;
-        const double vip = v[i * n + p], viq = v[i * n + q];
-        v[i * n + p] = c * vip - s * viq;
-        v[i * n + q] = s * vip + c * viq;
-      }
-      __syncthreads();
-      // rows: A <- J^T A
-      for (int64_t w = tid; w < (int64_t)half * n; w += nt) {
-        const int k = (int)(w / n);
-        const int64_t j = w % n;
-        const int p = pp[k], q = qq[k];
-        if (q >= n || sn[k] == 0.0) continue;
-        const double c = cs[k], s = sn[k];
-        const double apj = a[(int64_t)p * n + j], aqj = a[(int64_t)q * n + j];
-        a[(int64_t)p * n + j] = c * apj - s * aqj;
-        a[(int64_t)q * n + j] = s * apj + c * aqj;
-      }
-      __syncthreads();
-      for (int k = tid; k < half; k += nt) {
-        const int p = pp[k], q = qq[k];
-        if (q < n && sn[k] != 0.0) {
-          a[(int64_t)p * n + q] = 0.0;
-          a[(int64_t)q * n + p] = 0.0;
-        }
-      }
-      __syncthreads();
-    }
-  }
-  // sort descending (rank by counting; ties by index)
-  for (int i = tid; i < n; i += nt) {
-    const double di = a[(int64_t)i * n + i];
-    int rank = 0;
-    for (int j = 0; j < n; ++j) {
-      const double dj = a[(int64_t)j * n + j];
-      rank += (dj > di) || (dj == di && j < i);
-    }
-    ev[rank] = di;
-    for (int r = 0; r < n; ++r) vo[(int64_t)r * n + rank] = v[(int64_t)r * n + i];
   }
 }
 
@@ -625,13 +688,29 @@ extern "C" int flux_batched_syevj(int64_t nb, const int64_t *ns, int64_t nmax, d
   FLUX_CHECK(nb >= 0 && nmax >= 0, "flux_batched_syevj: bad sizes");
   FLUX_CHECK(nmax <= 1024, "flux_batched_syevj: matrices above 1024 x 1024 are not supported");
   FLUX_CHECK(nb <= 0x7fffffff, "flux_batched_syevj: too many matrices");
-  if (nb == 0) return 0;
-  if (nmax <= kEigLds)
-    hipLaunchKernelGGL(k_batched_syevj_lds, dim3((unsigned)nb), dim3(256), 0,
-                       as_stream(stream), ns, A, offA, Vwork, Vout, evals, offE, max_sweeps);
-  else
-    hipLaunchKernelGGL(k_batched_syevj, dim3((unsigned)nb), dim3(256), 0, as_stream(stream),
-                       ns, A, offA, Vwork, Vout, evals, offE, max_sweeps);
+  if (nb == 0 || nmax == 0) return 0;
+  hipStream_t st = as_stream(stream);
+  // rotations in Vout until the end, eigenvectors in Vwork
+  const dim3 cols((unsigned)nb, (unsigned)((nmax + 7) / 8));
+  const int sweeps = max_sweeps > 0 ? max_sweeps : 0;
+  for (int k = 0; k < (sweeps ? sweeps : 1); ++k) {
+    if (sweeps)
+      hipLaunchKernelGGL(k_eig_sweep, dim3((unsigned)nb), dim3(kEigThreads), 0, st, ns, A, offA,
+                         Vout, k);
+    const int init = k == 0, rotate = sweeps > 0;
+    if (nmax <= 128)
+      hipLaunchKernelGGL(k_eig_apply<1>, cols, dim3(256), 4 * 128 * sizeof(double2), st, ns, offA,
+                         Vout, Vwork, init, rotate);
+    else if (nmax <= 256)
+      hipLaunchKernelGGL(k_eig_apply<2>, cols, dim3(256), 4 * 256 * sizeof(double2), st, ns, offA,
+                         Vout, Vwork, init, rotate);
+    else
+      hipLaunchKernelGGL(k_eig_apply<8>, cols, dim3(256), 4 * 1024 * sizeof(double2), st, ns,
+                         offA, Vout, Vwork, init, rotate);
+    FLUX_LAUNCH_CHECK();
+  }
+  hipLaunchKernelGGL(k_eig_sort, dim3((unsigned)nb, 16), dim3(256), 0, st, ns, A, offA, Vwork,
+                     Vout, evals, offE);
   FLUX_LAUNCH_CHECK();
   return 0;
 }

@@ -262,8 +262,7 @@ int flux_batched_gemm(int64_t nb, const int64_t *desc, int64_t max_tiles,
                       void *stream);
 
 /* Symmetric eigen-decomposition of nb matrices (n_b <= 1024, row-major at
- * A + offA[b], destroyed) by parallel-order cyclic Jacobi, one workgroup
- * per matrix: eigenvalues descending at evals + offE[b], eigenvectors as
+ * A + offA[b], destroyed) by parallel-order cyclic Jacobi: eigenvalues descending at evals + offE[b], eigenvectors as
  * the columns of Vout + offA[b].  Vwork: same size as A. */
 int flux_batched_syevj(int64_t nb, const int64_t *ns, int64_t nmax, double *A,
                        const int64_t *offA, double *Vwork, double *Vout,
