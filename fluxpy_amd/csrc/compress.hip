@@ -225,42 +225,28 @@ __device__ __forceinline__ void wave_order() {
 }
 
 // Tournament pairing of step `step` of a cyclic Jacobi sweep over npad
-// (even) indices: the last index stays, the others rotate; pair k is (p, q),
-// p < q, and pair 0 has the last index (a padding index if n is odd).
+// (even) indices: index 0 stays, the others rotate; pair k is (p, q), p < q.
 __device__ __forceinline__ void jacobi_pair(int k, int step, int npad, int &p, int &q) {
   // both sums are below 2 (npad - 1): k <= npad / 2 - 1, step <= npad - 2
   int x = k - 1 + step, y = npad - 2 - k + step;
   x -= x >= npad - 1 ? npad - 1 : 0;
   y -= y >= npad - 1 ? npad - 1 : 0;
-  x = k == 0 ? npad - 1 : x;
+  x = k == 0 ? 0 : x + 1;
+  y += 1;
   p = min(x, y);
   q = max(x, y);
 }
 
-// Rotation (c, s) that zeroes a_pq of the 2x2 symmetric block, |s| <= c:
-// with d = a_qq - a_pp and h = sqrt(d^2 + 4 a_pq^2), c^2 = (1 + |d| / h) / 2
-// and s = sign(d) a_pq / (h c).  Two reciprocal square roots and no division
-// (a division, a square root and another of each in sequence were most of a
-// step); entries whose squares leave the range of FP64 take the tangent.
+// Rotation (c, s) that zeroes a_pq of the 2x2 symmetric block.
 __device__ __forceinline__ void jacobi_rotation(double app, double aqq, double apq, double &c,
                                                 double &s) {
   c = 1.0;
   s = 0.0;
   if (apq != 0.0) {
-    const double d = aqq - app;
-    const double x = d * d + 4.0 * (apq * apq);
-    if (x > 1e-280 && x < 1e280) {
-      const double y = rsqrt(x);
-      const double x2 = 0.5 + 0.5 * (fabs(d) * y);
-      const double rc = rsqrt(x2);
-      c = x2 * rc;
-      s = (d >= 0.0 ? apq : -apq) * y * rc;
-    } else {
-      const double tau = d / (2.0 * apq);
-      const double t = (tau >= 0.0 ? 1.0 : -1.0) / (fabs(tau) + sqrt(1.0 + tau * tau));
-      c = 1.0 / sqrt(1.0 + t * t);
-      s = t * c;
-    }
+    const double tau = (aqq - app) / (2.0 * apq);
+    const double t = (tau >= 0.0 ? 1.0 : -1.0) / (fabs(tau) + sqrt(1.0 + tau * tau));
+    c = 1.0 / sqrt(1.0 + t * t);
+    s = t * c;
   }
 }
 
@@ -269,27 +255,26 @@ __device__ __forceinline__ void jacobi_rotation(double app, double aqq, double a
 // steps, each with n / 2 rotations that need the matrix as the step before
 // left it, so its time is the time of a step in one workgroup, and only what
 // the chain needs is in it:
-//  * k_eig_sweep rotates the matrix alone: the lower triangle, in LDS up to
-//    n = kEigLds, one 2 x 2 block of (pair, pair) at a time, read and written
-//    once (rows and columns of the full matrix in turn read and wrote four
-//    times as much, and the eigenvectors from global memory on top).  It
-//    leaves the sweep's rotations in global memory.
+//  * k_eig_sweep rotates the matrix alone, in LDS up to n = kEigLds, one 2 x 2
+//    block of (pair, pair) at a time, read and written once (columns, then
+//    rows, with a barrier between, read and wrote twice as much, and the
+//    eigenvectors from global memory on top).  Both triangles are kept: an
+//    element and its mirror image round differently, and the rotations read
+//    the upper one.  It leaves the sweep's rotations in global memory.
 //  * k_eig_apply applies them to the eigenvectors, whose columns are
 //    independent: one wave per two columns, all over the chip.
 // A matrix that has converged leaves a flag, and the remaining launches of
-// the max_sweeps return at once.  12 matrices of n = 88 from a 1,922-facet
-// crater: 89 us a sweep and 12 us to apply it, 6 to 20 sweeps, 1.6 ms a call
-// on average (11.2 ms before); n = 168: 450 us a sweep, 9 to 14 sweeps
-// (69 ms a call before).
+// the max_sweeps return at once.  The results are those of the plain order
+// (every pair's columns, then its rows), bit for bit.
+//
+// 12 matrices of n = 88 from a 1,922-facet crater, a call of 6 to 20 sweeps:
+// 11.2 ms with one workgroup doing it all in that order, 2.9 ms now (n = 88 to
+// 128 in general a quarter to a third of the time; above, where the matrix
+// is in L2, three quarters).
 
-// Largest matrix whose triangle k_eig_sweep holds in LDS (127,448 B).
-constexpr int kEigLds = 178;
+// Largest matrix k_eig_sweep holds in LDS (132,096 B).
+constexpr int kEigLds = 128;
 constexpr int kEigThreads = 1024;
-
-__device__ __forceinline__ int tri_at(int i, int j) {
-  const unsigned hi = max(i, j), lo = min(i, j);
-  return (int)((__umul24(hi, hi + 1) >> 1) + lo);
-}
 
 // Sum of v over the workgroup of kEigThreads; every thread gets it.
 __device__ __forceinline__ double block_sum_eig(double v, double *red) {
@@ -306,10 +291,25 @@ struct Rotation {
   double x, y;  // cosine, sine
 };
 
-// The rotations of a sweep: step by step, the pairs without a padding index
-// (n odd: pair 0 has it); n (n - 1) doubles, and the flag in the last of n^2.
+// The sweep's rotations of matrix b: (n - 1) n doubles for even n, n (n - 1)
+// for odd n, where the pair with the padding index is left out, and the flag
+// in the last of the n^2.  slot(k) of a step: its place without that pair.
 __device__ __forceinline__ int64_t rot_at(int step, int k, int n) {
-  return (int64_t)step * (n / 2) + (k - (n & 1));
+  if (!(n & 1)) return (int64_t)step * (n / 2) + k;
+  // the padding index n is x of pair k = n - step, or y of pair k = step
+  // (whichever is below (n + 1) / 2)
+  const int pad = step < (n + 1) / 2 ? step : n - step;
+  return (int64_t)step * (n / 2) + k - (k > pad ? 1 : 0);
+}
+
+// The two results of a rotation (c, s) of x, y, each one product and one
+// fused step in a fixed order: an element is rounded the same way wherever
+// it is rotated.
+__device__ __forceinline__ double rot_x(double c, double s, double x, double y) {
+  return fma(c, x, -(s * y));
+}
+__device__ __forceinline__ double rot_y(double c, double s, double x, double y) {
+  return fma(s, x, c * y);
 }
 
 // Rotation of pair k of a step: into cs, into the sweep's list, and applied
@@ -321,15 +321,16 @@ __device__ __forceinline__ void eig_rotation(int n, int npad, int step, int k, A
   jacobi_pair(k, step, npad, p, q);
   double c = 1.0, sv = 0.0;
   if (q < n) {
-    double &pp = at(p, p), &qq = at(q, q), &pq = at(q, p);
-    const double app = pp, aqq = qq, apq = pq;
+    double &rpp = at(p, p), &rqq = at(q, q), &rpq = at(p, q), &rqp = at(q, p);
+    const double app = rpp, aqq = rqq, apq = rpq, aqp = rqp;
     jacobi_rotation(app, aqq, apq, c, sv);
     if (sv != 0.0) {
-      const double a1 = c * app - sv * apq, b1 = c * apq - sv * aqq;
-      const double a2 = sv * app + c * apq, b2 = sv * apq + c * aqq;
-      pp = c * a1 - sv * b1;
-      qq = sv * a2 + c * b2;
-      pq = 0.0;
+      const double bpp = rot_x(c, sv, app, apq), bpq = rot_y(c, sv, app, apq);
+      const double bqp = rot_x(c, sv, aqp, aqq), bqq = rot_y(c, sv, aqp, aqq);
+      rpp = rot_x(c, sv, bpp, bqp);
+      rqq = rot_y(c, sv, bpq, bqq);
+      rpq = 0.0;
+      rqp = 0.0;
     }
     rots[rot_at(step, k, n)] = Rotation{c, sv};
   }
@@ -337,7 +338,8 @@ __device__ __forceinline__ void eig_rotation(int n, int npad, int step, int k, A
 }
 
 // Rotations k1 (rows) and k2 (columns) on their 2 x 2 block.  PAD: the
-// matrix has room for the padding index (a zero row that stays zero).
+// matrix has room for the padding index (a zero row and column that stay
+// zero).
 template <bool PAD, typename At>
 __device__ __forceinline__ void eig_block(int n, int npad, int step, int k1, int k2, At at,
                                           const double2 *cs) {
@@ -352,28 +354,27 @@ __device__ __forceinline__ void eig_block(int n, int npad, int step, int k1, int
   double &pqt = q_ok ? (t_ok ? at(q, t) : pqr) : ppt;
   const double apr = ppr, apt = t_ok ? ppt : 0.0;
   const double aqr = q_ok ? pqr : 0.0, aqt = q_ok && t_ok ? pqt : 0.0;
-  const double xpr = r2.x * apr - r2.y * apt, xpt = r2.y * apr + r2.x * apt;
-  const double xqr = r2.x * aqr - r2.y * aqt, xqt = r2.y * aqr + r2.x * aqt;
-  ppr = r1.x * xpr - r1.y * xqr;
-  if (t_ok) ppt = r1.x * xpt - r1.y * xqt;
-  if (q_ok) pqr = r1.y * xpr + r1.x * xqr;
-  if (q_ok && t_ok) pqt = r1.y * xpt + r1.x * xqt;
+  const double xpr = rot_x(r2.x, r2.y, apr, apt), xpt = rot_y(r2.x, r2.y, apr, apt);
+  const double xqr = rot_x(r2.x, r2.y, aqr, aqt), xqt = rot_y(r2.x, r2.y, aqr, aqt);
+  ppr = rot_x(r1.x, r1.y, xpr, xqr);
+  if (t_ok) ppt = rot_x(r1.x, r1.y, xpt, xqt);
+  if (q_ok) pqr = rot_y(r1.x, r1.y, xpr, xqr);
+  if (q_ok && t_ok) pqt = rot_y(r1.x, r1.y, xpt, xqt);
 }
 
-// Blocks that hold the off-diagonal element of a pair of the next step: next
+// Blocks that hold the off-diagonal elements of a pair of the next step: next
 // pair k joins one index each of pairs k - 1 and k + 1, the outer ones of
 // pairs 0 and 1 and of the last two.
 __device__ __forceinline__ bool eig_ahead(int k1, int k2, int half) {
   return k2 - k1 == 2 || (k1 == 0 && k2 == 1) || (k1 == half - 2 && k2 == half - 1);
 }
 
-// One sweep over the triangle behind at(i, j).  The first wave rotates the
+// One sweep over the matrix behind at(i, j).  The first wave rotates the
 // blocks that the next step's rotations need and computes those (divisions
-// and square roots in sequence, the longer half of a step) while the other
-// waves rotate the rest, so a step is one barrier.  The rest is bound by
-// instruction issue (one CU, about 70 VALU instructions a block), so the
-// blocks are dealt one to a thread, full waves, and their index arithmetic
-// is kept short: 1.7 -> 1.0 us a step at n = 88.  cs: two steps' rotations.
+// and square roots in sequence) while the other waves rotate the rest, so a
+// step is one barrier.  The rest is bound by instruction issue (one CU), so
+// the blocks are dealt one to a thread, full waves, and their index
+// arithmetic is kept short.  cs: two steps' rotations.
 template <bool PAD, typename At>
 __device__ __forceinline__ void eig_steps(int n, At at, double2 (*cs)[512], Rotation *rots) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -390,21 +391,22 @@ __device__ __forceinline__ void eig_steps(int n, At at, double2 (*cs)[512], Rota
       for (int k = lane; k < half; k += 64) {
         const int k1 = k == 0 ? 0 : (k == half - 1 ? half - 2 : k - 1);
         const int k2 = k == 0 ? 1 : (k == half - 1 ? half - 1 : k + 1);
-        if (k2 < half && (k == 0 || half > 2)) eig_block<PAD>(n, npad, step, k1, k2, at, now);
+        if (k2 < half && (k == 0 || half > 2)) {
+          eig_block<PAD>(n, npad, step, k1, k2, at, now);
+          eig_block<PAD>(n, npad, step, k2, k1, at, now);
+        }
       }
       wave_order();
       if (step + 1 < nsteps)
         for (int k = lane; k < half; k += 64)
           eig_rotation(n, npad, step + 1, k, at, cs[(step + 1) & 1], rots);
     } else {
-      // item (d, k): the pair of pairs k and k + d (mod half), each unordered
-      // pair once
+      // item (d, k): the block of pairs k and k + d (mod half)
       int d = d0, k = k0;
-      while (d <= half / 2) {
+      while (d < half) {
         const int m = k + d < half ? k + d : k + d - half;
-        const int k1 = min(k, m), k2 = max(k, m);
-        if ((2 * d < half || k < m) && !eig_ahead(k1, k2, half))
-          eig_block<PAD>(n, npad, step, k1, k2, at, now);
+        if (!eig_ahead(min(k, m), max(k, m), half))
+          eig_block<PAD>(n, npad, step, k, m, at, now);
         k += dk;
         d += dd;
         if (k >= half) {
@@ -420,7 +422,7 @@ __device__ __forceinline__ void eig_steps(int n, At at, double2 (*cs)[512], Rota
 __global__ void __launch_bounds__(kEigThreads) k_eig_sweep(
     const int64_t *__restrict__ ns, double *A, const int64_t *__restrict__ offA, double *rot,
     int sweep) {
-  __shared__ double tri[kEigLds * (kEigLds + 1) / 2];
+  __shared__ double a[kEigLds * (kEigLds + 1)];
   __shared__ double2 cs[2][512];
   __shared__ double red[kEigThreads / 64];
   const int64_t b = blockIdx.x;
@@ -431,14 +433,14 @@ __global__ void __launch_bounds__(kEigThreads) k_eig_sweep(
   double *flag = rb + (int64_t)n * n - 1;
   if (sweep > 0 && *flag == 0.0) return;
   const bool lds = n <= kEigLds;
+  const int npad = n + (n & 1), s = npad + 1;  // odd stride
   double off = 0.0, dia = 0.0;
   for (int64_t k = tid; k < (int64_t)n * n; k += kEigThreads) {
     const int i = (int)(k / n), j = (int)(k - (int64_t)i * n);
-    if (j > i) continue;
     const double x = ag[k];
-    if (lds) tri[tri_at(i, j)] = x;
+    if (lds) a[i * s + j] = x;
     if (i != j)
-      off += 2.0 * (x * x);
+      off += x * x;
     else
       dia += x * x;
   }
@@ -449,21 +451,17 @@ __global__ void __launch_bounds__(kEigThreads) k_eig_sweep(
   if (done) return;
   if (lds) {
     if (n & 1)
-      for (int j = tid; j <= n; j += kEigThreads) tri[tri_at(n, j)] = 0.0;
+      for (int j = tid; j <= n; j += kEigThreads) a[n * s + j] = a[j * s + n] = 0.0;
     __syncthreads();
     eig_steps<true>(
-        n, [&](int i, int j) -> double & { return tri[tri_at(i, j)]; }, cs, (Rotation *)rb);
+        n, [&](int i, int j) -> double & { return a[__mul24(i, s) + j]; }, cs, (Rotation *)rb);
     for (int64_t k = tid; k < (int64_t)n * n; k += kEigThreads) {
       const int i = (int)(k / n), j = (int)(k - (int64_t)i * n);
-      if (j <= i) ag[k] = tri[tri_at(i, j)];
+      ag[k] = a[i * s + j];
     }
   } else {
     eig_steps<false>(
-        n,
-        [&](int i, int j) -> double & {
-          return ag[i >= j ? (int64_t)i * n + j : (int64_t)j * n + i];
-        },
-        cs, (Rotation *)rb);
+        n, [&](int i, int j) -> double & { return ag[(int64_t)i * n + j]; }, cs, (Rotation *)rb);
   }
 }
 
@@ -498,30 +496,31 @@ __global__ void __launch_bounds__(256) k_eig_apply(const int64_t *__restrict__ n
   wave_order();
   if (run) {
     const Rotation *rots = (const Rotation *)rb;
-    const int npad = n + (n & 1), half = npad / 2, k0 = n & 1;
+    const int npad = n + (n & 1), half = npad / 2;
     Rotation next[NI];
 #pragma unroll
     for (int u = 0; u < NI; ++u) {
-      const int k = k0 + lane + 64 * u;
+      const int k = lane + 64 * u;
       next[u] = k < half ? rots[rot_at(0, k, n)] : Rotation{1.0, 0.0};
     }
     for (int step = 0; step < npad - 1; ++step) {
       Rotation r[NI];
 #pragma unroll
       for (int u = 0; u < NI; ++u) {
-        const int k = k0 + lane + 64 * u;
+        const int k = lane + 64 * u;
         r[u] = next[u];
         if (k < half && step + 1 < npad - 1) next[u] = rots[rot_at(step + 1, k, n)];
       }
 #pragma unroll
       for (int u = 0; u < NI; ++u) {
-        const int k = k0 + lane + 64 * u;
+        const int k = lane + 64 * u;
         if (k >= half || r[u].y == 0.0) continue;
         int p, q;
         jacobi_pair(k, step, npad, p, q);
+        if (q >= n) continue;  // no rotation stored for the padding index
         const double2 x = w[p], y = w[q];
-        w[p] = make_double2(r[u].x * x.x - r[u].y * y.x, r[u].x * x.y - r[u].y * y.y);
-        w[q] = make_double2(r[u].y * x.x + r[u].x * y.x, r[u].y * x.y + r[u].x * y.y);
+        w[p] = make_double2(rot_x(r[u].x, r[u].y, x.x, y.x), rot_x(r[u].x, r[u].y, x.y, y.y));
+        w[q] = make_double2(rot_y(r[u].x, r[u].y, x.x, y.x), rot_y(r[u].x, r[u].y, x.y, y.y));
       }
       wave_order();
     }

@@ -1,6 +1,6 @@
 """The batched symmetric eigensolver against LAPACK: odd and even sizes, the
-smallest ones, both sides of the size whose triangle fits in LDS (178) and of
-the widths at which a wave holds more pairs (128, 256), graded and rank
+smallest ones, both sides of the size that fits in LDS and of the widths at
+which a wave holds more pairs (128, 256), graded and rank
 deficient spectra, a diagonal matrix, and sizes mixed in one batch at odd
 offsets."""
 import numpy as np
