@@ -1,12 +1,12 @@
 // CSR products and the fused Jacobi radiosity step (solve.py:25-45).
 //
-// One wave per CSR row.  With nrhs right-hand sides the 64 lanes split into
-// G = 64/R groups of R = min(64, pow2ceil(nrhs)) lanes: lane (g, c) sums the
-// nonzeros k = g, g+G, ... of the row for column c, then the groups are
-// reduced with cross-lane shuffles.  The summation order is fixed, so every
-// product is deterministic.
+// One wave per CSR row; the lanes' partial sums are reduced with cross-lane
+// shuffles.  The summation order is fixed, so every product is
+// deterministic.
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
+
+#include <type_traits>
 
 #include "common.h"
 
@@ -48,85 +48,284 @@ __device__ inline void atomic_max_nonneg(double *addr, double v) {
   atomicMax((unsigned long long *)addr, (unsigned long long)__double_as_longlong(v));
 }
 
+template <typename T, int V>
+struct Vec {
+  T v[V];
+};
+
+// V consecutive elements from any element-aligned address (one load: global
+// loads of 16 bytes need 4-byte alignment).
+template <int V, typename T>
+__device__ __forceinline__ Vec<T, V> load_vec(const T *p) {
+  Vec<T, V> r;
+  __builtin_memcpy(&r, p, sizeof(r));
+  return r;
+}
+
+// One right-hand side: a wave per row (walking rows so that a workgroup
+// issues one atomic per Jacobi step), a lane per nonzero.  Consecutive lanes
+// take consecutive nonzeros: their columns are close, so a gather touches few
+// cache lines (four consecutive nonzeros per lane load indices and values in
+// a third of the instructions, but the gathers of 64 lanes then span 256
+// nonzeros: 81 -> 112 us for 35.9 M nonzeros).
 template <typename TA, typename TX, typename TAcc, int MODE>
-__global__ void __launch_bounds__(256) k_csr_rows(
+__global__ void __launch_bounds__(256) k_csr_vec(
     int64_t m, const int64_t *__restrict__ indptr, const int32_t *__restrict__ indices,
-    const TA *__restrict__ data, const TX *__restrict__ X, int64_t nrhs, int R,
-    TX *__restrict__ Y, const TX *__restrict__ E, const TX *__restrict__ rho, double rho_s,
+    const TA *__restrict__ data, const TX *__restrict__ X, TX *__restrict__ Y,
+    const TX *__restrict__ E, const TX *__restrict__ rho, double rho_s,
     double *__restrict__ colmax, int64_t row0) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int G = 64 / R;
-  const int g = lane / R, c = lane % R;
-  // Jacobi steps with at most 64 right-hand sides: each wave walks rows
-  // w0, w0 + (waves in the grid), ... and keeps its column maxima, and the
-  // block issues one atomic per column (one atomic per row from every wave
-  // contends on the same address).  Otherwise one row per wave.
-  const bool stride = MODE != SPMM_PLAIN && nrhs <= 64;
-  const int64_t step = stride ? (int64_t)gridDim.x * (blockDim.x >> 6) : m;
+  const int64_t step = (int64_t)gridDim.x * (blockDim.x >> 6);
   double rmax = 0.0;
   for (int64_t row = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6; row < m;
        row += step) {
-  const int64_t k0 = indptr[row], k1 = indptr[row + 1];
-  for (int64_t c0 = 0; c0 < nrhs; c0 += R) {
-    const int64_t col = c0 + c;
-    const bool active = col < nrhs;
+    const int64_t k0 = indptr[row], k1 = indptr[row + 1];
     TAcc acc = 0;
-    if (active) {
-      // kU consecutive strides per pass: the index and value loads of a pass,
-      // then its gathers, are all in flight before the first product (each
-      // lane still adds its terms in increasing k order)
-      // Loads go out unconditionally from clamped addresses (k1 - 1 >= kb
-      // is a valid entry of this row): a load behind a branch would make
-      // the compiler wait for the earlier ones and serialise the pass.
-      constexpr int kU = 8;
-      for (int64_t kb = k0 + g; kb < k1; kb += (int64_t)kU * G) {
-        int32_t jj[kU];
-        TAcc av[kU], xv[kU];
+    // kU consecutive strides per pass: the index and value loads of a pass,
+    // then its gathers, are all in flight before the first product.  Loads
+    // go out unconditionally from clamped addresses (k1 - 1 is a valid entry
+    // of this row): a load behind a branch would make the compiler wait for
+    // the earlier ones and serialise the pass.
+    constexpr int kU = 8;
+    for (int64_t kb = k0 + lane; kb < k1; kb += kU * 64) {
+      int32_t jj[kU];
+      TAcc av[kU], xv[kU];
 #pragma unroll
-        for (int u = 0; u < kU; ++u) {
-          const int64_t k = min(kb + (int64_t)u * G, k1 - 1);
-          jj[u] = indices[k];
-          av[u] = (TAcc)widen(data[k]);
-        }
-#pragma unroll
-        for (int u = 0; u < kU; ++u) {
-          TAcc x = (TAcc)X[(int64_t)jj[u] * nrhs + col];
-          if (MODE == SPMM_JACOBI_RIGHT) x = (rho ? (TAcc)rho[jj[u]] : (TAcc)rho_s) * x;
-          xv[u] = x;
-        }
-#pragma unroll
-        for (int u = 0; u < kU; ++u)
-          if (kb + (int64_t)u * G < k1) acc += av[u] * xv[u];
+      for (int u = 0; u < kU; ++u) {
+        const int64_t k = min(kb + u * 64, k1 - 1);
+        jj[u] = indices[k];
+        av[u] = (TAcc)widen(data[k]);
       }
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        TAcc x = (TAcc)X[jj[u]];
+        if (MODE == SPMM_JACOBI_RIGHT) x = (rho ? (TAcc)rho[jj[u]] : (TAcc)rho_s) * x;
+        xv[u] = x;
+      }
+#pragma unroll
+      for (int u = 0; u < kU; ++u)
+        if (kb + u * 64 < k1) acc += av[u] * xv[u];
     }
-    for (int off = R; off < 64; off <<= 1) acc += __shfl_xor(acc, off, 64);
-    if (g == 0 && active) {
-      const int64_t o = (row0 + row) * nrhs + col;  // row0: first row of a row chunk
+    for (int off = 1; off < 64; off <<= 1) acc += __shfl_xor(acc, off, 64);
+    if (lane == 0) {
+      const int64_t o = row0 + row;  // row0: first row of a row chunk
       if (MODE == SPMM_PLAIN) {
         Y[o] = (TX)acc;
       } else {
         TAcc y = acc;
-        if (MODE == SPMM_JACOBI_LEFT) y = (rho ? (TAcc)rho[row0 + row] : (TAcc)rho_s) * y;
+        if (MODE == SPMM_JACOBI_LEFT) y = (rho ? (TAcc)rho[o] : (TAcc)rho_s) * y;
         const TX b1 = (TX)((TAcc)E[o] + y);
         Y[o] = b1;
-        const double diff = fabs((double)b1 - (double)X[o]);
-        if (stride)
-          rmax = fmax(rmax, diff);
-        else
-          atomic_max_nonneg(colmax + col, diff);
+        rmax = fmax(rmax, fabs((double)b1 - (double)X[o]));
       }
     }
   }
-  }
-  if (stride) {
-    __shared__ double sd[4][64];
-    sd[w][lane] = lane < R ? rmax : 0.0;
+  if (MODE != SPMM_PLAIN) {
+    __shared__ double sd[4];
+    if (lane == 0) sd[w] = rmax;
     __syncthreads();
-    if (threadIdx.x < R && threadIdx.x < nrhs) {
-      const int t = threadIdx.x;
-      atomic_max_nonneg(colmax + t, fmax(fmax(sd[0][t], sd[1][t]), fmax(sd[2][t], sd[3][t])));
+    if (threadIdx.x == 0)
+      atomic_max_nonneg(colmax, fmax(fmax(sd[0], sd[1]), fmax(sd[2], sd[3])));
+  }
+}
+
+// Products with two or more right-hand sides.  A lane takes V right-hand
+// sides of one nonzero in one 16-byte gather (V = 2 in FP64, 4 in FP32), LP
+// lanes cover a row of X (or of a tile of it: more than 64 V right-hand sides
+// go in equal tiles), and the G = 64 / LP groups of a wave take G nonzeros
+// at a time.  The indices and values of 64 S nonzeros are loaded once,
+// coalesced, a pass ahead, and handed round through LDS (LP = 1: a lane
+// keeps its own), with the albedo of the column multiplied in.
+//
+// What bounds it: with a lane per right-hand side, every lane loading the
+// index, the value and the albedo of its nonzero, it was the rate of the
+// address unit (64 lanes in 16 cycles whatever a lane loads: 4 instructions
+// per 4 nonzeros at 16 FP64 right-hand sides, 10 per 64 here); now it is the
+// gathers from L2 (10.7 M nonzeros, 128 bytes each, in 111 us: 12 TB/s).  10.7
+// M nonzeros, product / Jacobi step with per-facet albedo 'right', us:
+// FP64 k = 3: 53 / 85 -> 48 / 64, k = 8: 97 / 167 -> 72 / 88, k = 16: 187 / 311
+// -> 112 / 134, k = 64: 707 / 1110 -> 390 / 425; FP32 k = 16: 151 / 181 -> 59 /
+// 74.  Workgroups of 8 or 16 waves (neighbouring rows on one CU) were slower.
+//
+// A lane past the end of a row of X loads the row's last V values instead
+// (nothing is read outside X) and stores what no other lane has.
+constexpr int kBlockWaves = 4;
+
+template <typename TA, typename TX, typename TAcc, int MODE, int V, int LP1, int S, int kU>
+__global__ void __launch_bounds__(64 * kBlockWaves) k_csr_block(
+    int64_t m, const int64_t *__restrict__ indptr, const int32_t *__restrict__ indices,
+    const TA *__restrict__ data, const TX *__restrict__ X, int64_t nrhs, int lp_log2,
+    TX *__restrict__ Y, const TX *__restrict__ E, const TX *__restrict__ rho, double rho_s,
+    double *__restrict__ colmax, int64_t row0) {
+  // this workgroup's right-hand sides: tile blockIdx.y of gridDim.y
+  const int64_t c_lo = nrhs * blockIdx.y / gridDim.y, c_hi = nrhs * (blockIdx.y + 1) / gridDim.y;
+  const int cols = (int)(c_hi - c_lo);
+  X += c_lo;
+  Y += c_lo;
+  if (MODE != SPMM_PLAIN) {
+    E += c_lo;
+    colmax += c_lo;
+  }
+  __shared__ int32_t sidx[LP1 ? 1 : kBlockWaves][LP1 ? 1 : 64 * S];
+  __shared__ TAcc sval[LP1 ? 1 : kBlockWaves][LP1 ? 1 : 64 * S];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int LP = LP1 ? 1 : 1 << lp_log2, G = LP1 ? 64 : 64 >> lp_log2;
+  const int g = LP1 ? lane : lane >> lp_log2, c = LP1 ? 0 : (lane & (LP - 1)) * V;
+  const int col = min(c, cols - V);  // cols >= V
+  const int fresh = c - col;         // values below this one belong to another lane
+  const int64_t step = (int64_t)gridDim.x * kBlockWaves;
+  double rmax[V];
+  for (int v = 0; v < V; ++v) rmax[v] = 0.0;
+  for (int64_t row = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6; row < m;
+       row += step) {
+    const int64_t k0 = indptr[row], k1 = indptr[row + 1];
+    TAcc acc[V];
+    for (int v = 0; v < V; ++v) acc[v] = 0;
+    int32_t idx[S];
+    TAcc val[S];
+    auto load = [&](int64_t kb) {
+#pragma unroll
+      for (int u = 0; u < S; ++u) {
+        const int64_t k = min(kb + u * 64 + lane, k1 - 1);
+        idx[u] = indices[k];
+        val[u] = (TAcc)widen(data[k]);
+      }
+    };
+    auto scale = [&]() {
+      if (MODE == SPMM_JACOBI_RIGHT) {
+#pragma unroll
+        for (int u = 0; u < S; ++u) val[u] *= rho ? (TAcc)rho[idx[u]] : (TAcc)rho_s;
+      }
+    };
+    if (k0 < k1) {
+      load(k0);
+      scale();
+    }
+    for (int64_t kb = k0; kb < k1; kb += 64 * S) {
+      const int cnt = (int)min(k1 - kb, (int64_t)(64 * S));
+      if constexpr (LP1) {
+        // a lane's own nonzeros
+        Vec<TX, V> xv[S];
+        TAcc av[S];
+#pragma unroll
+        for (int u = 0; u < S; ++u) {
+          xv[u] = load_vec<V>(X + (int64_t)idx[u] * nrhs + col);
+          av[u] = val[u];
+        }
+        if (kb + 64 * S < k1) load(kb + 64 * S);
+#pragma unroll
+        for (int u = 0; u < S; ++u)
+          if (u * 64 + lane < cnt)
+            for (int v = 0; v < V; ++v) acc[v] += av[u] * (TAcc)xv[u].v[v];
+        if (kb + 64 * S < k1) scale();
+      } else {
+#pragma unroll
+        for (int u = 0; u < S; ++u) {
+          sidx[w][u * 64 + lane] = idx[u];
+          sval[w][u * 64 + lane] = val[u];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        // the next nonzeros, on their way during this pass
+        if (kb + 64 * S < k1) load(kb + 64 * S);
+        // kU groups of nonzeros at a time, the rest of the pass two at a time
+        auto terms = [&](int s, auto groups) {
+          constexpr int n = decltype(groups)::value;
+          TAcc av[n];
+          Vec<TX, V> xv[n];
+#pragma unroll
+          for (int u = 0; u < n; ++u) {
+            const int e = min(s + u * G + g, cnt - 1);
+            av[u] = sval[w][e];
+            xv[u] = load_vec<V>(X + (int64_t)sidx[w][e] * nrhs + col);
+          }
+#pragma unroll
+          for (int u = 0; u < n; ++u)
+            if (s + u * G + g < cnt)
+              for (int v = 0; v < V; ++v) acc[v] += av[u] * (TAcc)xv[u].v[v];
+        };
+        int s = 0;
+        for (; s + (kU - 2) * G < cnt; s += kU * G) terms(s, std::integral_constant<int, kU>());
+        for (; s < cnt; s += 2 * G) terms(s, std::integral_constant<int, 2>());
+        if (kb + 64 * S < k1) scale();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      }
+    }
+    for (int off = LP; off < 64; off <<= 1)
+      for (int v = 0; v < V; ++v) acc[v] += __shfl_xor(acc[v], off, 64);
+    if (g == 0 && c < cols) {
+      const int64_t o = (row0 + row) * nrhs + col;  // row0: first row of a row chunk
+      for (int v = 0; v < V; ++v) {
+        if (v < fresh) continue;
+        if (MODE == SPMM_PLAIN) {
+          Y[o + v] = (TX)acc[v];
+        } else {
+          TAcc y = acc[v];
+          if (MODE == SPMM_JACOBI_LEFT) y = (rho ? (TAcc)rho[row0 + row] : (TAcc)rho_s) * y;
+          const TX b1 = (TX)((TAcc)E[o + v] + y);
+          Y[o + v] = b1;
+          rmax[v] = fmax(rmax[v], fabs((double)b1 - (double)X[o + v]));
+        }
+      }
     }
   }
+  if (MODE != SPMM_PLAIN) {
+    // one atomic per column and workgroup
+    __shared__ double sd[kBlockWaves][64 * V];
+    if (g == 0)
+      for (int v = 0; v < V; ++v) sd[w][(lane & (LP - 1)) * V + v] = rmax[v];
+    __syncthreads();
+    for (int t = threadIdx.x; t < LP * V; t += blockDim.x) {
+      // column of the lane-major slot t, unless another lane has it
+      const int cc = t / V * V, base = min(cc, cols - V), v = t - cc;
+      if (cc < cols && v >= cc - base) {
+        double mx = 0.0;
+        for (int q = 0; q < kBlockWaves; ++q) mx = fmax(mx, sd[q][t]);
+        atomic_max_nonneg(colmax + base + v, mx);
+      }
+    }
+  }
+}
+
+// Workgroups for m rows: a wave per row, so that rows of uneven length spread
+// over the chip as waves end (a wave walking rows took 88 us where this
+// takes 81), except in Jacobi steps, whose workgroups end with atomics on the
+// column maxima (2048 workgroups).
+template <int MODE>
+static unsigned row_blocks(int64_t m) {
+  const int64_t rb = (m + kBlockWaves - 1) / kBlockWaves;
+  const int64_t most = MODE == SPMM_PLAIN ? kMaxGrid1D : 2048;
+  return (unsigned)(rb < most ? rb : most);
+}
+
+template <typename TA, typename TX, int MODE, int V>
+static int launch_block(int64_t m, const int64_t *indptr, const int32_t *indices,
+                        const void *data, const void *X, int64_t nrhs, void *Y, const void *E,
+                        const void *rho, double rho_s, double *colmax, hipStream_t st,
+                        int64_t row0) {
+  using TAcc = typename AccOf<decltype(typename WideOf<TA>::type() + TX())>::type;
+  const int64_t tiles = (nrhs + 64 * V - 1) / (64 * V), width = (nrhs + tiles - 1) / tiles;
+  FLUX_CHECK(tiles <= 65535, "csr product: too many right-hand sides");
+  int lp = 0;
+  while (((int64_t)V << lp) < width) ++lp;
+  const dim3 grid(row_blocks<MODE>(m), (unsigned)tiles);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * kBlockWaves), 0, st, m, indptr, indices,
+                       (const TA *)data, (const TX *)X, nrhs, lp, (TX *)Y, (const TX *)E,
+                       (const TX *)rho, rho_s, colmax, row0);
+  };
+  // nonzeros staged per pass: 64 S; groups in flight: kU (kU G <= 64 S)
+  if (lp == 0)
+    launch(k_csr_block<TA, TX, TAcc, MODE, V, 1, 4, 4>);
+  else if (lp == 1)
+    launch(k_csr_block<TA, TX, TAcc, MODE, V, 0, 2, 4>);
+  else if (lp == 2)
+    launch(k_csr_block<TA, TX, TAcc, MODE, V, 0, 2, 8>);
+  else
+    launch(k_csr_block<TA, TX, TAcc, MODE, V, 0, 1, 8>);
+  FLUX_LAUNCH_CHECK();
+  return 0;
 }
 
 template <typename TA, typename TX, int MODE>
@@ -135,15 +334,18 @@ static int launch_rows(int64_t m, const int64_t *indptr, const int32_t *indices,
                        const void *rho, double rho_s, double *colmax, hipStream_t st,
                        int64_t row0) {
   using TAcc = typename AccOf<decltype(typename WideOf<TA>::type() + TX())>::type;
-  int R = 1;
-  while (R < nrhs && R < 64) R <<= 1;
-  // Jacobi steps with nrhs <= 64 walk rows with a bounded grid (see the kernel)
-  const bool stride = MODE != SPMM_PLAIN && nrhs <= 64;
-  const unsigned rb = ceil_div_u(m, 4), blocks = stride && rb > 2048u ? 2048u : rb;
-  if (blocks == 0) return 0;
-  hipLaunchKernelGGL((k_csr_rows<TA, TX, TAcc, MODE>), dim3(blocks), dim3(256), 0, st, m,
-                     indptr, indices, (const TA *)data, (const TX *)X, nrhs, R, (TX *)Y,
-                     (const TX *)E, (const TX *)rho, rho_s, colmax, row0);
+  constexpr int V = 16 / (int)sizeof(TX);
+  if (m <= 0) return 0;
+  if (nrhs >= V)
+    return launch_block<TA, TX, MODE, V>(m, indptr, indices, data, X, nrhs, Y, E, rho, rho_s,
+                                         colmax, st, row0);
+  if (nrhs >= 2)
+    return launch_block<TA, TX, MODE, 2>(m, indptr, indices, data, X, nrhs, Y, E, rho, rho_s,
+                                         colmax, st, row0);
+  const unsigned blocks = row_blocks<MODE>(m);
+  hipLaunchKernelGGL((k_csr_vec<TA, TX, TAcc, MODE>), dim3(blocks), dim3(256), 0, st, m, indptr,
+                     indices, (const TA *)data, (const TX *)X, (TX *)Y, (const TX *)E,
+                     (const TX *)rho, rho_s, colmax, row0);
   FLUX_LAUNCH_CHECK();
   return 0;
 }
