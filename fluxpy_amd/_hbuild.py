@@ -859,6 +859,10 @@ class HOperator:
                   _lib.ptr(rscale), _lib.stream())
         return Y
 
+    def jacobi_csr(self):
+        """The CSR whose fused Jacobi steps are this operator's, or None."""
+        return self.near if self.fused_jacobi else None
+
     def jacobi_step(self, E, B, rho, left, B1, colmax):
         t = _lib.torch()
         if self.fused_jacobi:

@@ -12,7 +12,25 @@
 
 namespace flux {
 
-enum { SPMM_PLAIN = 0, SPMM_JACOBI_RIGHT = 1, SPMM_JACOBI_LEFT = 2 };
+// SPMM_JACOBI_SCALED: 'right' with X = rho o B kept beside B, so that no
+// nonzero multiplies by (or gathers) an albedo.
+enum { SPMM_PLAIN = 0, SPMM_JACOBI_RIGHT = 1, SPMM_JACOBI_LEFT = 2, SPMM_JACOBI_SCALED = 3 };
+
+// What a Jacobi step takes beside the matrix and its vector X.  B is the
+// iterate X stands for (X itself unless scaled), Xn the next scaled one.
+// prev / tol: the column maxima of the step before and their bounds (tol_cols
+// of them, 1 or one per column); a step after one that met them all does
+// nothing, so a run of steps can be issued without reading the maxima back.
+template <typename TX>
+struct JacobiArgs {
+  const TX *E, *B;
+  TX *Xn;
+  const TX *rho;
+  double rho_s;
+  double *colmax;
+  const double *prev, *tol;
+  int64_t tol_cols;
+};
 
 template <typename T>
 struct AccOf {
@@ -62,6 +80,17 @@ __device__ __forceinline__ Vec<T, V> load_vec(const T *p) {
   return r;
 }
 
+// True if the step before met its bounds in every column (then its column
+// maxima, and this step's, which stay zero, do so for the next step too).
+template <typename TX>
+__device__ __forceinline__ bool jacobi_met(const JacobiArgs<TX> &jac, int64_t nrhs) {
+  if (!jac.prev) return false;
+  bool met = true;
+  for (int64_t c = threadIdx.x & 63; c < nrhs; c += 64)
+    met = met && jac.prev[c] <= jac.tol[jac.tol_cols == 1 ? 0 : c];
+  return __all(met);
+}
+
 // One right-hand side: a wave per row (walking rows so that a workgroup
 // issues one atomic per Jacobi step), a lane per nonzero.  Consecutive lanes
 // take consecutive nonzeros: their columns are close, so a gather touches few
@@ -72,9 +101,11 @@ template <typename TA, typename TX, typename TAcc, int MODE>
 __global__ void __launch_bounds__(256) k_csr_vec(
     int64_t m, const int64_t *__restrict__ indptr, const int32_t *__restrict__ indices,
     const TA *__restrict__ data, const TX *__restrict__ X, TX *__restrict__ Y,
-    const TX *__restrict__ E, const TX *__restrict__ rho, double rho_s,
-    double *__restrict__ colmax, int64_t row0) {
+    JacobiArgs<TX> jac, int64_t row0) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if (MODE != SPMM_PLAIN && jacobi_met(jac, 1)) return;
+  const TX *__restrict__ E = jac.E, *__restrict__ rho = jac.rho, *__restrict__ B = jac.B;
+  const double rho_s = jac.rho_s;
   const int64_t step = (int64_t)gridDim.x * (blockDim.x >> 6);
   double rmax = 0.0;
   for (int64_t row = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6; row < m;
@@ -116,7 +147,8 @@ __global__ void __launch_bounds__(256) k_csr_vec(
         if (MODE == SPMM_JACOBI_LEFT) y = (rho ? (TAcc)rho[o] : (TAcc)rho_s) * y;
         const TX b1 = (TX)((TAcc)E[o] + y);
         Y[o] = b1;
-        rmax = fmax(rmax, fabs((double)b1 - (double)X[o]));
+        if (MODE == SPMM_JACOBI_SCALED) jac.Xn[o] = rho[o] * b1;
+        rmax = fmax(rmax, fabs((double)b1 - (double)B[o]));
       }
     }
   }
@@ -125,7 +157,7 @@ __global__ void __launch_bounds__(256) k_csr_vec(
     if (lane == 0) sd[w] = rmax;
     __syncthreads();
     if (threadIdx.x == 0)
-      atomic_max_nonneg(colmax, fmax(fmax(sd[0], sd[1]), fmax(sd[2], sd[3])));
+      atomic_max_nonneg(jac.colmax, fmax(fmax(sd[0], sd[1]), fmax(sd[2], sd[3])));
   }
 }
 
@@ -155,8 +187,11 @@ template <typename TA, typename TX, typename TAcc, int MODE, int V, int LP1, int
 __global__ void __launch_bounds__(64 * kBlockWaves) k_csr_block(
     int64_t m, const int64_t *__restrict__ indptr, const int32_t *__restrict__ indices,
     const TA *__restrict__ data, const TX *__restrict__ X, int64_t nrhs, int lp_log2,
-    TX *__restrict__ Y, const TX *__restrict__ E, const TX *__restrict__ rho, double rho_s,
-    double *__restrict__ colmax, int64_t row0) {
+    TX *__restrict__ Y, JacobiArgs<TX> jac, int64_t row0) {
+  if (MODE != SPMM_PLAIN && jacobi_met(jac, nrhs)) return;
+  const TX *__restrict__ E = jac.E, *__restrict__ rho = jac.rho, *__restrict__ B = jac.B;
+  const double rho_s = jac.rho_s;
+  double *__restrict__ colmax = jac.colmax;
   // this workgroup's right-hand sides: tile blockIdx.y of gridDim.y
   const int64_t c_lo = nrhs * blockIdx.y / gridDim.y, c_hi = nrhs * (blockIdx.y + 1) / gridDim.y;
   const int cols = (int)(c_hi - c_lo);
@@ -164,6 +199,7 @@ __global__ void __launch_bounds__(64 * kBlockWaves) k_csr_block(
   Y += c_lo;
   if (MODE != SPMM_PLAIN) {
     E += c_lo;
+    B += c_lo;
     colmax += c_lo;
   }
   __shared__ int32_t sidx[LP1 ? 1 : kBlockWaves][LP1 ? 1 : 64 * S];
@@ -265,7 +301,8 @@ __global__ void __launch_bounds__(64 * kBlockWaves) k_csr_block(
           if (MODE == SPMM_JACOBI_LEFT) y = (rho ? (TAcc)rho[row0 + row] : (TAcc)rho_s) * y;
           const TX b1 = (TX)((TAcc)E[o + v] + y);
           Y[o + v] = b1;
-          rmax[v] = fmax(rmax[v], fabs((double)b1 - (double)X[o + v]));
+          if (MODE == SPMM_JACOBI_SCALED) jac.Xn[c_lo + o + v] = rho[row0 + row] * b1;
+          rmax[v] = fmax(rmax[v], fabs((double)b1 - (double)B[o + v]));
         }
       }
     }
@@ -301,9 +338,8 @@ static unsigned row_blocks(int64_t m) {
 
 template <typename TA, typename TX, int MODE, int V>
 static int launch_block(int64_t m, const int64_t *indptr, const int32_t *indices,
-                        const void *data, const void *X, int64_t nrhs, void *Y, const void *E,
-                        const void *rho, double rho_s, double *colmax, hipStream_t st,
-                        int64_t row0) {
+                        const void *data, const void *X, int64_t nrhs, void *Y,
+                        const JacobiArgs<TX> &jac, hipStream_t st, int64_t row0) {
   using TAcc = typename AccOf<decltype(typename WideOf<TA>::type() + TX())>::type;
   const int64_t tiles = (nrhs + 64 * V - 1) / (64 * V), width = (nrhs + tiles - 1) / tiles;
   FLUX_CHECK(tiles <= 65535, "csr product: too many right-hand sides");
@@ -312,8 +348,7 @@ static int launch_block(int64_t m, const int64_t *indptr, const int32_t *indices
   const dim3 grid(row_blocks<MODE>(m), (unsigned)tiles);
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, dim3(64 * kBlockWaves), 0, st, m, indptr, indices,
-                       (const TA *)data, (const TX *)X, nrhs, lp, (TX *)Y, (const TX *)E,
-                       (const TX *)rho, rho_s, colmax, row0);
+                       (const TA *)data, (const TX *)X, nrhs, lp, (TX *)Y, jac, row0);
   };
   // nonzeros staged per pass: 64 S; groups in flight: kU (kU G <= 64 S)
   if (lp == 0)
@@ -330,49 +365,62 @@ static int launch_block(int64_t m, const int64_t *indptr, const int32_t *indices
 
 template <typename TA, typename TX, int MODE>
 static int launch_rows(int64_t m, const int64_t *indptr, const int32_t *indices,
-                       const void *data, const void *X, int64_t nrhs, void *Y, const void *E,
-                       const void *rho, double rho_s, double *colmax, hipStream_t st,
-                       int64_t row0) {
+                       const void *data, const void *X, int64_t nrhs, void *Y,
+                       const JacobiArgs<TX> &jac, hipStream_t st, int64_t row0) {
   using TAcc = typename AccOf<decltype(typename WideOf<TA>::type() + TX())>::type;
   constexpr int V = 16 / (int)sizeof(TX);
   if (m <= 0) return 0;
   if (nrhs >= V)
-    return launch_block<TA, TX, MODE, V>(m, indptr, indices, data, X, nrhs, Y, E, rho, rho_s,
-                                         colmax, st, row0);
+    return launch_block<TA, TX, MODE, V>(m, indptr, indices, data, X, nrhs, Y, jac, st, row0);
   if (nrhs >= 2)
-    return launch_block<TA, TX, MODE, 2>(m, indptr, indices, data, X, nrhs, Y, E, rho, rho_s,
-                                         colmax, st, row0);
+    return launch_block<TA, TX, MODE, 2>(m, indptr, indices, data, X, nrhs, Y, jac, st, row0);
   const unsigned blocks = row_blocks<MODE>(m);
   hipLaunchKernelGGL((k_csr_vec<TA, TX, TAcc, MODE>), dim3(blocks), dim3(256), 0, st, m, indptr,
-                     indices, (const TA *)data, (const TX *)X, (TX *)Y, (const TX *)E,
-                     (const TX *)rho, rho_s, colmax, row0);
+                     indices, (const TA *)data, (const TX *)X, (TX *)Y, jac, row0);
   FLUX_LAUNCH_CHECK();
   return 0;
 }
 
+// A Jacobi step's arguments before the vector type is known.
+struct JacobiVoid {
+  const void *E, *B, *rho;
+  void *Xn;
+  double rho_s;
+  double *colmax;
+  const double *prev, *tol;
+  int64_t tol_cols;
+  template <typename TX>
+  JacobiArgs<TX> as() const {
+    return JacobiArgs<TX>{(const TX *)E, (const TX *)B, (TX *)Xn, (const TX *)rho,
+                          rho_s,         colmax,        prev,     tol,
+                          tol_cols};
+  }
+};
+
 template <int MODE>
 static int dispatch_rows(int64_t m, const int64_t *indptr, const int32_t *indices,
                          const void *data, int dtype, const void *X, int64_t nrhs, void *Y,
-                         int xdtype, const void *E, const void *rho, double rho_s,
-                         double *colmax, hipStream_t st, int64_t row0 = 0) {
+                         int xdtype, const JacobiVoid &jac, hipStream_t st, int64_t row0 = 0) {
   if (dtype == FLUX_F64 && xdtype == FLUX_F64)
-    return launch_rows<double, double, MODE>(m, indptr, indices, data, X, nrhs, Y, E, rho,
-                                             rho_s, colmax, st, row0);
+    return launch_rows<double, double, MODE>(m, indptr, indices, data, X, nrhs, Y,
+                                             jac.as<double>(), st, row0);
   if (dtype == FLUX_F32 && xdtype == FLUX_F64)
-    return launch_rows<float, double, MODE>(m, indptr, indices, data, X, nrhs, Y, E, rho,
-                                            rho_s, colmax, st, row0);
-  if (dtype == FLUX_F64 && xdtype == FLUX_F32)
-    return launch_rows<double, float, MODE>(m, indptr, indices, data, X, nrhs, Y, E, rho,
-                                            rho_s, colmax, st, row0);
-  if (dtype == FLUX_BF16 && xdtype == FLUX_F32)
-    return launch_rows<__hip_bfloat16, float, MODE>(m, indptr, indices, data, X, nrhs, Y, E,
-                                                    rho, rho_s, colmax, st, row0);
-  if (dtype == FLUX_F16 && xdtype == FLUX_F32)
-    return launch_rows<__half, float, MODE>(m, indptr, indices, data, X, nrhs, Y, E, rho,
-                                            rho_s, colmax, st, row0);
+    return launch_rows<float, double, MODE>(m, indptr, indices, data, X, nrhs, Y,
+                                            jac.as<double>(), st, row0);
   if (dtype == FLUX_F32 && xdtype == FLUX_F32)
-    return launch_rows<float, float, MODE>(m, indptr, indices, data, X, nrhs, Y, E, rho,
-                                           rho_s, colmax, st, row0);
+    return launch_rows<float, float, MODE>(m, indptr, indices, data, X, nrhs, Y,
+                                           jac.as<float>(), st, row0);
+  if constexpr (MODE != SPMM_JACOBI_SCALED) {
+    if (dtype == FLUX_F64 && xdtype == FLUX_F32)
+      return launch_rows<double, float, MODE>(m, indptr, indices, data, X, nrhs, Y,
+                                              jac.as<float>(), st, row0);
+    if (dtype == FLUX_BF16 && xdtype == FLUX_F32)
+      return launch_rows<__hip_bfloat16, float, MODE>(m, indptr, indices, data, X, nrhs, Y,
+                                                      jac.as<float>(), st, row0);
+    if (dtype == FLUX_F16 && xdtype == FLUX_F32)
+      return launch_rows<__half, float, MODE>(m, indptr, indices, data, X, nrhs, Y,
+                                              jac.as<float>(), st, row0);
+  }
   set_error("csr product: unsupported dtypes (%d, %d)", dtype, xdtype);
   return -2;
 }
@@ -445,7 +493,7 @@ extern "C" int flux_csr_spmm(int64_t m, int64_t n, const int64_t *indptr,
   if (m == 0 || nrhs == 0) return 0;
   FLUX_CHECK(indptr && X && Y, "flux_csr_spmm: NULL array");
   return dispatch_rows<SPMM_PLAIN>(m, indptr, indices, data, dtype, X, nrhs, Y, xdtype,
-                                   nullptr, nullptr, 0.0, nullptr, as_stream(stream));
+                                   JacobiVoid{}, as_stream(stream));
 }
 
 // Scan of int64 values (formfactor.hip).
@@ -519,14 +567,15 @@ extern "C" int flux_csr_rows_chunk(int64_t m, int64_t row0, const int64_t *indpt
   FLUX_CHECK(mode == 0 || (E && colmax && X != Y),
              "flux_csr_rows_chunk: a Jacobi step needs E, colmax and Y != X");
   hipStream_t st = as_stream(stream);
+  const JacobiVoid jac{E, X, rho, nullptr, rho_scalar, colmax, nullptr, nullptr, 0};
   if (mode == 0)
-    return dispatch_rows<SPMM_PLAIN>(m, indptr, indices, data, dtype, X, nrhs, Y, xdtype,
-                                     nullptr, nullptr, 0.0, nullptr, st, row0);
+    return dispatch_rows<SPMM_PLAIN>(m, indptr, indices, data, dtype, X, nrhs, Y, xdtype, jac, st,
+                                     row0);
   if (mode == 2)
     return dispatch_rows<SPMM_JACOBI_LEFT>(m, indptr, indices, data, dtype, X, nrhs, Y, xdtype,
-                                           E, rho, rho_scalar, colmax, st, row0);
+                                           jac, st, row0);
   return dispatch_rows<SPMM_JACOBI_RIGHT>(m, indptr, indices, data, dtype, X, nrhs, Y, xdtype,
-                                          E, rho, rho_scalar, colmax, st, row0);
+                                          jac, st, row0);
 }
 
 extern "C" int flux_csr_jacobi_step(int64_t m, const int64_t *indptr, const int32_t *indices,
@@ -542,9 +591,52 @@ extern "C" int flux_csr_jacobi_step(int64_t m, const int64_t *indptr, const int3
   hipLaunchKernelGGL(k_fill_f64, dim3(ceil_div_u(nrhs, 256)), dim3(256), 0, st, colmax, nrhs,
                      0.0);
   FLUX_LAUNCH_CHECK();
+  const JacobiVoid jac{E, B, rho, nullptr, rho_scalar, colmax, nullptr, nullptr, 0};
   if (left)
     return dispatch_rows<SPMM_JACOBI_LEFT>(m, indptr, indices, data, dtype, B, nrhs, B1, xdtype,
-                                           E, rho, rho_scalar, colmax, st);
+                                           jac, st);
   return dispatch_rows<SPMM_JACOBI_RIGHT>(m, indptr, indices, data, dtype, B, nrhs, B1, xdtype,
-                                          E, rho, rho_scalar, colmax, st);
+                                          jac, st);
+}
+
+extern "C" int flux_csr_jacobi_run(int64_t m, const int64_t *indptr, const int32_t *indices,
+                                   const void *data, int dtype, const void *E, void *B0, void *B1,
+                                   void *X0, void *X1, int64_t nrhs, const void *rho,
+                                   double rho_scalar, int left, int xdtype, const double *tol,
+                                   int64_t tol_cols, int64_t first, int64_t nsteps,
+                                   double *colmax, void *stream) {
+  FLUX_CHECK(m >= 0 && nrhs >= 0 && first >= 0 && nsteps >= 0,
+             "flux_csr_jacobi_run: negative sizes");
+  if (m == 0 || nrhs == 0 || nsteps == 0) return 0;
+  FLUX_CHECK(indptr && E && B0 && B1 && tol && colmax, "flux_csr_jacobi_run: NULL array");
+  FLUX_CHECK(B0 != B1, "flux_csr_jacobi_run: B0 and B1 must not alias");
+  FLUX_CHECK(tol_cols == 1 || tol_cols == nrhs, "flux_csr_jacobi_run: tol_cols");
+  FLUX_CHECK(!X0 == !X1 && (!X0 || (rho && !left && X0 != X1)),
+             "flux_csr_jacobi_run: scaled iterates need rho, 'right' and two buffers");
+  hipStream_t st = as_stream(stream);
+  const int64_t nm = nsteps * nrhs;
+  hipLaunchKernelGGL(k_fill_f64, dim3(ceil_div_u(nm, 256)), dim3(256), 0, st, colmax, nm, 0.0);
+  FLUX_LAUNCH_CHECK();
+  for (int64_t s = 0; s < nsteps; ++s) {
+    const bool odd = (first + s) & 1;
+    void *B = odd ? B1 : B0, *Bn = odd ? B0 : B1;
+    void *X = X0 ? (odd ? X1 : X0) : B, *Xn = X0 ? (odd ? X0 : X1) : nullptr;
+    const JacobiVoid jac{E,          B,
+                         rho,        Xn,
+                         rho_scalar, colmax + s * nrhs,
+                         s > 0 ? colmax + (s - 1) * nrhs : nullptr,
+                         tol,        tol_cols};
+    int rc;
+    if (X0)
+      rc = dispatch_rows<SPMM_JACOBI_SCALED>(m, indptr, indices, data, dtype, X, nrhs, Bn, xdtype,
+                                             jac, st);
+    else if (left || !rho)  // F (rho x) = rho (F x) for a scalar
+      rc = dispatch_rows<SPMM_JACOBI_LEFT>(m, indptr, indices, data, dtype, X, nrhs, Bn, xdtype,
+                                           jac, st);
+    else
+      rc = dispatch_rows<SPMM_JACOBI_RIGHT>(m, indptr, indices, data, dtype, X, nrhs, Bn, xdtype,
+                                            jac, st);
+    if (rc) return rc;
+  }
+  return 0;
 }

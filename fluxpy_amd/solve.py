@@ -39,6 +39,9 @@ class _CsrOperator:
     def apply(self, X, out=None):
         return self.csr.matmat(X, out=out)
 
+    def jacobi_csr(self):
+        return self.csr
+
     def jacobi_step(self, E, B, rho, left, B1, colmax):
         t = _lib.torch()
         n = B.shape[0]
@@ -145,9 +148,12 @@ def solve_radiosity(FF, E, rho=1, albedo_placement='right', method='jacobi', tol
     E2 = _to_internal(op, E2)
     left = albedo_placement == 'left'
     if method == 'jacobi':
-        if tol is None:
-            emax = float(abs(E).max()) if host else float(Ed.abs().max())
-            tol = np.finfo(np.dtype(str(E2.dtype).replace("torch.", ""))).resolution * emax
+        res = np.finfo(np.dtype(str(E2.dtype).replace("torch.", ""))).resolution
+        if tol is None and not host and _run_csr(op) is not None:
+            # the tolerance stays on the device, with the convergence test
+            tol = (Ed.abs().max() * float(res)).reshape(1)
+        elif tol is None:
+            tol = res * (float(abs(E).max()) if host else float(Ed.abs().max()))
         B, niter = _jacobi(op, E2, rho_d, left, tol, maxiter or 100000)
     elif method == 'cg':
         if tol is None:
@@ -164,10 +170,21 @@ def solve_radiosity(FF, E, rho=1, albedo_placement='right', method='jacobi', tol
     return (B.cpu().numpy() if host else B), niter
 
 
+def _run_csr(op):
+    """The CSR of an operator whose Jacobi steps are the fused CSR ones, or
+    None."""
+    return op.jacobi_csr() if hasattr(op, "jacobi_csr") else None
+
+
 def _jacobi(op, E, rho, left, tol, maxiter):
-    """solve.py:25-45, fused into one kernel per iteration for CSR operators."""
+    """solve.py:25-45, fused into one kernel per iteration for CSR operators.
+    ``tol``: a scalar, one value per column, or a device vector of either
+    (operators with a ``_run_csr`` only)."""
     t = _lib.torch()
     k = E.shape[1]
+    csr = _run_csr(op)
+    if csr is not None:
+        return _jacobi_runs(csr, E, rho, left, tol, maxiter)
     tol_c = np.broadcast_to(np.asarray(tol, dtype=np.float64), (k,))
     B = E.clone()
     B1 = t.empty_like(E)
@@ -180,11 +197,75 @@ def _jacobi(op, E, rho, left, tol, maxiter):
         if np.all(d <= tol_c):
             break
         if niter >= maxiter:
-            warnings.warn(f"Jacobi did not converge in {maxiter} iterations "
-                          f"(max |B1 - B| = {d.max():.3e} > tol)", RuntimeWarning)
+            _warn_jacobi(maxiter, d)
             break
         B, B1 = B1, B
     return B, niter
+
+
+def _warn_jacobi(maxiter, d):
+    warnings.warn(f"Jacobi did not converge in {maxiter} iterations "
+                  f"(max |B1 - B| = {d.max():.3e} > tol)", RuntimeWarning)
+
+
+JACOBI_RUN = (6, 24)    # iterations of the first run, and at most in any
+
+
+def _jacobi_runs(csr, E, rho, left, tol, maxiter):
+    """The same iteration in runs of several steps per call and readback.  A
+    step after the one that met the tolerance writes nothing
+    (``flux_csr_jacobi_run``), so the host finds the iterate that the
+    step-by-step loop returns.  A run after the first has the length that the
+    maxima's rate of decrease predicts."""
+    t = _lib.torch()
+    n, k = E.shape
+    f64 = t.float64
+    if isinstance(tol, t.Tensor):
+        tol_d = tol.to(f64)
+    elif np.ndim(tol) == 0 or np.size(tol) == 1:
+        tol_d = t.full((1,), float(np.asarray(tol).reshape(())), dtype=f64, device=E.device)
+    else:
+        tol_d = _lib.to_dev(np.ascontiguousarray(
+            np.broadcast_to(np.asarray(tol, dtype=np.float64), (k,))))
+    rho_t, rho_s = (rho, 0.0) if isinstance(rho, t.Tensor) else (None, float(rho))
+    B, B1 = E.clone(), t.empty_like(E)
+    X = X1 = None
+    # rho o B beside B, unless that would round FP64 products to FP32
+    if rho_t is not None and not left and (csr.data.dtype, E.dtype) != (f64, t.float32) \
+            and csr.data.dtype in (f64, t.float32):
+        X, X1 = _kernels.rowscale(rho_t, B), t.empty_like(B)
+    first, most = JACOBI_RUN
+    # a run's maxima and the tolerances, read back together
+    back = t.empty((most + 1) * k, dtype=f64, device=E.device)
+    back[most * k:] = tol_d
+    niter, steps, last = 0, first, None
+    while True:
+        steps = min(steps, maxiter - niter)
+        _lib.call("flux_csr_jacobi_run", n, csr.indptr.data_ptr(), csr.indices.data_ptr(),
+                  csr.data.data_ptr(), _lib.dtype_code(csr.data.dtype), E.data_ptr(),
+                  B.data_ptr(), B1.data_ptr(), _lib.ptr(X), _lib.ptr(X1), k, _lib.ptr(rho_t),
+                  rho_s, int(left), _lib.dtype_code(E.dtype), tol_d.data_ptr(), tol_d.numel(),
+                  niter, steps, back.data_ptr(), _lib.stream())
+        h = back.cpu().numpy().reshape(most + 1, k)
+        d, tol_c = h[:steps], h[most]
+        met = (d <= tol_c).all(1)
+        if met.any():
+            niter += int(met.argmax()) + 1
+            break
+        niter += steps
+        if niter >= maxiter:
+            _warn_jacobi(maxiter, d[-1])
+            break
+        # iterations left: the worst column's excess over its rate
+        with np.errstate(all="ignore"):
+            over = (d[-1] / tol_c).max()
+            prev = d[-2].max() if steps > 1 else (last if last is not None else np.inf)
+            rate = d[-1].max() / prev
+            left_ = np.log(over) / -np.log(rate)
+        last = d[-1].max()
+        steps = int(min(max(np.ceil(left_), 1), most)) if np.isfinite(left_) else first
+    # the iterate before the last update
+    return (B if niter % 2 else B1), niter
 
 
 def _cg(op, E, rho, left, tol, maxiter):

@@ -224,6 +224,22 @@ int flux_csr_jacobi_step(int64_t m, const int64_t *indptr,
                          const void *rho, double rho_scalar, int left,
                          void *B1, int xdtype, double *colmax, void *stream);
 
+/* nsteps of those iterations in one call, without a readback between them.
+ * Iteration first + s reads B[(first + s) % 2] and writes the other of B0,
+ * B1, its column maxima go to colmax + s nrhs (nsteps x nrhs doubles), and
+ * iterations after one whose maxima are all <= tol (tol_cols device doubles,
+ * 1 or nrhs) write nothing and leave zero maxima.  X0, X1: NULL, or for
+ * 'right' with a per-facet albedo the iterates rho o B beside B0, B1 (the
+ * caller fills the one of iteration `first`), which spares every nonzero the
+ * albedo; matrix and vectors then in FP32 or in FP64 vectors only. */
+int flux_csr_jacobi_run(int64_t m, const int64_t *indptr,
+                        const int32_t *indices, const void *data, int dtype,
+                        const void *E, void *B0, void *B1, void *X0, void *X1,
+                        int64_t nrhs, const void *rho, double rho_scalar,
+                        int left, int xdtype, const double *tol,
+                        int64_t tol_cols, int64_t first, int64_t nsteps,
+                        double *colmax, void *stream);
+
 /* ---------------------------------------------------------------------- */
 /* Hierarchical compression (compressed_form_factors.py:285-405 and        */
 /* linalg.py:8-50).  Block descriptors are int64 rows (r0, r1, c0, c1) of  */

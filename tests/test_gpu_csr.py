@@ -65,3 +65,60 @@ def test_products_and_jacobi_steps(adt, xdt, k):
             assert (np.abs(got - want)
                     <= bound(absA @ np.abs(Xh) + np.abs(Eh), want)).all()
             assert np.array_equal(cm.cpu().numpy(), np.abs(got - Xh).max(0))
+
+
+@pytest.mark.parametrize("k", [1, 3, 16])
+@pytest.mark.parametrize("adt,xdt", [("f64", "f64"), ("f32", "f64"), ("f64", "f32"),
+                                     ("f32", "f32"), ("bf16", "f32")])
+@pytest.mark.parametrize("placement", ["left", "right", "scalar"])
+def test_runs_equal_single_steps(adt, xdt, k, placement):
+    """Runs of Jacobi steps return the iterate and the count of the loop that
+    reads the maxima back after every step: convergence inside the first run,
+    in a later one, at the first step, at an iteration limit, and columns
+    with tolerances of their own."""
+    import torch
+    import warnings
+    from fluxpy_amd import _kernels
+    from fluxpy_amd.solve import _CsrOperator, _jacobi_runs
+    torch.cuda.set_device(0)
+    n = 600
+    rng = np.random.default_rng(k)
+    A = _matrix(n, n, rng, np.float64 if adt == "f64" else np.float32)
+    A.data *= 0.9 / A.sum(1).max()
+    csr = _kernels.DeviceCSR.from_scipy(A)
+    if adt == "bf16":
+        csr = csr.astype(torch.bfloat16)
+    xt = torch.float64 if xdt == "f64" else torch.float32
+    E = torch.from_numpy(rng.uniform(0, 1, (n, k))).cuda().to(xt)
+    rho = 0.6 if placement == "scalar" else \
+        torch.from_numpy(rng.uniform(0.5, 0.7, n)).cuda().to(xt)
+    left = placement == "left"
+    op = _CsrOperator(csr)
+
+    def steps(tol, maxiter):
+        B, B1 = E.clone(), torch.empty_like(E)
+        cm = torch.empty(k, dtype=torch.float64, device="cuda")
+        for it in range(1, maxiter + 1):
+            op.jacobi_step(E, B, rho, left, B1, cm)
+            if (cm.cpu().numpy() <= tol).all():
+                break
+            B, B1 = B1, B
+        else:
+            B = B1      # the loop breaks before its last swap
+        return B, it
+
+    eps = np.finfo(np.float64 if xdt == "f64" else np.float32).eps
+    tols = [3.0, 1e-2, 3e-6] + ([1e-12] if xdt == "f64" else [])
+    for tol, maxiter in [(x, 500) for x in tols] + [(1e-9, 4), (1e-9, 7), (1e-9, 1)]:
+        cols = np.full(k, tol) * np.linspace(1.0, 3.0, k)
+        for bound in (tol, cols, torch.from_numpy(cols).cuda()):
+            lim = np.broadcast_to(tol if np.ndim(bound) == 0 else cols, (k,))
+            want, it = steps(lim, maxiter)
+            with warnings.catch_warnings():
+                warnings.simplefilter("ignore")
+                got, niter = _jacobi_runs(csr, E, rho, left, bound, maxiter)
+            # the albedo may multiply elsewhere: a rounding per term and step,
+            # summed over a contraction of 0.63
+            assert niter == it
+            d = (got - want).abs().max() / want.abs().max()
+            assert d <= 30 * eps, (tol, maxiter, float(d))
