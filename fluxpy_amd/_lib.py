@@ -51,7 +51,7 @@ SIGNATURES = {
                                      _c_int, _vp, _vp, _c_dbl, _c_int, _vp, _vp]),
     "flux_csr_jacobi_run": (_c_int, [_c_i64, _vp, _vp, _vp, _c_int, _vp, _vp, _vp, _vp, _vp,
                                      _c_i64, _vp, _c_dbl, _c_int, _c_int, _vp, _c_i64, _c_i64,
-                                     _c_i64, _vp, _vp]),
+                                     _c_i64, _c_int, _vp, _vp]),
     "flux_csr_jacobi_step": (_c_int, [_c_i64, _vp, _vp, _vp, _c_int, _vp, _vp, _c_i64, _vp,
                                       _c_dbl, _c_int, _vp, _c_int, _vp, _vp]),
     "flux_csr_transpose": (_c_int, [_c_i64, _c_i64, _vp, _vp, _vp, _c_int, _vp, _vp, _vp,

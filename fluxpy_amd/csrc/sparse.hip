@@ -21,6 +21,11 @@ enum { SPMM_PLAIN = 0, SPMM_JACOBI_RIGHT = 1, SPMM_JACOBI_LEFT = 2, SPMM_JACOBI_
 // prev / tol: the column maxima of the step before and their bounds (tol_cols
 // of them, 1 or one per column); a step after one that met them all does
 // nothing, so a run of steps can be issued without reading the maxima back.
+// The maxima are kept in `slots` rows of one value per column, 256 bytes or
+// more apart, and workgroups are dealt out over them: atomics on one cache
+// line take about 10 ns each, and with the rows the step also needs no cap on
+// its workgroups (1 column of 20,402 facets: 36 us with one row and 2,048
+// workgroups, 24 with 16 rows; 64 values side by side: 72).
 template <typename TX>
 struct JacobiArgs {
   const TX *E, *B;
@@ -30,6 +35,7 @@ struct JacobiArgs {
   double *colmax;
   const double *prev, *tol;
   int64_t tol_cols;
+  int slots;  // a power of two
 };
 
 template <typename T>
@@ -80,14 +86,24 @@ __device__ __forceinline__ Vec<T, V> load_vec(const T *p) {
   return r;
 }
 
+// Distance of the rows of column maxima, in doubles.
+__host__ __device__ __forceinline__ int64_t slot_stride(int64_t nrhs) {
+  return (nrhs + 31) / 32 * 32;
+}
+
 // True if the step before met its bounds in every column (then its column
 // maxima, and this step's, which stay zero, do so for the next step too).
 template <typename TX>
 __device__ __forceinline__ bool jacobi_met(const JacobiArgs<TX> &jac, int64_t nrhs) {
   if (!jac.prev) return false;
   bool met = true;
-  for (int64_t c = threadIdx.x & 63; c < nrhs; c += 64)
-    met = met && jac.prev[c] <= jac.tol[jac.tol_cols == 1 ? 0 : c];
+  const int lane = threadIdx.x & 63;
+  int kk = 1;  // lanes per slot
+  while (kk < nrhs && kk < 64) kk <<= 1;
+  const int64_t stride = slot_stride(nrhs);
+  for (int s = lane / kk; s < jac.slots; s += 64 / kk)
+    for (int64_t c = lane & (kk - 1); c < nrhs; c += 64)
+      met = met && jac.prev[s * stride + c] <= jac.tol[jac.tol_cols == 1 ? 0 : c];
   return __all(met);
 }
 
@@ -157,7 +173,8 @@ __global__ void __launch_bounds__(256) k_csr_vec(
     if (lane == 0) sd[w] = rmax;
     __syncthreads();
     if (threadIdx.x == 0)
-      atomic_max_nonneg(jac.colmax, fmax(fmax(sd[0], sd[1]), fmax(sd[2], sd[3])));
+      atomic_max_nonneg(jac.colmax + (blockIdx.x & (jac.slots - 1)) * slot_stride(1),
+                        fmax(fmax(sd[0], sd[1]), fmax(sd[2], sd[3])));
   }
 }
 
@@ -200,7 +217,7 @@ __global__ void __launch_bounds__(64 * kBlockWaves) k_csr_block(
   if (MODE != SPMM_PLAIN) {
     E += c_lo;
     B += c_lo;
-    colmax += c_lo;
+    colmax += (blockIdx.x & (jac.slots - 1)) * slot_stride(nrhs) + c_lo;
   }
   __shared__ int32_t sidx[LP1 ? 1 : kBlockWaves][LP1 ? 1 : 64 * S];
   __shared__ TAcc sval[LP1 ? 1 : kBlockWaves][LP1 ? 1 : 64 * S];
@@ -327,12 +344,12 @@ __global__ void __launch_bounds__(64 * kBlockWaves) k_csr_block(
 
 // Workgroups for m rows: a wave per row, so that rows of uneven length spread
 // over the chip as waves end (a wave walking rows took 88 us where this
-// takes 81), except in Jacobi steps, whose workgroups end with atomics on the
-// column maxima (2048 workgroups).
+// takes 81), except in Jacobi steps whose workgroups all end with atomics on
+// the same column maxima (2048 workgroups).
 template <int MODE>
-static unsigned row_blocks(int64_t m) {
+static unsigned row_blocks(int64_t m, int slots) {
   const int64_t rb = (m + kBlockWaves - 1) / kBlockWaves;
-  const int64_t most = MODE == SPMM_PLAIN ? kMaxGrid1D : 2048;
+  const int64_t most = MODE == SPMM_PLAIN || slots > 1 ? kMaxGrid1D : 2048;
   return (unsigned)(rb < most ? rb : most);
 }
 
@@ -345,7 +362,7 @@ static int launch_block(int64_t m, const int64_t *indptr, const int32_t *indices
   FLUX_CHECK(tiles <= 65535, "csr product: too many right-hand sides");
   int lp = 0;
   while (((int64_t)V << lp) < width) ++lp;
-  const dim3 grid(row_blocks<MODE>(m), (unsigned)tiles);
+  const dim3 grid(row_blocks<MODE>(m, jac.slots), (unsigned)tiles);
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, dim3(64 * kBlockWaves), 0, st, m, indptr, indices,
                        (const TA *)data, (const TX *)X, nrhs, lp, (TX *)Y, jac, row0);
@@ -374,7 +391,7 @@ static int launch_rows(int64_t m, const int64_t *indptr, const int32_t *indices,
     return launch_block<TA, TX, MODE, V>(m, indptr, indices, data, X, nrhs, Y, jac, st, row0);
   if (nrhs >= 2)
     return launch_block<TA, TX, MODE, 2>(m, indptr, indices, data, X, nrhs, Y, jac, st, row0);
-  const unsigned blocks = row_blocks<MODE>(m);
+  const unsigned blocks = row_blocks<MODE>(m, jac.slots);
   hipLaunchKernelGGL((k_csr_vec<TA, TX, TAcc, MODE>), dim3(blocks), dim3(256), 0, st, m, indptr,
                      indices, (const TA *)data, (const TX *)X, (TX *)Y, jac, row0);
   FLUX_LAUNCH_CHECK();
@@ -389,11 +406,12 @@ struct JacobiVoid {
   double *colmax;
   const double *prev, *tol;
   int64_t tol_cols;
+  int slots = 1;
   template <typename TX>
   JacobiArgs<TX> as() const {
     return JacobiArgs<TX>{(const TX *)E, (const TX *)B, (TX *)Xn, (const TX *)rho,
                           rho_s,         colmax,        prev,     tol,
-                          tol_cols};
+                          tol_cols,      slots};
   }
 };
 
@@ -567,7 +585,7 @@ extern "C" int flux_csr_rows_chunk(int64_t m, int64_t row0, const int64_t *indpt
   FLUX_CHECK(mode == 0 || (E && colmax && X != Y),
              "flux_csr_rows_chunk: a Jacobi step needs E, colmax and Y != X");
   hipStream_t st = as_stream(stream);
-  const JacobiVoid jac{E, X, rho, nullptr, rho_scalar, colmax, nullptr, nullptr, 0};
+  const JacobiVoid jac{E, X, rho, nullptr, rho_scalar, colmax, nullptr, nullptr, 0, 1};
   if (mode == 0)
     return dispatch_rows<SPMM_PLAIN>(m, indptr, indices, data, dtype, X, nrhs, Y, xdtype, jac, st,
                                      row0);
@@ -591,7 +609,7 @@ extern "C" int flux_csr_jacobi_step(int64_t m, const int64_t *indptr, const int3
   hipLaunchKernelGGL(k_fill_f64, dim3(ceil_div_u(nrhs, 256)), dim3(256), 0, st, colmax, nrhs,
                      0.0);
   FLUX_LAUNCH_CHECK();
-  const JacobiVoid jac{E, B, rho, nullptr, rho_scalar, colmax, nullptr, nullptr, 0};
+  const JacobiVoid jac{E, B, rho, nullptr, rho_scalar, colmax, nullptr, nullptr, 0, 1};
   if (left)
     return dispatch_rows<SPMM_JACOBI_LEFT>(m, indptr, indices, data, dtype, B, nrhs, B1, xdtype,
                                            jac, st);
@@ -604,17 +622,19 @@ extern "C" int flux_csr_jacobi_run(int64_t m, const int64_t *indptr, const int32
                                    void *X0, void *X1, int64_t nrhs, const void *rho,
                                    double rho_scalar, int left, int xdtype, const double *tol,
                                    int64_t tol_cols, int64_t first, int64_t nsteps,
-                                   double *colmax, void *stream) {
+                                   int slots, double *colmax, void *stream) {
   FLUX_CHECK(m >= 0 && nrhs >= 0 && first >= 0 && nsteps >= 0,
              "flux_csr_jacobi_run: negative sizes");
   if (m == 0 || nrhs == 0 || nsteps == 0) return 0;
   FLUX_CHECK(indptr && E && B0 && B1 && tol && colmax, "flux_csr_jacobi_run: NULL array");
   FLUX_CHECK(B0 != B1, "flux_csr_jacobi_run: B0 and B1 must not alias");
   FLUX_CHECK(tol_cols == 1 || tol_cols == nrhs, "flux_csr_jacobi_run: tol_cols");
+  FLUX_CHECK(slots >= 1 && slots <= 1024 && (slots & (slots - 1)) == 0,
+             "flux_csr_jacobi_run: slots must be a power of two up to 1024");
   FLUX_CHECK(!X0 == !X1 && (!X0 || (rho && !left && X0 != X1)),
              "flux_csr_jacobi_run: scaled iterates need rho, 'right' and two buffers");
   hipStream_t st = as_stream(stream);
-  const int64_t nm = nsteps * nrhs;
+  const int64_t ns = slots * slot_stride(nrhs), nm = nsteps * ns;
   hipLaunchKernelGGL(k_fill_f64, dim3(ceil_div_u(nm, 256)), dim3(256), 0, st, colmax, nm, 0.0);
   FLUX_LAUNCH_CHECK();
   for (int64_t s = 0; s < nsteps; ++s) {
@@ -623,9 +643,10 @@ extern "C" int flux_csr_jacobi_run(int64_t m, const int64_t *indptr, const int32
     void *X = X0 ? (odd ? X1 : X0) : B, *Xn = X0 ? (odd ? X0 : X1) : nullptr;
     const JacobiVoid jac{E,          B,
                          rho,        Xn,
-                         rho_scalar, colmax + s * nrhs,
-                         s > 0 ? colmax + (s - 1) * nrhs : nullptr,
-                         tol,        tol_cols};
+                         rho_scalar, colmax + s * ns,
+                         s > 0 ? colmax + (s - 1) * ns : nullptr,
+                         tol,        tol_cols,
+                         slots};
     int rc;
     if (X0)
       rc = dispatch_rows<SPMM_JACOBI_SCALED>(m, indptr, indices, data, dtype, X, nrhs, Bn, xdtype,

@@ -226,9 +226,11 @@ int flux_csr_jacobi_step(int64_t m, const int64_t *indptr,
 
 /* nsteps of those iterations in one call, without a readback between them.
  * Iteration first + s reads B[(first + s) % 2] and writes the other of B0,
- * B1, its column maxima go to colmax + s nrhs (nsteps x nrhs doubles), and
- * iterations after one whose maxima are all <= tol (tol_cols device doubles,
- * 1 or nrhs) write nothing and leave zero maxima.  X0, X1: NULL, or for
+ * B1, and its column maxima go to colmax (nsteps x slots rows of nrhs doubles
+ * rounded up to 32; the maximum of a column is the largest of its `slots`
+ * values, a power of two: workgroups are dealt out over them).  Iterations
+ * after one whose maxima are all <= tol (tol_cols device doubles, 1 or nrhs)
+ * write nothing and leave zero maxima.  X0, X1: NULL, or for
  * 'right' with a per-facet albedo the iterates rho o B beside B0, B1 (the
  * caller fills the one of iteration `first`), which spares every nonzero the
  * albedo; matrix and vectors then in FP32 or in FP64 vectors only. */
@@ -238,7 +240,7 @@ int flux_csr_jacobi_run(int64_t m, const int64_t *indptr,
                         int64_t nrhs, const void *rho, double rho_scalar,
                         int left, int xdtype, const double *tol,
                         int64_t tol_cols, int64_t first, int64_t nsteps,
-                        double *colmax, void *stream);
+                        int slots, double *colmax, void *stream);
 
 /* ---------------------------------------------------------------------- */
 /* Hierarchical compression (compressed_form_factors.py:285-405 and        */
