@@ -78,65 +78,85 @@ def _svd_nbytes(m, n, nzrows, nzcols, k, itemsize):
 
 
 class _Cluster:
-    __slots__ = ("start", "end", "idx", "children", "parts", "level")
+    """The facets of one quadrant / octant.  ``children`` (list of _Cluster,
+    None if it does not split) and ``parts`` (their local positions, the
+    reference's _row_block_inds) are worked out when they are first asked
+    for: a build looks at the clusters its blocks reach, 85 of the 4,900 of a
+    1,922-facet crater at 4 levels of blocks."""
+    __slots__ = ("start", "end", "idx", "children", "parts", "level", "tree")
 
-    def __init__(self, start, end, idx, level):
+    def __init__(self, start, end, idx, level, tree):
         self.start, self.end, self.idx, self.level = start, end, idx, level
-        self.children = None     # list of _Cluster
-        self.parts = None        # local positions (reference _row_block_inds)
+        self.tree = tree
+
+    def __getattr__(self, name):     # only for slots not set yet
+        if name not in ("children", "parts"):
+            raise AttributeError(name)
+        parts, children = self.tree._children(self)
+        self.parts, self.children = parts, children
+        return children if name == "children" else parts
 
 
 class _ClusterTree:
     """Quadtree / octree of the centroids; ``perm`` orders the facets so that
     every cluster is the range [start, end)."""
+    max_levels = 48      # also of trees in files saved without it
 
     def __init__(self, P, dims, max_levels=48):
         self.dims = dims
         self.order = get_quadrant_order if dims == 2 else get_octant_order
+        self.max_levels = max_levels
         n = P.shape[0]
         self.P = P
-        self.root = _Cluster(0, n, np.arange(n), 0)
-        # split breadth first; a cluster stops splitting when it has <= 1
-        # point or all its points coincide (the split would not shrink it)
-        frontier = [self.root]
+        self.root = _Cluster(0, n, np.arange(n), 0, self)
+        self._sort(n)
+        self.iperm = np.empty_like(self.perm)
+        self.iperm[self.perm] = np.arange(n)
+
+    def _sort(self, n):
+        """``perm`` and ``levels``: the clusters of a level split together.  A
+        cluster is a run of ``perm``; sorting the run by child (the quadrant
+        or octant numbers of ``order``), stably, makes every child a run.  One
+        call of ``order`` per cluster took 16.6 ms at 1,922 facets (1,225
+        clusters that split), half of the matrix's construction; this takes
+        about 1 ms."""
+        perm = np.arange(n, dtype=np.int64)
+        P, dims = self.P[:, :self.dims], self.dims
         self.levels = 0
-        while frontier and self.levels < max_levels:
-            nxt = []
-            for c in frontier:
-                if c.idx.size <= 1:
-                    continue
-                parts = self.order(P[c.idx, :dims])
-                if max(p.size for p in parts) == c.idx.size:
-                    continue
-                c.parts = parts
-                c.children = [_Cluster(0, 0, c.idx[p], c.level + 1) for p in parts]
-                nxt.extend(ch for ch in c.children if ch.idx.size > 1)
-            if nxt:
-                self.levels += 1
-            frontier = nxt
-        # permutation: leaves in DFS preorder; a cluster is then the
-        # contiguous range from its first child's start to its last child's end
-        perm = np.empty(n, dtype=np.int64)
-        pos = 0
-        stack = [self.root]
-        order = []
-        while stack:
-            c = stack.pop()
-            order.append(c)
-            if c.children is not None:
-                stack.extend(reversed(c.children))
-        for c in order:
-            if c.children is None:
-                c.start = pos
-                perm[pos:pos + c.idx.size] = c.idx
-                pos += c.idx.size
-                c.end = pos
-        for c in reversed(order):
-            if c.children is not None:
-                c.start, c.end = c.children[0].start, c.children[-1].end
+        at = np.arange(n)                       # places in perm still to split,
+        sizes = np.array([n] if n > 1 else [], dtype=np.int64)      # by cluster
+        while sizes.size and self.levels < self.max_levels:
+            X = P[perm[at]]
+            first = np.cumsum(sizes) - sizes
+            mid = (np.minimum.reduceat(X, first, axis=0)
+                   + np.maximum.reduceat(X, first, axis=0)) / 2
+            high = ~(X <= np.repeat(mid, sizes, axis=0))
+            key = np.repeat(np.arange(sizes.size), sizes)
+            for d in range(dims):
+                key = 2 * key + high[:, d]
+            counts = np.bincount(key, minlength=sizes.size << dims).reshape(sizes.size, -1)
+            perm[at] = perm[at][np.argsort(key, kind="stable")]
+            # children of one point are done, and so are clusters whose points
+            # all fall into one child (they coincide)
+            more = (counts > 1) & (counts.max(axis=1) < sizes)[:, None]
+            at = at[np.repeat(more.ravel(), counts.ravel())]
+            sizes = counts[more]
+            self.levels += int(sizes.size > 0)
         self.perm = perm
-        self.iperm = np.empty_like(perm)
-        self.iperm[perm] = np.arange(n)
+
+    def _children(self, c):
+        """(parts, children) of c, (None, None) if it has <= 1 point or all
+        its points coincide (a split would not shrink it)."""
+        if c.idx.size <= 1 or c.level >= self.max_levels:
+            return None, None
+        parts = self.order(self.P[c.idx, :self.dims])
+        if max(p.size for p in parts) == c.idx.size:
+            return None, None
+        children, pos = [], c.start
+        for p in parts:
+            children.append(_Cluster(pos, pos + p.size, c.idx[p], c.level + 1, self))
+            pos += p.size
+        return parts, children
 
     def split(self, c):
         """Children of c; a cluster that cannot split yields itself followed
@@ -152,9 +172,9 @@ class _ClusterTree:
         kids = []
         for p in parts:
             if p.size == c.idx.size and c.idx.size:
-                k = _Cluster(c.start, c.end, c.idx, c.level + 1)
+                k = _Cluster(c.start, c.end, c.idx, c.level + 1, self)
             else:
-                k = _Cluster(c.start, c.start, c.idx[:0], c.level + 1)
+                k = _Cluster(c.start, c.start, c.idx[:0], c.level + 1, self)
             kids.append(k)
         return kids, parts
 

@@ -53,6 +53,50 @@ def test_cluster_tree_is_consistent(dims):
     check(ct.root)
 
 
+@pytest.mark.parametrize("dims", [2, 3])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n,kind", [(0, "random"), (1, "random"), (2, "random"), (300, "random"),
+                                    (300, "repeated"), (300, "line"), (40, "nan"), (200, "deep")])
+def test_cluster_order_equals_splitting_one_by_one(n, kind, dtype, dims):
+    import pickle
+
+    from fluxpy_amd.compressed_form_factors import _ClusterTree
+    from fluxpy_amd.octree import get_octant_order
+    from fluxpy_amd.quadtree import get_quadrant_order
+    rng = np.random.default_rng(7)
+    P = rng.normal(size=(n, 3)).astype(dtype)
+    if kind == "repeated":
+        P = P[rng.integers(0, 60, n)]
+    elif kind == "line":
+        P[:, 1] = 0
+    elif kind == "nan":
+        P[1, 0] = np.nan
+    elif kind == "deep":              # more levels than the tree may have
+        P = (2.0 ** -rng.integers(0, 90, (n, 3))).astype(dtype)
+    order = get_quadrant_order if dims == 2 else get_octant_order
+    most = 12
+    perm, levels = [], 0
+
+    def visit(ids, level):
+        nonlocal levels
+        parts = order(P[ids, :dims]) if ids.size > 1 and level < most else [ids]
+        if max(p.size for p in parts) == ids.size:
+            perm.extend(ids)
+            return
+        if max(p.size for p in parts) > 1:
+            levels = max(levels, level + 1)
+        for p in parts:
+            visit(ids[p], level + 1)
+
+    visit(np.arange(n), 0)
+    ct = _ClusterTree(P, dims, most)
+    assert ct.perm.tolist() == perm and ct.levels == levels
+    assert np.array_equal(ct.perm[ct.iperm], np.arange(n))
+    back = pickle.loads(pickle.dumps(ct))
+    assert back.root.children is None or \
+        [c.start for c in back.root.children] == [c.start for c in ct.root.children]
+
+
 def test_byte_rules_match_reference_formulas():
     from fluxpy_amd.compressed_form_factors import _csr_nbytes, _svd_nbytes
     import scipy.sparse
