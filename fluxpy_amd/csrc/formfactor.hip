@@ -263,7 +263,7 @@ __global__ void __launch_bounds__(256, 5) k_ff_mask_rays(
   src.lane = lane;
   src.exhausted = false;
   src.lp = src.lq = 0;
-  trace_wave(S, src, &stack[wv][0][lane]);
+  trace_wave<false>(S, src, &stack[wv][0][lane]);
 }
 
 // The same for all pairs of one list of n facets in CGAL mode, where the
@@ -417,7 +417,7 @@ __global__ void __launch_bounds__(256, 5) k_ff_mask_both(
   src.lane = lane;
   src.exhausted = false;
   src.lp = src.lq = 0;
-  trace_wave(S, src, &stack[wv][0][lane]);
+  trace_wave<false>(S, src, &stack[wv][0][lane]);
 }
 
 // mask and the tile counter set to zero (no memset: callers may capture)

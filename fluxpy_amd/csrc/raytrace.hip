@@ -3,20 +3,31 @@
 
 namespace flux {
 
-template <typename Query>
+template <typename Query, bool kShare>
 __global__ void __launch_bounds__(256, 5) k_query(flux_scene S, Query q, int64_t total,
                                                   int64_t block) {
   __shared__ int stack[4][kStackRows][64];
   IndexSource<Query> src;
   src.init(q, total, block);
-  trace_wave(S, src, &stack[threadIdx.x >> 6][0][threadIdx.x & 63]);
+  trace_wave<kShare>(S, src, &stack[threadIdx.x >> 6][0][threadIdx.x & 63]);
 }
+
+// Queries of up to this many rays share the walks that are left once a wave
+// has handed out its rays: such a query lasts as long as its longest walk
+// and leaves the VALUs idle.  One sun over 10,368 facets: 69 us without
+// sharing, 32 with; over 41,472: 105 and 47.  With 25 rays a wave (124,416)
+// 135 and 94; with 50 (248,832) sharing costs instructions that the chip has
+// no time for (150 and 190).
+constexpr int64_t kShareRays = 131072;
 
 template <typename Query>
 static int launch_query(const flux_scene *scene, const Query &q, int64_t total, hipStream_t st) {
   const int64_t block = trace_block(total);
-  hipLaunchKernelGGL(k_query<Query>, dim3(trace_groups((total + block - 1) / block)), dim3(256),
-                     0, st, *scene, q, total, block);
+  const dim3 grid(trace_groups((total + block - 1) / block));
+  if (total <= kShareRays)
+    hipLaunchKernelGGL((k_query<Query, true>), grid, dim3(256), 0, st, *scene, q, total, block);
+  else
+    hipLaunchKernelGGL((k_query<Query, false>), grid, dim3(256), 0, st, *scene, q, total, block);
   FLUX_LAUNCH_CHECK();
   return 0;
 }

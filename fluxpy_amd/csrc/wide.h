@@ -11,7 +11,9 @@
 //  * each lane is at a node, at a leaf or without work, and every iteration
 //    of the wave runs one of the two steps, for the larger group;
 //  * lanes whose ray has ended take new rays once a quarter of the wave is
-//    out of work, instead of waiting for the longest ray of 64.
+//    out of work, instead of waiting for the longest ray of 64;
+//  * in small queries, which last as long as their longest walk, lanes
+//    without work take deferred children off other lanes' stacks.
 //
 // Decisions do not depend on any of this: the set of triangles tested always
 // contains every triangle the FP64 test hits on the queried segment (the
@@ -38,7 +40,16 @@ constexpr int kStackRows = kWideStack + 3;
 // one node step, whatever the number of lanes it serves.
 constexpr int kRefill = 16;
 
-enum : int { kFlagPair = 1, kFlagReverse = 2, kFlagLost = 4 };
+// Steps between two rounds of sharing, and the lanes without work that one
+// needs (trace_share).  A round costs about as much as a third of a step:
+// one sun over 10,368 facets takes 32 us with a round after every step, 37
+// after two, 55 after four; 33 with 8 lanes and 36 with 32.
+constexpr int kShareSteps = 1;
+constexpr int kShareIdle = 16;
+static_assert(kShareSteps >= 1, "the walk goes on between two rounds");
+
+// kFlagHelper: the lane walks a part of the ray of lane flags >> 8.
+enum : int { kFlagPair = 1, kFlagReverse = 2, kFlagLost = 4, kFlagHelper = 8 };
 
 struct LaneRay {
   Ray64 r;
@@ -296,31 +307,6 @@ __device__ __forceinline__ void lane_recover(const flux_scene &S, LaneRay &L) {
   L.flags &= ~kFlagLost;
 }
 
-// The wave's loop.  src.refill(S, L) ends the rays of done lanes, hands new
-// ones out and returns false once no lane of the wave has one and none are
-// left; src.drained() says that none are left to hand out.
-template <typename Src>
-__device__ __forceinline__ void trace_wave(const flux_scene &S, Src &src, int *stk) {
-  LaneRay L;
-  L.cur = kLaneIdle;
-  L.sp = 0;
-  L.flags = 0;
-  while (true) {
-    const int nn = __popcll(__ballot(L.cur >= 0));
-    const int nl = __popcll(__ballot(L.cur < 0 && L.cur > kLaneDone));
-    if (nn + nl == 0 || (nn + nl <= 64 - kRefill && !src.drained())) {
-      lane_recover(S, L);
-      if (!src.refill(S, L)) break;
-      continue;
-    }
-    if (nn >= nl) {
-      if (L.cur >= 0) lane_node(S, L, stk);
-    } else {
-      if (L.cur < 0 && L.cur > kLaneDone) src.leaf(S, L, stk);
-    }
-  }
-}
-
 // LDS written by some lanes of the wave is read by others (the wave's LDS
 // operations complete in order; this keeps the compiler's order too).
 __device__ __forceinline__ void wave_lds_order() {
@@ -332,6 +318,136 @@ __device__ __forceinline__ void wave_lds_order() {
 __device__ __forceinline__ int lane_rank(uint64_t m) {
   return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
                                         __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+// Helpers that are done, and lanes at a ray that is known to be blocked,
+// hand in what they found: the lane that owns the ray (the one that refill
+// gave it to) takes it over, the helpers are free again.  What several lanes
+// found of a pair's ray adds up like what one lane finds: a blocker of both
+// directions decides both, else any of them may ask for the reverse walk.
+__device__ __forceinline__ void share_report(LaneRay &L, int *stk) {
+  enum : int { kBlocked = 1, kReverse = 2, kBothBlocked = 4 };
+  const int lane = threadIdx.x & 63;
+  int *found = stk - lane + kWideStack * 64;  // rows past the deferred children
+  const bool helper = L.flags & kFlagHelper;
+  const bool done = L.cur <= kLaneDone && L.cur != kLaneIdle && !(L.flags & kFlagLost);
+  int bits = 0;
+  if (done && L.cur == kLaneBlocked)
+    bits = (L.flags & (kFlagPair | kFlagReverse)) == kFlagPair ? kBlocked | kBothBlocked
+                                                               : kBlocked;
+  if (done && (L.flags & kFlagReverse)) bits |= kReverse;
+  found[lane] = helper ? 0 : bits;
+  wave_lds_order();
+  const int own = helper ? L.flags >> 8 : lane;
+  if (helper && bits) atomicOr(&found[own], bits);
+  wave_lds_order();
+  const int all = found[own];
+  if (helper) {
+    if (done || (all & kBlocked)) {
+      L.cur = kLaneIdle;
+      L.flags = 0;
+    }
+  } else if (L.cur != kLaneIdle) {
+    if (all & kBlocked) L.cur = kLaneBlocked;
+    if (L.flags & kFlagPair) {
+      if (all & kBothBlocked)
+        L.flags &= ~kFlagReverse;
+      else if (all & kReverse)
+        L.flags |= kFlagReverse;
+    }
+  }
+  wave_lds_order();
+}
+
+template <typename V>
+__device__ __forceinline__ void take_from(V &v, int lane) {
+  v = __shfl(v, lane);
+}
+
+// Lanes without work take the first deferred child (the largest part left)
+// of lanes that have one, with their rays.
+__device__ __forceinline__ void trace_share(LaneRay &L, int *stk) {
+  share_report(L, stk);
+  const int lane = threadIdx.x & 63;
+  int *donor = stk - lane + kWideStack * 64, *child = donor + 64;
+  const uint64_t idle = __ballot(L.cur == kLaneIdle);
+  const bool can = L.cur > kLaneDone && L.sp > 0;
+  const uint64_t give = __ballot(can);
+  const int count = min(__popcll(idle), __popcll(give));
+  if (count == 0) return;
+  if (can) {
+    const int k = lane_rank(give);
+    if (k < count) {
+      donor[k] = lane;
+      child[k] = stk[0];
+      L.sp -= 64;
+      stk[0] = stk[L.sp];
+    }
+  }
+  wave_lds_order();
+  const int k = lane_rank(idle);
+  const bool take = L.cur == kLaneIdle && k < count;
+  const int from = take ? donor[k] : lane;
+  const int cur = take ? child[k] : L.cur, sp = take ? 0 : L.sp;
+  const int flags = take ? 0 : L.flags;
+  for (int c = 0; c < 3; ++c) {
+    take_from(L.r.o[c], from);
+    take_from(L.inv[c], from);
+    take_from(L.oi[c], from);
+  }
+  take_from(L.r.Sx, from);
+  take_from(L.r.Sy, from);
+  take_from(L.r.Sz, from);
+  take_from(L.r.kx, from);
+  take_from(L.r.ky, from);
+  take_from(L.r.kz, from);
+  take_from(L.oct, from);
+  take_from(L.tlim, from);
+  take_from(L.klim, from);
+  take_from(L.skip1, from);
+  take_from(L.skip2, from);
+  const int f = __shfl(L.flags, from);
+  L.flags = take ? (f & (kFlagPair | kFlagReverse)) | kFlagHelper |
+                       (f & kFlagHelper ? f & ~0xff : from << 8)
+                 : flags;
+  L.cur = cur;
+  L.sp = sp;
+  wave_lds_order();
+}
+
+// The wave's loop.  src.refill(S, L) ends the rays of done lanes, hands new
+// ones out and returns false once no lane of the wave has one and none are
+// left; src.drained() says that none are left to hand out (from then on
+// refill runs only when every lane is done, and so has every helper).
+template <bool kShare, typename Src>
+__device__ __forceinline__ void trace_wave(const flux_scene &S, Src &src, int *stk) {
+  LaneRay L;
+  L.cur = kLaneIdle;
+  L.sp = 0;
+  L.flags = 0;
+  int steps = 0;
+  while (true) {
+    const int nn = __popcll(__ballot(L.cur >= 0));
+    const int nl = __popcll(__ballot(L.cur < 0 && L.cur > kLaneDone));
+    if (nn + nl == 0 || (nn + nl <= 64 - kRefill && !src.drained())) {
+      lane_recover(S, L);
+      if (kShare && __ballot(L.flags & kFlagHelper)) share_report(L, stk);
+      if (!src.refill(S, L)) break;
+      continue;
+    }
+    // no rays left: the ones under way are walked by all lanes (the last
+    // refill of a wave follows when the last lane is done)
+    if (kShare && nn + nl <= 64 - kShareIdle && --steps < 0) {
+      steps = kShareSteps;
+      trace_share(L, stk);
+      continue;
+    }
+    if (nn >= nl) {
+      if (L.cur >= 0) lane_node(S, L, stk);
+    } else {
+      if (L.cur < 0 && L.cur > kLaneDone) src.leaf(S, L, stk);
+    }
+  }
 }
 
 // Rays numbered 0 .. total - 1 for trace_wave: a wave takes blocks of

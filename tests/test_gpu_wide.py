@@ -81,6 +81,32 @@ def test_stack_overflow_matches_oracle(torch_dev, oracle_mod):
     assert np.array_equal(sm.get_visibility(I, I), S.vis_mn(I, I))
 
 
+@pytest.mark.parametrize("mesh", ["soup", "deep", "terrain"])
+def test_small_queries_equal_large_ones(torch_dev, mesh):
+    """Lanes without work take parts of other lanes' walks in queries of up
+    to 131,072 rays only: the same rays in one larger query."""
+    from fluxpy_amd.shape import CgalTrimeshShapeModel
+    if mesh == "soup":
+        V, F = _soup(400, 11)
+    elif mesh == "deep":
+        V, F = deep_mesh()
+    else:
+        V, F = meshes.fractal_terrain(grid=80, levels=6, n_craters=12, seed=4)
+    sm = CgalTrimeshShapeModel(V, F)
+    nf = sm.num_faces
+    I, J = np.arange(nf), np.linspace(0, nf - 1, -(-140000 // nf)).astype(np.int64)
+    assert nf * J.size > 131072 and nf * (J.size // 2) <= 131072
+    full = sm.get_visibility(I, J)
+    for a in np.array_split(np.arange(J.size), 3) + [np.array([J.size - 1])]:
+        assert np.array_equal(sm.get_visibility(I, J[a]), full[:, a])
+    few = I[:: max(1, nf // 50)]
+    assert np.array_equal(sm.get_visibility(few, J), full[few])
+    D = meshes.sun_directions(-(-140000 // nf), seed=2)
+    E = sm.get_direct_irradiance_multi(1.0, D)
+    for k in range(0, D.shape[0], max(1, D.shape[0] // 12)):
+        assert np.array_equal(sm.get_direct_irradiance_multi(1.0, D[k:k + 1])[:, 0], E[:, k])
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("mesh", ["soup", "crater", "terrain", "far", "sheet"])
 def test_square_mask_equals_general_mask(torch_dev, oracle_mod, mesh, dtype):
