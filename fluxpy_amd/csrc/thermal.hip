@@ -4,10 +4,11 @@
 // the explicit radiance update of model.py:44-69 around it.
 //
 // One thread per facet, one wave per workgroup (a facet's solve is a serial
-// recurrence, so the work is spread over as many CUs as there are waves).
+// recurrence, so the work is spread over as many CUs as there are waves),
+// with the profiles in LDS unless there are very many (conduction_lds).
 // Profiles are stored layer-major, T[l * nf + f] for layer l = 0 (surface)
-// .. nz of facet f, so a wave's loads of one layer are contiguous.  The step reads T_in and writes T_out (the caller swaps them),
-// which keeps the previous profile for the predictor-corrector repeats of
+// .. nz of facet f, so a wave's loads of one layer are contiguous.  The step
+// reads T_in and writes T_out (the caller swaps them), which keeps the previous profile for the predictor-corrector repeats of
 // conductionQ and leaves the state untouched when the caller rejects a step.
 //
 // The coefficients depend on z, ti, rhoc and dt only; k_conduction_coef
@@ -135,10 +136,88 @@ __device__ __forceinline__ double conduction_solve(int64_t nf, int64_t f, int nz
   return u;
 }
 
+// The same with the wave's profile in LDS: row l of Uc / Gc holds layer l of
+// u and of the multipliers, 64 facets wide, and Tin is staged into Uc before
+// the elimination overwrites it row by row.  With few waves on the chip the
+// step is bound by latency: in global memory every eighth row waited for its
+// loads and the way back for the stores before it.  Here a row's operands are
+// read one row ahead and a row takes the latency of its division (two chains
+// of 60 for every repeat of the linearisation).  Steps of 10,368 facets with
+// 60 layers: 77 us before, 56 now.  u stays in Uc for the caller to store.
+__device__ __forceinline__ double conduction_solve_lds(
+    int64_t nf, int64_t f, int nz, const double *__restrict__ z, double dt,
+    const double *__restrict__ rhoc, const double *__restrict__ alpha,
+    const double *__restrict__ gamma, double fgeo, double b1, double r1, double T1, double T2,
+    const double *__restrict__ Tin, double *__restrict__ Uc, double *__restrict__ Gc, int &bad) {
+#pragma clang fp contract(off)
+#pragma unroll 20
+  for (int j = 3; j <= nz; ++j) Uc[j * 64] = Tin[(int64_t)j * nf + f];
+  double bet = b1;
+  if (bet == 0.0) bad |= kPivot1;
+  double u = r1 / bet;
+  Uc[64] = u;
+  double tm = T1, tc = T2;
+  double al1 = alpha[1], al = alpha[2], ga = gamma[2];  // rows j - 1 and j
+  double tp = nz > 2 ? Uc[3 * 64] : 0.0;
+#pragma unroll 4
+  for (int j = 2; j < nz; ++j) {
+    // the next row's operands (the last time the bottom row's)
+    const double tn = Uc[min(j + 2, nz) * 64], aln = alpha[j + 1], gan = gamma[j + 1];
+    const double aj = -ga;
+    const double bj = 1. + al + ga;
+    const double rj = ga * tm + (1 - al - ga) * tc + al * tp;
+    tm = tc;
+    tc = tp;
+    const double gam = -al1 / bet;
+    bet = bj - aj * gam;
+    if (bet == 0.0) bad |= kPivot;
+    u = (rj - aj * u) / bet;
+    Gc[j * 64] = gam;
+    Uc[j * 64] = u;
+    al1 = al;
+    al = aln;
+    ga = gan;
+    tp = tn;
+  }
+  {  // bottom row: geothermal flux
+    const double aj = -ga;
+    const double bj = 1. + ga;
+    const double rj = ga * tm + (1. - ga) * tc + dt / rhoc[nz] * fgeo / (z[nz] - z[nz - 1]);
+    const double gam = -al1 / bet;
+    bet = bj - aj * gam;
+    if (bet == 0.0) bad |= kPivot;
+    u = (rj - aj * u) / bet;
+    Gc[nz * 64] = gam;
+    Uc[nz * 64] = u;
+  }
+  if (!isfinite(u)) bad |= kNanT;
+  if (u < 0.0) bad |= kNegT;
+  double g = Gc[nz * 64], v = Uc[(nz - 1) * 64];
+#pragma unroll 4
+  for (int j = nz - 1; j >= 1; --j) {
+    const double gn = Gc[max(j, 2) * 64], vn = Uc[max(j - 1, 1) * 64];
+    u = v - g * u;
+    Uc[j * 64] = u;
+    if (!isfinite(u)) bad |= kNanT;
+    if (u < 0.0) bad |= kNegT;
+    g = gn;
+    v = vn;
+  }
+  return u;
+}
+
+// Stores the solution of a wave from LDS.
+__device__ __forceinline__ void conduction_store(int64_t nf, int64_t f, int nz, const double *Uc,
+                                                 double *__restrict__ Tout) {
+#pragma unroll 8
+  for (int j = 1; j <= nz; ++j) Tout[(int64_t)j * nf + f] = Uc[j * 64];
+}
+
 __device__ __forceinline__ int input_flags(double x) {
   return (isfinite(x) ? 0 : kBadInput) | (x < 0.0 ? kNegInput : 0);
 }
 
+template <bool kLds>
 __global__ __launch_bounds__(64) void k_conduction_q(
     int64_t nf, int nz, const double *__restrict__ z, double dt, const double *__restrict__ Qn,
     const double *__restrict__ Qnp1, const double *__restrict__ Tin, double *__restrict__ Tout,
@@ -148,7 +227,9 @@ __global__ __launch_bounds__(64) void k_conduction_q(
 #pragma clang fp contract(off)
   const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (f >= nf) return;
+  extern __shared__ double cols[];
   const int n1 = nz + 1;
+  double *Uc = cols + threadIdx.x, *Gc = Uc + 64 * n1;
   const double *alpha = coef, *gamma = coef + n1;
   const double kz1 = coef[2 * n1], k1 = coef[2 * n1 + 1];
   const double em = emiss[f], qn = Qn[f], qn1 = Qnp1[f], fg = fgeo[f];
@@ -167,8 +248,10 @@ __global__ __launch_bounds__(64) void k_conduction_q(
     const double r1 = gamma[1] * (annp1 + ann) +
                       (1. - alpha[1] - gamma[1] + gamma[1] * bn) * T1 + alpha[1] * T2;
     int bad = 0;
-    u1 = conduction_solve(nf, f, nz, z, dt, rhoc, alpha, gamma, fg, b1, r1, Tin, Tout, gamw,
-                          bad);
+    u1 = kLds ? conduction_solve_lds(nf, f, nz, z, dt, rhoc, alpha, gamma, fg, b1, r1, T1, T2,
+                                     Tin, Uc, Gc, bad)
+              : conduction_solve(nf, f, nz, z, dt, rhoc, alpha, gamma, fg, b1, r1, Tin, Tout,
+                                 gamw, bad);
     T0 = 0.5 * (annp1 + bn * u1 + u1);
     if ((T0 > 1.2 * Tr || T0 < 0.8 * Tr) && iter < 10) {
       ++iter;
@@ -178,6 +261,7 @@ __global__ __launch_bounds__(64) void k_conduction_q(
     flags |= bad;
     break;
   }
+  if (kLds) conduction_store(nf, f, nz, Uc, Tout);
   if (!isfinite(T0)) flags |= kNanT;
   if (T0 < 0.0) flags |= kNegT;
   Tout[f] = T0;
@@ -186,6 +270,7 @@ __global__ __launch_bounds__(64) void k_conduction_q(
   if (iter >= 9) atomicAdd(status + 1, 1);
 }
 
+template <bool kLds>
 __global__ __launch_bounds__(64) void k_conduction_t(
     int64_t nf, int nz, const double *__restrict__ z, double dt, const double *__restrict__ Tin,
     double *__restrict__ Tout, const double *__restrict__ Tsurf,
@@ -195,7 +280,9 @@ __global__ __launch_bounds__(64) void k_conduction_t(
 #pragma clang fp contract(off)
   const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (f >= nf) return;
+  extern __shared__ double cols[];
   const int n1 = nz + 1;
+  double *Uc = cols + threadIdx.x, *Gc = Uc + 64 * n1;
   const double *alpha = coef, *gamma = coef + n1;
   const double kz1 = coef[2 * n1];
   const double ts = Tsurf[f], ts1 = Tsurfp1[f];
@@ -205,8 +292,11 @@ __global__ __launch_bounds__(64) void k_conduction_t(
   const double r1 = alpha[1] * T2 + (1. - alpha[1] - gamma[1]) * T1 + gamma[1] * (ts + ts1);
   int bad = 0;
   const double u1 =
-      conduction_solve(nf, f, nz, z, dt, rhoc, alpha, gamma, fgeo[f], b1, r1, Tin, Tout, gamw,
-                       bad);
+      kLds ? conduction_solve_lds(nf, f, nz, z, dt, rhoc, alpha, gamma, fgeo[f], b1, r1, T1, T2,
+                                  Tin, Uc, Gc, bad)
+           : conduction_solve(nf, f, nz, z, dt, rhoc, alpha, gamma, fgeo[f], b1, r1, Tin, Tout,
+                              gamw, bad);
+  if (kLds) conduction_store(nf, f, nz, Uc, Tout);
   flags |= bad;
   // conductionT leaves T[0] as it was
   if (!isfinite(T0)) flags |= kNanT;
@@ -286,6 +376,20 @@ static double *conduction_coef(int64_t nf, int nz, void *work, double **gamw) {
   return static_cast<double *>(work);
 }
 
+// LDS of a wave's profiles and multipliers, or 0 where the step works in
+// global memory: layers that need more than a CU has, and more waves than
+// one and a half times what the chip holds at once (their number of rounds
+// then counts, not the latency of one).  60 layers, LDS / global: 450 facets
+// 40 / 58 us, 10,368 41 / 47, 41,472 82 / 107, 300,000 467 / 341; 20 layers:
+// 10,368 38 / 45; 110 layers: 10,368 95 / 128, 41,472 289 / 250.
+constexpr int64_t kLdsBytes = 160 * 1024;
+constexpr int64_t kCus = 256;
+
+static size_t conduction_lds(int64_t nf, int nz) {
+  const int64_t b = (int64_t)(nz + 1) * 2 * 64 * 8, waves = (nf + 63) / 64;
+  return b <= kLdsBytes && 2 * waves <= 3 * kCus * (kLdsBytes / b) ? (size_t)b : 0;
+}
+
 extern "C" int flux_conduction_q(int64_t nf, int nz, const double *z, double dt,
                                  const double *Qn, const double *Qnp1, const double *T_in,
                                  double *T_out, const double *ti, const double *rhoc,
@@ -300,8 +404,10 @@ extern "C" int flux_conduction_q(int64_t nf, int nz, const double *z, double dt,
   hipStream_t st = as_stream(stream);
   hipLaunchKernelGGL(k_conduction_coef, dim3(1), dim3(256), 0, st, nz, z, dt, ti, rhoc, 1, coef,
                      status);
-  hipLaunchKernelGGL(k_conduction_q, dim3(ceil_div_u(nf, 64)), dim3(64), 0, st, nf, nz, z, dt,
-                     Qn, Qnp1, T_in, T_out, rhoc, emiss, Fgeotherm, coef, Fsurf, gamw, status);
+  const size_t lds = conduction_lds(nf, nz);
+  hipLaunchKernelGGL(lds ? k_conduction_q<true> : k_conduction_q<false>,
+                     dim3(ceil_div_u(nf, 64)), dim3(64), lds, st, nf, nz, z, dt, Qn, Qnp1, T_in,
+                     T_out, rhoc, emiss, Fgeotherm, coef, Fsurf, gamw, status);
   FLUX_LAUNCH_CHECK();
   return 0;
 }
@@ -320,8 +426,10 @@ extern "C" int flux_conduction_t(int64_t nf, int nz, const double *z, double dt,
   hipStream_t st = as_stream(stream);
   hipLaunchKernelGGL(k_conduction_coef, dim3(1), dim3(256), 0, st, nz, z, dt, ti, rhoc, 0, coef,
                      status);
-  hipLaunchKernelGGL(k_conduction_t, dim3(ceil_div_u(nf, 64)), dim3(64), 0, st, nf, nz, z, dt,
-                     T_in, T_out, Tsurf, Tsurfp1, rhoc, Fgeotherm, coef, Fsurf, gamw, status);
+  const size_t lds = conduction_lds(nf, nz);
+  hipLaunchKernelGGL(lds ? k_conduction_t<true> : k_conduction_t<false>,
+                     dim3(ceil_div_u(nf, 64)), dim3(64), lds, st, nf, nz, z, dt, T_in, T_out,
+                     Tsurf, Tsurfp1, rhoc, Fgeotherm, coef, Fsurf, gamw, status);
   FLUX_LAUNCH_CHECK();
   return 0;
 }

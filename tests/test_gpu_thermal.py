@@ -65,6 +65,43 @@ def test_conduction_q_matches_oracle(torch_dev, oracle_mod):
     assert model.current_time == 6 * 20000.
 
 
+@pytest.mark.parametrize("bcond", ["Q", "T"])
+@pytest.mark.parametrize("nz", [2, 3, 4, 21, 158, 159, 160, 171])
+def test_steps_in_lds_and_in_global_memory(torch_dev, oracle_mod, nz, bcond):
+    """Profiles in LDS (up to 159 layers, few facets) and in global memory:
+    both against the oracle, and the same facets among very many others."""
+    # 2000 s: with 158 thin layers the oracle itself turns nonfinite in steps
+    # of 20,000 s under these jumps of the flux
+    nf, steps, dt = 70, 3, 2000.
+    rng, z, T, ti, rhoc, em, fg, Qn = _state(9, nf=nf, nz=max(nz, 6))
+    z, T, ti, rhoc = z[:nz + 1], np.ascontiguousarray(T[:, :nz + 1]), ti[:nz + 1], rhoc[:nz + 1]
+    X = [rng.uniform(0, 1500, nf) if bcond == "Q" else rng.uniform(150, 350, nf)
+         for _ in range(steps)]
+
+    def run(rep):
+        model = PccThermalModel1D(z, np.tile(T, (rep, 1)), ti, rhoc, np.tile(em, rep),
+                                  np.tile(fg, rep), np.tile(Qn, rep), np.tile(T[:, 0], rep),
+                                  bcond=bcond)
+        for x in X:
+            model.step(dt, np.tile(x, rep))
+        return model.T, model.Fsurf
+
+    Tg, Fg = run(1)
+    To, prev = T.copy(), Qn if bcond == "Q" else T[:, 0].copy()
+    for x in X:
+        if bcond == "Q":
+            oracle_mod.conduction_q(z, dt, prev, x, To, ti, rhoc, em, fg)
+        else:
+            oracle_mod.conduction_t(z, dt, To, prev, x, ti, rhoc, fg)
+        prev = x
+    assert _max_rel(Tg, To) <= 1e-14
+    if 2 * nz > 159:                           # 384 waves: more than LDS has room for
+        rep = 384 * 64 // nf + 2
+        Tm, Fm = run(rep)
+        assert np.array_equal(Tm, np.tile(Tg, (rep, 1)))
+        assert np.array_equal(Fm, np.tile(Fg, rep))
+
+
 def test_conduction_t_matches_oracle(torch_dev, oracle_mod):
     rng, z, T, ti, rhoc, em, fg, _ = _state(6, nf=777, nz=33)
     print("case: conduction_t, 777 facets, 33 layers, 5 steps", flush=True)
