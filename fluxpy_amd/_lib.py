@@ -56,6 +56,8 @@ SIGNATURES = {
                                       _c_dbl, _c_int, _vp, _c_int, _vp, _vp]),
     "flux_csr_transpose": (_c_int, [_c_i64, _c_i64, _vp, _vp, _vp, _c_int, _vp, _vp, _vp,
                                     _vp]),
+    "flux_direct_irradiance_sun": (_c_int, [_vp, _vp, _vp, _c_int, _vp, _c_dbl, _c_int, _vp,
+                                            _vp]),
     "flux_direct_irradiance":(_c_int, [_vp, _vp, _vp, _c_int, _vp, _c_i64, _c_dbl, _c_int,
                                         _vp, _vp]),
     "flux_block_stats": (_c_int, [_vp, _vp, _c_i64, _vp, _vp, _vp, _vp]),

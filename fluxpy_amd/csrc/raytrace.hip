@@ -114,20 +114,27 @@ struct OccQuery {
 template <typename T>
 struct IrradianceQuery {
   const T *Nrm, *P;
-  const double *D;
+  const double *D;  // NULL: the one direction `sun`
   int64_t M;
   double F0;
   int mode;
   T *E;
+  double sun[3];
+
+  __device__ __forceinline__ void direction(int64_t k, double d[3]) const {
+    for (int c = 0; c < 3; ++c) d[c] = D ? D[k * 3 + c] : sun[c];
+  }
 
   __device__ __forceinline__ void begin(const flux_scene &S, LaneRay &L, int64_t r) const {
     const int64_t k = r / S.nf;
-    sun_begin(S, L, S.order[r - k * S.nf], D + k * 3, mode, P, Nrm);
+    double d[3];
+    direction(k, d);
+    sun_begin(S, L, S.order[r - k * S.nf], d, mode, P, Nrm);
   }
   __device__ __forceinline__ void end(const flux_scene &S, int64_t r, bool blocked) const {
     const int64_t k = r / S.nf, f = S.order[r - k * S.nf];
-    const double *d = D + k * 3;
-    double nf3[3];
+    double d[3], nf3[3];
+    direction(k, d);
     load3(Nrm, f, nf3);
     const double cosi = (nf3[0] * d[0] + nf3[1] * d[1]) + nf3[2] * d[2];
     E[f * M + k] = blocked ? (T)0 : (T)(F0 * (cosi > 0.0 ? cosi : 0.0));
@@ -155,9 +162,9 @@ __global__ void k_intersect1(flux_scene S, const double *__restrict__ x,
 
 using namespace flux;
 
-extern "C" int flux_direct_irradiance(const flux_scene *scene, const void *P, const void *Nrm,
-                                      int dtype, const double *D, int64_t M, double F0,
-                                      int mode, void *E, void *stream) {
+static int direct_irradiance(const flux_scene *scene, const void *P, const void *Nrm, int dtype,
+                             const double *D, const double *sun, int64_t M, double F0, int mode,
+                             void *E, void *stream) {
   FLUX_CHECK(scene != nullptr, "flux_direct_irradiance: NULL scene");
   FLUX_CHECK(M >= 0, "flux_direct_irradiance: negative M");
   FLUX_CHECK(dtype == FLUX_F32 || dtype == FLUX_F64, "flux_direct_irradiance: bad dtype");
@@ -165,18 +172,33 @@ extern "C" int flux_direct_irradiance(const flux_scene *scene, const void *P, co
              "flux_direct_irradiance: bad mode");
   const int64_t total = scene->nf * M;
   if (total == 0) return 0;
-  FLUX_CHECK(Nrm && D && E && (mode == FLUX_MODE_CGAL || P),
+  FLUX_CHECK(Nrm && (D || sun) && E && (mode == FLUX_MODE_CGAL || P),
              "flux_direct_irradiance: NULL array");
   hipStream_t st = as_stream(stream);
+  const double s[3] = {sun ? sun[0] : 0.0, sun ? sun[1] : 0.0, sun ? sun[2] : 0.0};
   if (dtype == FLUX_F64)
     return launch_query(scene,
                         IrradianceQuery<double>{(const double *)Nrm, (const double *)P, D, M, F0,
-                                                mode, (double *)E},
+                                                mode, (double *)E, {s[0], s[1], s[2]}},
                         total, st);
   return launch_query(scene,
                       IrradianceQuery<float>{(const float *)Nrm, (const float *)P, D, M, F0, mode,
-                                             (float *)E},
+                                             (float *)E, {s[0], s[1], s[2]}},
                       total, st);
+}
+
+extern "C" int flux_direct_irradiance(const flux_scene *scene, const void *P, const void *Nrm,
+                                      int dtype, const double *D, int64_t M, double F0,
+                                      int mode, void *E, void *stream) {
+  return direct_irradiance(scene, P, Nrm, dtype, D, nullptr, M, F0, mode, E, stream);
+}
+
+// The direction travels with the launch: the copy of 24 bytes that a time
+// step started with held the host for 15 us and the GPU idle for about 35.
+extern "C" int flux_direct_irradiance_sun(const flux_scene *scene, const void *P, const void *Nrm,
+                                          int dtype, const double *sun, double F0, int mode,
+                                          void *E, void *stream) {
+  return direct_irradiance(scene, P, Nrm, dtype, nullptr, sun, 1, F0, mode, E, stream);
 }
 
 extern "C" int flux_vis_mn(const flux_scene *scene, const int64_t *I, int64_t m,

@@ -123,6 +123,11 @@ int flux_direct_irradiance(const flux_scene *scene, const void *P,
                            const void *Nrm, int dtype, const double *D,
                            int64_t M, double F0, int mode, void *E,
                            void *stream);
+/* The same for one direction, 3 doubles on the host, read before the call
+ * returns. */
+int flux_direct_irradiance_sun(const flux_scene *scene, const void *P,
+                               const void *Nrm, int dtype, const double *sun,
+                               double F0, int mode, void *E, void *stream);
 
 /* Closest hit of n_rays rays x + t d (t >= 0), nothing skipped.  Replaces
  * cgal_aabb_intersect1 (aabb_wrapper.cpp:110-129).  hit_index[k] = -1 when

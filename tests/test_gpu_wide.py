@@ -145,3 +145,22 @@ def test_square_mask_equals_general_mask(torch_dev, oracle_mod, mesh, dtype):
     sub = rng.integers(0, nf, max(1, nf // 3))                # a list with repeats
     assert (get_form_factor_matrix(sm, sub, sub).toarray()
             == full.toarray()[np.ix_(sub, sub)]).all()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("cls", ["cgal", "embree"])
+def test_one_sun_by_value(torch_dev, cls, dtype):
+    """The direction as an argument of the launch and as a device array."""
+    from fluxpy_amd import _lib
+    from fluxpy_amd.shape import CgalTrimeshShapeModel, EmbreeTrimeshShapeModel
+    V, F = meshes.fractal_terrain(grid=20, levels=5, n_craters=6, seed=8)
+    sm = (CgalTrimeshShapeModel if cls == "cgal" else EmbreeTrimeshShapeModel)(V.astype(dtype), F)
+    for d in np.concatenate([meshes.sun_directions(3, seed=5), -np.eye(3)[2:]]):
+        want = sm.get_direct_irradiance_multi(1365.0, d[None])[:, 0]
+        P, N = _lib.to_dev(sm.P), _lib.to_dev(sm.N)
+        E = torch_dev.empty(sm.num_faces, dtype=_lib.torch_dtype(sm.dtype), device="cuda")
+        d = np.ascontiguousarray(d)
+        _lib.call("flux_direct_irradiance_sun", sm._scene.handle, P.data_ptr(), N.data_ptr(),
+                  _lib.dtype_code(sm.dtype), d.ctypes.data, 1365.0, sm._mode, E.data_ptr(),
+                  _lib.stream())
+        assert np.array_equal(E.cpu().numpy(), want)
