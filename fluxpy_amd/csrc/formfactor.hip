@@ -77,16 +77,7 @@ __global__ void __launch_bounds__(256) k_ff_candidates(int64_t nf, const T *__re
   }
 }
 
-// Rays of the pairs (p, q) of m x n positions for trace_wave (wide.h).  A
-// wave takes tiles of one row p and up to 64 words of 64 columns each,
-// evaluates the prefilter 64 columns at a time and keeps the pairs that
-// need a ray in a small queue in LDS, from which lanes out of work are
-// served (the prefilter keeps ~1/4 of the pairs on terrain).  A visible
-// pair sets its bit in the zeroed mask.  Lanes of a wave may work on
-// different rows, so no lane waits for the end of a row: with one wave per
-// row and batches of 64 rays, a row of a small mesh was a serial chain of
-// batches (1131 us for 1,922 facets) and every batch waited for its longest
-// ray.
+// Candidate pairs a wave keeps in LDS.
 constexpr int kPairQueue = 128;  // < 64 left over + one word of 64
 
 // The tiles of a wave.  Large problems draw them from a counter, one atomic
@@ -138,8 +129,9 @@ static inline int64_t tile_width(int64_t words) {
 // one wave per row and batches of 64 rays, a row of a small mesh was a
 // serial chain of batches and every batch waited for its longest ray.
 // Binary walks in such batches took 404 ms for the 41,472-facet terrain
-// (seed 5) and 1131 us for a 1,922-facet crater; this takes 90.7 ms and
-// 214 us.  It is bound by VALU issue (99 % busy, 52 % of lanes active).
+// (seed 5) and 1131 us for a 1,922-facet crater; this took 90.7 ms and
+// 214 us before the node step was shortened by a third (wide.h).  It is bound
+// by VALU issue (98 % busy, 62 % of lanes active).
 template <typename T>
 struct PairSource {
   const T *P, *N;
@@ -270,7 +262,10 @@ __global__ void __launch_bounds__(256, 5) k_ff_mask_rays(
 // rays i -> j and j -> i run along one line: one walk decides both unless
 // rounding may (wide.h), so the pairs s < t are walked once.  The list is
 // taken in Morton order of the facets (I == NULL: facet ids) or in its own
-// order (cluster order elsewhere).
+// order (cluster order elsewhere).  41,472-facet terrain, assembled with a
+// walk per direction 131 ms, with one 65.5, with the shorter node step 48.8;
+// a 1,922-facet crater, whose waves have about one batch of rays each, 407,
+// 412 and 352 us.  Bound by VALU issue like the above.
 template <typename T>
 struct BothSource {
   const T *P, *N;
