@@ -378,16 +378,18 @@ static double *conduction_coef(int64_t nf, int nz, void *work, double **gamw) {
 
 // LDS of a wave's profiles and multipliers, or 0 where the step works in
 // global memory: layers that need more than a CU has, and more waves than
-// one and a half times what the chip holds at once (their number of rounds
-// then counts, not the latency of one).  60 layers, LDS / global: 450 facets
-// 40 / 58 us, 10,368 41 / 47, 41,472 82 / 107, 300,000 467 / 341; 20 layers:
-// 10,368 38 / 45; 110 layers: 10,368 95 / 128, 41,472 289 / 250.
+// the chip holds at once (then the rounds count, not the latency of one).
+// 60 layers and fluxes that jump, LDS / global: 450 facets 40 / 58 us,
+// 10,368 41 / 47; 20 layers: 10,368 38 / 45; 110 layers: 10,368 95 / 128.
+// 41,472 facets with 60 layers, a quarter more waves than fit, take 82 / 107
+// us where the linearisation repeats and 50 / 44 where it does not; 300,000
+// take 467 / 341.
 constexpr int64_t kLdsBytes = 160 * 1024;
 constexpr int64_t kCus = 256;
 
 static size_t conduction_lds(int64_t nf, int nz) {
   const int64_t b = (int64_t)(nz + 1) * 2 * 64 * 8, waves = (nf + 63) / 64;
-  return b <= kLdsBytes && 2 * waves <= 3 * kCus * (kLdsBytes / b) ? (size_t)b : 0;
+  return b <= kLdsBytes && waves <= kCus * (kLdsBytes / b) ? (size_t)b : 0;
 }
 
 extern "C" int flux_conduction_q(int64_t nf, int nz, const double *z, double dt,

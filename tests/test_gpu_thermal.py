@@ -95,8 +95,8 @@ def test_steps_in_lds_and_in_global_memory(torch_dev, oracle_mod, nz, bcond):
             oracle_mod.conduction_t(z, dt, To, prev, x, ti, rhoc, fg)
         prev = x
     assert _max_rel(Tg, To) <= 1e-14
-    if 2 * nz > 159:                           # 384 waves: more than LDS has room for
-        rep = 384 * 64 // nf + 2
+    if 2 * nz > 159:                           # over 256 waves, of which LDS has room
+        rep = 256 * 64 // nf + 2
         Tm, Fm = run(rep)
         assert np.array_equal(Tm, np.tile(Tg, (rep, 1)))
         assert np.array_equal(Fm, np.tile(Fg, rep))
