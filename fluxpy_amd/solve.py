@@ -324,6 +324,8 @@ def _gmres(op, E, rho, left, rtol, maxiter, restart, x0):
     out_dtype = E.dtype
     E = E.to(t.float64).contiguous()
     f64 = t.float64
+    if isinstance(rho, t.Tensor):
+        rho = rho.to(f64)        # it comes in E's dtype
     vo = _kernels.VecOps(k)
     X = (t.zeros_like(E) if x0 is None
          else _lib.to_dev(x0).reshape(n, k).to(f64).contiguous().clone())

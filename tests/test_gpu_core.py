@@ -404,6 +404,26 @@ def test_gmres_restarts_against_dense(torch_dev, oracle_mod, crater, restart):
     assert B3.dtype == np.float32 and abs(B3 - Bd).max() <= 1e-5 * abs(Bd).max()
 
 
+@pytest.mark.parametrize("place", ["right", "left"])
+def test_gmres_fp32_vectors_and_albedo_per_facet(torch_dev, oracle_mod, crater, place):
+    """FP32 input with an albedo per facet: the albedo comes in FP32 and the
+    solver's vectors are FP64.  Bound: the stopping rule (1e-6 of |E_c|) and
+    FP32 rounding of E, rho and the result, as for a scalar albedo above."""
+    from fluxpy_amd.form_factors import FormFactorMatrix
+    from fluxpy_amd.solve import solve_radiosity
+    V, F = crater
+    sm = _model(V, F)
+    Fm = FormFactorMatrix.from_shape_model(sm)
+    rng = np.random.default_rng(4)
+    rho = rng.uniform(0.1, 0.7, sm.num_faces).astype(np.float32)
+    E = sm.get_direct_irradiance_multi(1365.0, meshes.sun_directions(2, seed=8)).astype(np.float32)
+    E64, r64, A = E.astype(np.float64), rho.astype(np.float64), Fm.tocsr().toarray()
+    K = np.eye(len(r64)) - (A * r64 if place == "right" else r64[:, None] * A)
+    want = np.linalg.solve(K, E64)
+    B, _ = solve_radiosity(Fm, E, rho, place, method="gmres", tol=1e-6)
+    assert B.dtype == np.float32 and abs(B - want).max() <= 1e-5 * abs(want).max()
+
+
 def test_steady_state_temperature(torch_dev, oracle_mod, crater):
     from fluxpy_amd.form_factors import FormFactorMatrix
     from fluxpy_amd.model import compute_steady_state_temp
