@@ -287,8 +287,10 @@ __device__ __forceinline__ void both_leaf(const flux_scene &S, LaneRay &L, const
     lane_pop(L, stk);
 }
 
-// A walk that ran out of stack has skipped children: repeat it on the
-// stackless layout unless it found a blocker anyway.
+// A walk that ran out of stack has skipped children: once it has ended,
+// repeat it on the stackless layout unless it found a blocker anyway.  Rays
+// are handed out while other lanes walk: those keep their mark, and the
+// lanes that take new rays have none.
 __device__ __forceinline__ void lane_recover(const flux_scene &S, LaneRay &L) {
   if (L.cur == kLaneVisible && (L.flags & kFlagLost)) {
     // the ray's box test again, from the shears
@@ -304,7 +306,7 @@ __device__ __forceinline__ void lane_recover(const flux_scene &S, LaneRay &L) {
     if (any_blocker(S, L.r, rb, L.tlim, L.klim, L.skip1, L.skip2)) L.cur = kLaneBlocked;
     if (L.flags & kFlagPair) L.flags |= kFlagReverse;
   }
-  L.flags &= ~kFlagLost;
+  if (L.cur <= kLaneDone) L.flags &= ~kFlagLost;
 }
 
 // LDS written by some lanes of the wave is read by others (the wave's LDS
