@@ -219,6 +219,8 @@ def _jacobi_runs(csr, E, rho, left, tol, maxiter):
     maxima's rate of decrease predicts."""
     t = _lib.torch()
     n, k = E.shape
+    if n == 0 or k == 0:        # no change to wait for
+        return E.clone(), 1
     f64 = t.float64
     if isinstance(tol, t.Tensor):
         tol_d = tol.to(f64)

@@ -122,3 +122,19 @@ def test_runs_equal_single_steps(adt, xdt, k, placement):
             assert niter == it
             d = (got - want).abs().max() / want.abs().max()
             assert d <= 30 * eps, (tol, maxiter, float(d))
+
+
+def test_jacobi_of_no_columns_and_no_rows():
+    """An empty batch with a tolerance of its own converges at once."""
+    import torch
+    from fluxpy_amd import _kernels
+    from fluxpy_amd.solve import _jacobi_runs, solve_radiosity
+    torch.cuda.set_device(0)
+    A = scipy.sparse.csr_matrix(np.diag([0.1, 0.2, 0.3]))
+    for E in (np.zeros((3, 0)), torch.zeros((3, 0), dtype=torch.float32, device="cuda")):
+        B, niter = solve_radiosity(A, E, 0.3, tol=1e-6)
+        assert B.shape == (3, 0) and B.dtype == E.dtype and niter == 1
+    E = torch.zeros((0, 4), dtype=torch.float64, device="cuda")
+    csr = _kernels.DeviceCSR.from_scipy(scipy.sparse.csr_matrix((0, 0)))
+    B, niter = _jacobi_runs(csr, E, 0.3, False, 1e-6, 100)
+    assert B.shape == (0, 4) and niter == 1
