@@ -178,8 +178,8 @@ def _run_csr(op):
 
 def _jacobi(op, E, rho, left, tol, maxiter):
     """solve.py:25-45, fused into one kernel per iteration for CSR operators.
-    ``tol``: a scalar, one value per column, or a device vector of either
-    (operators with a ``_run_csr`` only)."""
+    ``tol``: a scalar or one value per column; a device tensor of either for
+    operators with a ``_run_csr`` only."""
     t = _lib.torch()
     k = E.shape[1]
     csr = _run_csr(op)
@@ -208,6 +208,20 @@ def _warn_jacobi(maxiter, d):
                   f"(max |B1 - B| = {d.max():.3e} > tol)", RuntimeWarning)
 
 
+def _tol_device(tol, k, device):
+    """The tolerance of k columns, or of each, as one vector on the device."""
+    t = _lib.torch()
+    if not isinstance(tol, t.Tensor):
+        tol = np.array(tol, dtype=np.float64)
+        # a number travels with a fill, not with a copy from the host
+        tol = t.full((1,), float(tol), dtype=t.float64, device=device) if tol.ndim == 0 \
+            else t.from_numpy(tol)
+    if tol.shape not in ((), (1,), (k,)):
+        raise ValueError(f"tol must be a scalar or have {k} entries (got shape "
+                         f"{tuple(tol.shape)})")
+    return tol.to(device=device, dtype=t.float64).reshape(-1).contiguous()
+
+
 JACOBI_RUN = (6, 24)    # iterations of the first run, and at most in any
 
 
@@ -222,13 +236,7 @@ def _jacobi_runs(csr, E, rho, left, tol, maxiter):
     if n == 0 or k == 0:        # no change to wait for
         return E.clone(), 1
     f64 = t.float64
-    if isinstance(tol, t.Tensor):
-        tol_d = tol.to(f64)
-    elif np.ndim(tol) == 0 or np.size(tol) == 1:
-        tol_d = t.full((1,), float(np.asarray(tol).reshape(())), dtype=f64, device=E.device)
-    else:
-        tol_d = _lib.to_dev(np.ascontiguousarray(
-            np.broadcast_to(np.asarray(tol, dtype=np.float64), (k,))))
+    tol_d = _tol_device(tol, k, E.device)
     rho_t, rho_s = (rho, 0.0) if isinstance(rho, t.Tensor) else (None, float(rho))
     B, B1 = E.clone(), t.empty_like(E)
     X = X1 = None

@@ -138,3 +138,25 @@ def test_jacobi_of_no_columns_and_no_rows():
     csr = _kernels.DeviceCSR.from_scipy(scipy.sparse.csr_matrix((0, 0)))
     B, niter = _jacobi_runs(csr, E, 0.3, False, 1e-6, 100)
     assert B.shape == (0, 4) and niter == 1
+
+
+def test_tolerance_tensors_on_host_and_device():
+    """The tolerance may be a tensor on either side, and a strided one."""
+    import torch
+    from fluxpy_amd.solve import solve_radiosity
+    torch.cuda.set_device(0)
+    A = scipy.sparse.random(300, 300, 0.2, "csr", random_state=1)
+    A.data *= 0.9 / A.sum(1).max()
+    E = np.random.default_rng(2).uniform(0, 1, (300, 3))
+    cols = np.array([1e-3, 1e-9, 1e-6])
+    want, it = solve_radiosity(A, E, 0.5, tol=cols)
+    wide = torch.full((3, 4), 7.0, dtype=torch.float64)
+    wide[:, 1] = torch.from_numpy(cols)
+    for tol in (wide[:, 1], wide.cuda()[:, 1], torch.from_numpy(cols)):
+        got, niter = solve_radiosity(A, E, 0.5, tol=tol)
+        assert niter == it and np.array_equal(got, want)
+    want, it = solve_radiosity(A, E, 0.5, tol=1e-9)
+    for tol in (torch.tensor(1e-9, dtype=torch.float64),
+                torch.tensor([1e-9], dtype=torch.float64).expand(3)):
+        got, niter = solve_radiosity(A, E, 0.5, tol=tol)
+        assert niter == it and np.array_equal(got, want)

@@ -371,3 +371,88 @@ def test_morton_order_is_z_order():
     order = morton_order(g)
     assert [tuple(g[i].astype(int)) for i in order[:4]] == [(0, 0), (1, 0), (0, 1), (1, 1)]
     assert morton_order(np.zeros((5, 2))).tolist() == [0, 1, 2, 3, 4]
+
+
+@pytest.fixture
+def host_jacobi(monkeypatch):
+    """_jacobi_runs on the CPU: flux_csr_jacobi_run for FP64 and a scalar
+    albedo in NumPy, on the memory that the arguments point to."""
+    import ctypes
+    import types
+
+    import scipy.sparse
+    import torch
+
+    from fluxpy_amd import _lib, solve
+
+    def at(ptr, n, typ=ctypes.c_double):
+        return np.ctypeslib.as_array(ctypes.cast(ptr, ctypes.POINTER(typ)), (n,))
+
+    def call(name, n, ip, ix, data, dt, E, B0, B1, X0, X1, k, rho, rho_s, left, xdt, tol, ncol,
+             first, nsteps, slots, colmax, stream):
+        assert name == "flux_csr_jacobi_run" and X0 is None and rho is None and ncol in (1, k)
+        assert type(first) is int and type(nsteps) is int and nsteps >= 1
+        ip = at(ip, n + 1, ctypes.c_int64)
+        F = scipy.sparse.csr_matrix((at(data, ip[-1]), at(ix, ip[-1], ctypes.c_int32), ip), (n, n))
+        row = -(-k // 32) * 32
+        cm = at(colmax, nsteps * slots * row).reshape(nsteps, slots, row)
+        cm[:] = 0.0
+        B = [at(p, n * k).reshape(n, k) for p in (B0, B1)]
+        for s in range(nsteps):
+            if s and (cm[s - 1, :, :k].max(0) <= at(tol, ncol)).all():
+                continue
+            b, b1 = B[(first + s) % 2], B[(first + s + 1) % 2]
+            b1[:] = at(E, n * k).reshape(n, k) + rho_s * (F @ b)
+            cm[s, 0, :k] = np.abs(b1 - b).max(0)
+
+    monkeypatch.setattr(_lib, "call", call)
+    monkeypatch.setattr(_lib, "stream", lambda: None)
+    monkeypatch.setattr(_lib, "to_dev", torch.from_numpy)
+    rng = np.random.default_rng(0)
+    n, k, rho = 40, 3, 0.5
+    A = scipy.sparse.csr_matrix(rng.uniform(0, 1, (n, n)) * (rng.uniform(0, 1, (n, n)) < 0.3))
+    A = (A * (0.9 / A.sum(1).max())).tocsr()
+    csr = types.SimpleNamespace(indptr=torch.from_numpy(A.indptr.astype(np.int64)),
+                                indices=torch.from_numpy(A.indices.astype(np.int32)),
+                                data=torch.from_numpy(A.data))
+    E = rng.uniform(0, 1, (n, k)) * [1.0, 2.0, 4.0]
+
+    def loop(tol, maxiter):
+        """solve.py:25-45"""
+        B, it = E.copy(), 0
+        while True:
+            it += 1
+            B1 = E + rho * (A @ B)
+            if (np.abs(B1 - B).max(0) <= tol).all() or it >= maxiter:
+                return B, it
+            B = B1
+
+    def runs(tol, maxiter):
+        B, it = solve._jacobi_runs(csr, torch.from_numpy(E), rho, False, tol, maxiter)
+        return B.numpy(), it
+
+    return types.SimpleNamespace(loop=loop, runs=runs, k=k)
+
+
+def test_jacobi_tolerances(host_jacobi):
+    """One tolerance or one per column, as a number, a list, an array or a
+    tensor, whatever its strides and type; other shapes are refused."""
+    import torch
+    h = host_jacobi
+    cols = np.array([1e-3, 1e-9, 1e-6])
+    wide = torch.full((3, 4), 7.0, dtype=torch.float64)
+    wide[:, 1] = torch.from_numpy(cols)
+    forms = [(c, 1e-6) for c in (1e-6, np.float32(1e-6), [1e-6], np.array(1e-6),
+                                 torch.tensor(1e-6, dtype=torch.float64),
+                                 torch.tensor([1e-6], dtype=torch.float64).expand(h.k))]
+    forms += [(c, cols) for c in (cols, cols.tolist(), np.repeat(cols, 2)[::2], wide[:, 1])]
+    f32 = torch.from_numpy(cols).float()
+    forms.append((f32, f32.double().numpy()))
+    for tol, plain in forms:
+        want, it = h.loop(np.float64(plain), 1000)
+        got, niter = h.runs(tol, 1000)
+        assert niter == it and np.abs(got - want).max() <= 1e-14, tol
+    for tol in (cols[:2], cols[:, None], np.full((1, 1), 1e-6), torch.from_numpy(cols[:2].copy()),
+                torch.full((1, 3), 1e-6)):
+        with pytest.raises(ValueError):
+            h.runs(tol, 1000)
