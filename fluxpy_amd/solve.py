@@ -254,7 +254,8 @@ def _jacobi_runs(csr, E, rho, left, tol, maxiter):
     back[:k] = tol_d
     niter, steps, last = 0, first, None
     while True:
-        steps = min(steps, maxiter - niter)
+        # the limit as `niter >= maxiter` after single steps has it
+        steps = int(np.ceil(min(steps, max(maxiter - niter, 1))))
         _lib.call("flux_csr_jacobi_run", n, csr.indptr.data_ptr(), csr.indices.data_ptr(),
                   csr.data.data_ptr(), _lib.dtype_code(csr.data.dtype), E.data_ptr(),
                   B.data_ptr(), B1.data_ptr(), _lib.ptr(X), _lib.ptr(X1), k, _lib.ptr(rho_t),

@@ -456,3 +456,19 @@ def test_jacobi_tolerances(host_jacobi):
                 torch.full((1, 3), 1e-6)):
         with pytest.raises(ValueError):
             h.runs(tol, 1000)
+
+
+@pytest.mark.parametrize("maxiter", [1, 5, np.int64(9), 31, 4.0, 31.0, 4.5, np.inf, -1])
+def test_jacobi_iteration_limits(host_jacobi, maxiter):
+    """Limits inside the first run, in a later one and none; whole numbers
+    of any type, and what is not a whole positive number ends where a loop
+    that counts single steps does."""
+    import warnings
+    h = host_jacobi
+    tol = 1e-9 if maxiter == np.inf else 1e-300
+    want, it = h.loop(tol, maxiter)
+    with warnings.catch_warnings(record=True) as seen:
+        warnings.simplefilter("always")
+        got, niter = h.runs(tol, maxiter)
+    assert niter == it and np.abs(got - want).max() <= 1e-14
+    assert len(seen) == (0 if maxiter == np.inf else 1)
