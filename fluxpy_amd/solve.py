@@ -219,7 +219,7 @@ def _tol_device(tol, k, device):
     if tol.shape not in ((), (1,), (k,)):
         raise ValueError(f"tol must be a scalar or have {k} entries (got shape "
                          f"{tuple(tol.shape)})")
-    return tol.to(device=device, dtype=t.float64).reshape(-1).contiguous()
+    return tol.detach().to(device=device, dtype=t.float64).reshape(-1).contiguous()
 
 
 JACOBI_RUN = (6, 24)    # iterations of the first run, and at most in any

@@ -407,7 +407,7 @@ def host_jacobi(monkeypatch):
 
     monkeypatch.setattr(_lib, "call", call)
     monkeypatch.setattr(_lib, "stream", lambda: None)
-    monkeypatch.setattr(_lib, "to_dev", torch.from_numpy)
+    monkeypatch.setattr(_lib, "to_dev", lambda a: torch.as_tensor(a).contiguous())
     rng = np.random.default_rng(0)
     n, k, rho = 40, 3, 0.5
     A = scipy.sparse.csr_matrix(rng.uniform(0, 1, (n, n)) * (rng.uniform(0, 1, (n, n)) < 0.3))
@@ -431,7 +431,10 @@ def host_jacobi(monkeypatch):
         B, it = solve._jacobi_runs(csr, torch.from_numpy(E), rho, False, tol, maxiter)
         return B.numpy(), it
 
-    return types.SimpleNamespace(loop=loop, runs=runs, k=k)
+    monkeypatch.setattr(_lib, "require_gpu", lambda: torch)
+    op = types.SimpleNamespace(shape=A.shape, apply=None, jacobi_step=None,
+                               jacobi_csr=lambda: csr)
+    return types.SimpleNamespace(loop=loop, runs=runs, k=k, op=op, E=E, rho=rho)
 
 
 def test_jacobi_tolerances(host_jacobi):
@@ -472,3 +475,16 @@ def test_jacobi_iteration_limits(host_jacobi, maxiter):
         got, niter = h.runs(tol, maxiter)
     assert niter == it and np.abs(got - want).max() <= 1e-14
     assert len(seen) == (0 if maxiter == np.inf else 1)
+
+
+def test_jacobi_default_tolerance_of_a_leaf(host_jacobi):
+    """The default tolerance is taken from E on the device, which may be a
+    leaf of an autograd graph."""
+    import torch
+    from fluxpy_amd.solve import solve_radiosity
+    h = host_jacobi
+    want, it = h.loop(1e-15 * np.abs(h.E).max(), 1000)
+    for grad in (False, True):
+        E = torch.from_numpy(h.E.copy()).requires_grad_(grad)
+        B, niter = solve_radiosity(h.op, E, h.rho)
+        assert niter == it and np.abs(B.detach().numpy() - want).max() <= 1e-14
