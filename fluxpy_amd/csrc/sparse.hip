@@ -203,14 +203,15 @@ constexpr int kBlockWaves = 4;
 template <typename TA, typename TX, typename TAcc, int MODE, int V, int LP1, int S, int kU>
 __global__ void __launch_bounds__(64 * kBlockWaves) k_csr_block(
     int64_t m, const int64_t *__restrict__ indptr, const int32_t *__restrict__ indices,
-    const TA *__restrict__ data, const TX *__restrict__ X, int64_t nrhs, int lp_log2,
-    TX *__restrict__ Y, JacobiArgs<TX> jac, int64_t row0) {
+    const TA *__restrict__ data, const TX *__restrict__ X, int64_t nrhs, int64_t tiles,
+    int64_t tile0, int lp_log2, TX *__restrict__ Y, JacobiArgs<TX> jac, int64_t row0) {
   if (MODE != SPMM_PLAIN && jacobi_met(jac, nrhs)) return;
   const TX *__restrict__ E = jac.E, *__restrict__ rho = jac.rho, *__restrict__ B = jac.B;
   const double rho_s = jac.rho_s;
   double *__restrict__ colmax = jac.colmax;
-  // this workgroup's right-hand sides: tile blockIdx.y of gridDim.y
-  const int64_t c_lo = nrhs * blockIdx.y / gridDim.y, c_hi = nrhs * (blockIdx.y + 1) / gridDim.y;
+  // this workgroup's right-hand sides: one of `tiles` equal tiles
+  const int64_t tile = tile0 + blockIdx.y;
+  const int64_t c_lo = nrhs * tile / tiles, c_hi = nrhs * (tile + 1) / tiles;
   const int cols = (int)(c_hi - c_lo);
   X += c_lo;
   Y += c_lo;
@@ -359,13 +360,15 @@ static int launch_block(int64_t m, const int64_t *indptr, const int32_t *indices
                         const JacobiArgs<TX> &jac, hipStream_t st, int64_t row0) {
   using TAcc = typename AccOf<decltype(typename WideOf<TA>::type() + TX())>::type;
   const int64_t tiles = (nrhs + 64 * V - 1) / (64 * V), width = (nrhs + tiles - 1) / tiles;
-  FLUX_CHECK(tiles <= 65535, "csr product: too many right-hand sides");
   int lp = 0;
   while (((int64_t)V << lp) < width) ++lp;
-  const dim3 grid(row_blocks<MODE>(m, jac.slots), (unsigned)tiles);
+  const unsigned rows = row_blocks<MODE>(m, jac.slots);
   auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(64 * kBlockWaves), 0, st, m, indptr, indices,
-                       (const TA *)data, (const TX *)X, nrhs, lp, (TX *)Y, jac, row0);
+    constexpr int64_t most = 65535;  // of a grid's second dimension
+    for (int64_t t = 0; t < tiles; t += most)
+      hipLaunchKernelGGL(kernel, dim3(rows, (unsigned)(tiles - t < most ? tiles - t : most)),
+                         dim3(64 * kBlockWaves), 0, st, m, indptr, indices, (const TA *)data,
+                         (const TX *)X, nrhs, tiles, t, lp, (TX *)Y, jac, row0);
   };
   // nonzeros staged per pass: 64 S; groups in flight: kU (kU G <= 64 S)
   if (lp == 0)

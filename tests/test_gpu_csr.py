@@ -160,3 +160,20 @@ def test_tolerance_tensors_on_host_and_device():
                 torch.tensor([1e-9], dtype=torch.float64).expand(3)):
         got, niter = solve_radiosity(A, E, 0.5, tol=tol)
         assert niter == it and np.array_equal(got, want)
+
+
+def test_more_tiles_of_columns_than_a_grid_holds():
+    """Two columns more than 65,535 full tiles of 128 FP64 columns."""
+    import torch
+    from fluxpy_amd import _kernels
+    from fluxpy_amd.solve import _CsrOperator
+    torch.cuda.set_device(0)
+    k = 65535 * 128 + 2
+    A = np.array([[0.0, 0.5], [0.25, 0.125]])
+    csr = _kernels.DeviceCSR.from_scipy(scipy.sparse.csr_matrix(A))
+    X = torch.arange(2 * k, dtype=torch.float64, device="cuda").reshape(2, k)
+    want = torch.stack([0.5 * X[1], 0.25 * X[0] + 0.125 * X[1]])     # exact
+    assert torch.equal(csr.matmat(X), want)
+    B1, cm = torch.empty_like(X), torch.empty(k, dtype=torch.float64, device="cuda")
+    _CsrOperator(csr).jacobi_step(X, X, 2.0, False, B1, cm)
+    assert torch.equal(B1, X + 2.0 * want) and torch.equal(cm, (2.0 * want).abs().amax(0))
