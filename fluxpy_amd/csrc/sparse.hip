@@ -86,6 +86,12 @@ __device__ __forceinline__ Vec<T, V> load_vec(const T *p) {
   return r;
 }
 
+// A change as the bits that atomic_max_nonneg orders by.  One that is not a
+// number is above all others if it counts, else it is no change.
+__device__ __forceinline__ unsigned long long change_bits(double v, bool nan_counts) {
+  return v == v || nan_counts ? (unsigned long long)__double_as_longlong(v) : 0ull;
+}
+
 // Distance of the rows of column maxima, in doubles.
 __host__ __device__ __forceinline__ int64_t slot_stride(int64_t nrhs) {
   return (nrhs + 31) / 32 * 32;
@@ -198,6 +204,10 @@ __global__ void __launch_bounds__(256) k_csr_vec(
 //
 // A lane past the end of a row of X loads the row's last V values instead
 // (nothing is read outside X) and stores what no other lane has.
+//
+// With more than 64 right-hand sides a change that is not a number is its
+// column's maximum, so an iteration that overflows does not converge; with
+// fewer, here and in k_csr_vec, it is passed over.
 constexpr int kBlockWaves = 4;
 
 template <typename TA, typename TX, typename TAcc, int MODE, int V, int LP1, int S, int kU>
@@ -228,8 +238,9 @@ __global__ void __launch_bounds__(64 * kBlockWaves) k_csr_block(
   const int col = min(c, cols - V);  // cols >= V
   const int fresh = c - col;         // values below this one belong to another lane
   const int64_t step = (int64_t)gridDim.x * kBlockWaves;
-  double rmax[V];
-  for (int v = 0; v < V; ++v) rmax[v] = 0.0;
+  const bool nan_counts = nrhs > 64;
+  unsigned long long rmax[V];
+  for (int v = 0; v < V; ++v) rmax[v] = 0;
   for (int64_t row = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6; row < m;
        row += step) {
     const int64_t k0 = indptr[row], k1 = indptr[row + 1];
@@ -320,14 +331,14 @@ __global__ void __launch_bounds__(64 * kBlockWaves) k_csr_block(
           const TX b1 = (TX)((TAcc)E[o + v] + y);
           Y[o + v] = b1;
           if (MODE == SPMM_JACOBI_SCALED) jac.Xn[c_lo + o + v] = rho[row0 + row] * b1;
-          rmax[v] = fmax(rmax[v], fabs((double)b1 - (double)B[o + v]));
+          rmax[v] = max(rmax[v], change_bits(fabs((double)b1 - (double)B[o + v]), nan_counts));
         }
       }
     }
   }
   if (MODE != SPMM_PLAIN) {
     // one atomic per column and workgroup
-    __shared__ double sd[kBlockWaves][64 * V];
+    __shared__ unsigned long long sd[kBlockWaves][64 * V];
     if (g == 0)
       for (int v = 0; v < V; ++v) sd[w][(lane & (LP - 1)) * V + v] = rmax[v];
     __syncthreads();
@@ -335,9 +346,9 @@ __global__ void __launch_bounds__(64 * kBlockWaves) k_csr_block(
       // column of the lane-major slot t, unless another lane has it
       const int cc = t / V * V, base = min(cc, cols - V), v = t - cc;
       if (cc < cols && v >= cc - base) {
-        double mx = 0.0;
-        for (int q = 0; q < kBlockWaves; ++q) mx = fmax(mx, sd[q][t]);
-        atomic_max_nonneg(colmax + base + v, mx);
+        unsigned long long mx = 0;
+        for (int q = 0; q < kBlockWaves; ++q) mx = max(mx, sd[q][t]);
+        atomicMax((unsigned long long *)colmax + base + v, mx);
       }
     }
   }

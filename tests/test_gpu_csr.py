@@ -177,3 +177,24 @@ def test_more_tiles_of_columns_than_a_grid_holds():
     B1, cm = torch.empty_like(X), torch.empty(k, dtype=torch.float64, device="cuda")
     _CsrOperator(csr).jacobi_step(X, X, 2.0, False, B1, cm)
     assert torch.equal(B1, X + 2.0 * want) and torch.equal(cm, (2.0 * want).abs().amax(0))
+
+
+@pytest.mark.parametrize("k", [65, 130, 300])
+def test_a_solve_that_overflows_does_not_converge(k):
+    """With more than 64 columns a change that is not a number counts as the
+    largest: an iteration that runs off to infinity (inf - inf) ends at its
+    limit with a warning."""
+    import torch
+    from fluxpy_amd.solve import _CsrOperator, _jacobi_runs
+    from fluxpy_amd import _kernels
+    torch.cuda.set_device(0)
+    csr = _kernels.DeviceCSR.from_scipy(scipy.sparse.csr_matrix(np.diag(np.full(70, 2.0 ** 100))))
+    E = torch.ones((70, k), dtype=torch.float64, device="cuda")
+    with pytest.warns(RuntimeWarning, match="did not converge in 40"):
+        B, niter = _jacobi_runs(csr, E, 1.0, False, 1e-9, 40)
+    assert niter == 40 and torch.isinf(B).all()
+    X = E.clone()
+    X[3, 5] = X[69, k - 1] = float("nan")
+    cm = torch.empty(k, dtype=torch.float64, device="cuda")
+    _CsrOperator(csr).jacobi_step(E, X, 1.0, False, torch.empty_like(E), cm)
+    assert torch.isnan(cm).nonzero().reshape(-1).tolist() == [5, k - 1]
