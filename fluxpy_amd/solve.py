@@ -19,6 +19,7 @@ tensor (result stays on the device).  Unlike the reference, iterations are
 capped by ``maxiter`` (a warning is emitted when it is reached): the
 reference loops forever when rho * rowsum(F) >= 1.
 """
+import math
 import warnings
 
 import numpy as np
@@ -213,9 +214,9 @@ def _tol_device(tol, k, device):
     t = _lib.torch()
     if not isinstance(tol, t.Tensor):
         tol = np.array(tol, dtype=np.float64)
-        # a number travels with a fill, not with a copy from the host
-        tol = t.full((1,), float(tol), dtype=t.float64, device=device) if tol.ndim == 0 \
-            else t.from_numpy(tol)
+        if tol.ndim == 0:       # a number travels with a fill, not with a copy
+            return t.full((1,), float(tol), dtype=t.float64, device=device)
+        tol = t.from_numpy(tol)
     if tol.shape not in ((), (1,), (k,)):
         raise ValueError(f"tol must be a scalar or have {k} entries (got shape "
                          f"{tuple(tol.shape)})")
@@ -255,7 +256,7 @@ def _jacobi_runs(csr, E, rho, left, tol, maxiter):
     niter, steps, last = 0, first, None
     while True:
         # the limit as `niter >= maxiter` after single steps has it
-        steps = int(np.ceil(min(steps, max(maxiter - niter, 1))))
+        steps = math.ceil(min(steps, max(maxiter - niter, 1)))
         _lib.call("flux_csr_jacobi_run", n, csr.indptr.data_ptr(), csr.indices.data_ptr(),
                   csr.data.data_ptr(), _lib.dtype_code(csr.data.dtype), E.data_ptr(),
                   B.data_ptr(), B1.data_ptr(), _lib.ptr(X), _lib.ptr(X1), k, _lib.ptr(rho_t),
