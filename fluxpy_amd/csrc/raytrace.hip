@@ -79,6 +79,12 @@ __device__ __forceinline__ void sun_begin(const flux_scene &S, LaneRay &L, int64
   const double lo = sel3(S.box, L.r.kz), hi = sel3(S.box + 3, L.r.kz);
   const double tmax = fmax(((L.r.Sz < 0.0 ? lo : hi) - L.r.o[2]) * L.r.Sz, 0.0);
   lane_begin(S, L, o, d, tmax, INFINITY, 0x7fffffff, skip, -1);
+  // Along an infinite component every triangle is at t = 0, which has no
+  // place in a range of t / tmax: such a ray takes the stackless walk alone.
+  if (L.r.Sz == 0.0) {
+    L.cur = kLaneVisible;
+    L.flags |= kFlagLost;
+  }
 }
 
 // Occlusion of facet I[p] towards D[q] (or D[p]): all facets of one

@@ -64,21 +64,21 @@ struct LaneRay {
   int sp;        // deferred children, in LDS words
 };
 
-// Walk the ray up to tlim (finite).  Rounding of a plane's position, in
-// units of 2^-24 of the scene's scale: the FP32 origin 1, the reciprocal
-// direction over tmax 4, inv x origin 1, the two fused steps 2.  The node
+// Walk the ray up to tmax (finite).  The direction is scaled in FP64, where
+// its length does not matter.  Rounding of a plane's position, in units of
+// 2^-24 of the scene's scale: the FP32 origin 1, the reciprocal direction
+// over tmax 4, inv x origin 1, the two fused steps 2.  The node
 // boxes contain boxes padded by 16 units, so a triangle hit at t in 0 .. tlim
 // has a slab interval of positive length inside 0 .. 1.
 __device__ __forceinline__ void lane_begin(const flux_scene &S, LaneRay &L, const double o[3],
                                            const double d[3], double tmax, double tlim, int klim,
                                            int skip1, int skip2) {
-  const float rt = 1.0f / ((float)(tmax * (1.0 + 1e-5)) + 1e-30f);
+  const double scale = tmax * (1.0 + 1e-5);
   int oct = 0;
   for (int c = 0; c < 3; ++c) {
-    const float dc = (float)d[c];
+    const float dc = (float)(d[c] * scale);
     const bool neg = dc < 0.0f;
-    float iv = fabsf(1.0f / dc * rt);
-    iv = fminf(iv, S.inv_max);
+    const float iv = fminf(fabsf(1.0f / dc), S.inv_max);
     L.inv[c] = neg ? -iv : iv;
     L.oi[c] = (float)o[c] * L.inv[c];
     oct += neg ? 3 << c : 0;

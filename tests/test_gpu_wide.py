@@ -151,6 +151,36 @@ def test_stack_overflow_with_rays_under_way(torch_dev, oracle_mod, query):
                 for k in range(D.shape[0])], 1))
 
 
+@pytest.mark.parametrize("cls", ["cgal", "embree"])
+def test_directions_of_any_length(torch_dev, oracle_mod, cls):
+    """Sun directions that FP32 does not hold, finite and infinite ones,
+    against every triangle of the mesh: a direction at a time, and all of
+    them in many batches."""
+    from fluxpy_amd.shape import CgalTrimeshShapeModel, EmbreeTrimeshShapeModel
+    V, F = _soup(300, 21)
+    sm = (CgalTrimeshShapeModel if cls == "cgal" else EmbreeTrimeshShapeModel)(V, F)
+    S = oracle_mod.OracleScene(V, F, use_bvh=False)
+    kw = {} if cls == "cgal" else {"mode": oracle_mod.MODE_EMBREE, "P": sm.P, "N": sm.N}
+    I, inf = np.arange(300), np.inf
+    D = np.concatenate([meshes.sun_directions(4, seed=3) * s
+                        for s in (1.0, 1e-300, 1e-40, 1e-30, 1e30, 1e38, 1e39, 1e300)]
+                       + [[[inf, 0, 0], [-inf, 0, 0], [0, inf, 1.0], [0, -1.0, -inf],
+                           [inf, inf, 0], [np.nan, 0, 1.0]]])
+    if cls == "embree":     # rays are FP32 there: no direction is left of these
+        D = np.delete(D, np.s_[4:16], axis=0)
+    want = S.occluded(I, D, **kw)
+    assert 0.05 < want[:, :4].mean() < 0.95
+    for k, d in enumerate(D):
+        assert np.array_equal(sm.is_occluded(I, d), want[:, k]), d
+    many = np.tile(np.arange(len(D)), 100)
+    E = sm.get_direct_irradiance_multi(1.0, D[many])
+    with np.errstate(invalid="ignore"):
+        for k in range(len(D)):
+            cosi = sm.N[:, 0] * D[k, 0] + sm.N[:, 1] * D[k, 1] + sm.N[:, 2] * D[k, 2]
+            lit = np.where((cosi > 0) & ~want[:, k], cosi, 0.0)
+            assert (E[:, k::len(D)] == lit[:, None]).all(), D[k]
+
+
 @pytest.mark.parametrize("mesh", ["soup", "deep", "terrain"])
 def test_small_queries_equal_large_ones(torch_dev, mesh):
     """Lanes without work take parts of other lanes' walks in queries of up
