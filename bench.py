@@ -338,9 +338,12 @@ def main():
 
 
 def visibility(torch, _lib, sm, ClusterTree, tm):
-    """Rays of the form-factor pass and its mask kernel's rate, warmed, in
-    facet order and in cluster order (the order the compressed build casts
-    them in: neighbouring rows then trace neighbouring rays)."""
+    """Rays of the form-factor pass (pairs that pass the prefilter, each
+    direction for itself) and the rate at which the mask is decided, warmed,
+    in facet order and in cluster order (the order of the compressed build).
+    `ms` is the pass that assembles a whole mesh, one walk for both
+    directions of a pair; `one_way` the one that row chunks and blocks take,
+    a walk for each."""
     nf = sm.num_faces
     dev = torch.device("cuda", 0)
     st = _lib.stream()
@@ -358,14 +361,23 @@ def visibility(torch, _lib, sm, ClusterTree, tm):
                   I.data_ptr(), nf, I.data_ptr(), nf, 1e-5, mask.data_ptr(), cnt.data_ptr(), st)
         rays = int(cnt.sum().item())
 
-        def launch():
+        def square():
+            _lib.call("flux_ff_mask_square", sm._scene.handle, P.data_ptr(), N.data_ptr(),
+                      _lib.F32, None if name == "facet" else I.data_ptr(), nf, 1e-5,
+                      mask.data_ptr(), cnt.data_ptr(), st)
+
+        def one_way():
             _lib.call("flux_ff_mask", sm._scene.handle, P.data_ptr(), N.data_ptr(), _lib.F32,
                       I.data_ptr(), nf, I.data_ptr(), nf, 1e-5, _lib.MODE_CGAL,
                       mask.data_ptr(), cnt.data_ptr(), st)
-        ms = tm.us(launch, reps=2, warm=1) * 1e-3
-        out[name] = {"ms": round(ms, 2), "mrays_per_s": round(rays / (ms * 1e-3) / 1e6, 1)}
-        log(f"[bench] visibility ({name} order, warmed): rays={rays} {ms:.1f} ms -> "
-            f"{out[name]['mrays_per_s']:.0f} Mrays/s")
+        rec = out[name] = {}
+        for key, fn in (("", square), ("one_way_", one_way)):
+            ms = tm.us(fn, reps=2, warm=1) * 1e-3
+            rec[key + "ms"] = round(ms, 2)
+            rec[key + "mrays_per_s"] = round(rays / (ms * 1e-3) / 1e6, 1)
+        log(f"[bench] visibility ({name} order, warmed): rays={rays} {rec['ms']:.1f} ms -> "
+            f"{rec['mrays_per_s']:.0f} Mrays/s (a walk per direction {rec['one_way_ms']:.1f} ms, "
+            f"{rec['one_way_mrays_per_s']:.0f})")
     out["rays"] = rays
     out["mrays_per_s"] = max(out["facet"]["mrays_per_s"], out["cluster"]["mrays_per_s"])
     del mask
