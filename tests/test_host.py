@@ -488,3 +488,18 @@ def test_jacobi_default_tolerance_of_a_leaf(host_jacobi):
         E = torch.from_numpy(h.E.copy()).requires_grad_(grad)
         B, niter = solve_radiosity(h.op, E, h.rho)
         assert niter == it and np.abs(B.detach().numpy() - want).max() <= 1e-14
+
+
+@pytest.mark.parametrize("cls", ["CgalTrimeshShapeModel", "EmbreeTrimeshShapeModel"])
+def test_sun_directions_need_three_components(cls):
+    """Refused before anything is sent to the device, whose kernels would
+    read past the end of shorter ones."""
+    from fluxpy_amd import shape
+    V, F = meshes.spherical_crater(npts=6, seed=1)
+    sm = object.__new__(getattr(shape, cls))
+    sm.dtype, sm.V, sm.F = V.dtype, V, F
+    sm.P = V[F].mean(axis=1)
+    I = np.arange(len(F))
+    for D in (np.ones(2), np.ones(4), np.ones((5, 2)), np.ones((len(F), 2))):
+        with pytest.raises(ValueError):
+            sm.is_occluded(I, D)
