@@ -131,7 +131,8 @@ static inline int64_t tile_width(int64_t words) {
 // Binary walks in such batches took 404 ms for the 41,472-facet terrain
 // (seed 5) and 1131 us for a 1,922-facet crater; this took 90.7 ms and
 // 214 us before the node step was shortened by a third (wide.h).  It is bound
-// by VALU issue (98 % busy, 62 % of lanes active).
+// by VALU issue (all pairs of the 41,472-facet terrain of the bench: VALUs
+// 92 % busy, 57 to 60 % of the lanes active).
 template <typename T>
 struct PairSource {
   const T *P, *N;
@@ -265,7 +266,8 @@ __global__ void __launch_bounds__(256, 5) k_ff_mask_rays(
 // order (cluster order elsewhere).  41,472-facet terrain, assembled with a
 // walk per direction 131 ms, with one 65.5, with the shorter node step 48.8;
 // a 1,922-facet crater, whose waves have about one batch of rays each, 407,
-// 412 and 352 us.  Bound by VALU issue like the above.
+// 412 and 352 us.  Bound by VALU issue like the above (94 to 95 % busy, 60 %
+// of the lanes; 0.97 L1 accesses a clock).
 template <typename T>
 struct BothSource {
   const T *P, *N;

@@ -142,8 +142,11 @@ __device__ __forceinline__ double conduction_solve(int64_t nf, int64_t f, int nz
 // step is bound by latency: in global memory every eighth row waited for its
 // loads and the way back for the stores before it.  Here a row's operands are
 // read one row ahead and a row takes the latency of its division (two chains
-// of 60 for every repeat of the linearisation).  Steps of 10,368 facets with
-// 60 layers: 77 us before, 56 now.  u stays in Uc for the caller to store.
+// of 60 for every solve, and a solve more for every repeat of the
+// linearisation).  10,368 facets with 60 layers: 77 us before, 56 now in the
+// hourly steps of a terrain under a moving sun, whose slowest wave repeats
+// twice, 47 and 41 where every wave repeats once.  u stays in Uc for the
+// caller to store.
 __device__ __forceinline__ double conduction_solve_lds(
     int64_t nf, int64_t f, int nz, const double *__restrict__ z, double dt,
     const double *__restrict__ rhoc, const double *__restrict__ alpha,
@@ -379,11 +382,11 @@ static double *conduction_coef(int64_t nf, int nz, void *work, double **gamw) {
 // LDS of a wave's profiles and multipliers, or 0 where the step works in
 // global memory: layers that need more than a CU has, and more waves than
 // the chip holds at once (then the rounds count, not the latency of one).
-// 60 layers and fluxes that jump, LDS / global: 450 facets 40 / 58 us,
-// 10,368 41 / 47; 20 layers: 10,368 38 / 45; 110 layers: 10,368 95 / 128.
-// 41,472 facets with 60 layers, a quarter more waves than fit, take 82 / 107
-// us where the linearisation repeats and 50 / 44 where it does not; 300,000
-// take 467 / 341.
+// 60 layers and fluxes drawn anew for every facet and step (one repeat of the
+// linearisation in every wave), LDS / global: 450 facets 40 / 58 us, 10,368
+// 41 / 47; 20 layers: 10,368 38 / 45; 110 layers: 10,368 95 / 128.  41,472
+// facets with 60 layers, a quarter more waves than fit, take 82 / 107 us so
+// and 50 / 44 without a repeat; 300,000 take 467 / 341.
 constexpr int64_t kLdsBytes = 160 * 1024;
 constexpr int64_t kCus = 256;
 
